@@ -136,7 +136,7 @@ __global__ __launch_bounds__(256) void k_adj(const SimParams P, const DevState D
         dop.last = 0;
         dop.reject = 0;
         dop.nstep = 0;
-        dop.k1 = poly_rhs(0.0, u, qb, qb.pon ? -(qb.pag * cos(qb.pw * rec.t)) : 0.0);
+        dop.k1 = poly_rhs(0.0, u, qb, -qb.pag, qb.pon ? phase_cos(qb.pw * rec.t) : 0.0);
         int st = 0;
         while ((st = dop_trial_fast_t<true, PULSE>(P, F, dop, u, h, sb, qb, nacc, nrej, &Q)) == 0) {
         }

@@ -622,6 +622,36 @@ ST_HD __forceinline__ void small_sincos(double th, double& s, double& c) {
     s = th * taylor_sum<1, 8>(t2);
 }
 
+// sin and cos of the pulse's phase w*t (fast variant): n = rint(2x/pi) and
+// x - n pi/2 with pi/2 in three parts -- the first product is exact to the
+// last bit of the difference, so the reduced argument is good to half an ulp
+// of pi/4 -- then the Taylor series (terms to r^16 and r^17; the first omitted
+// ones are below 3e-18).  Within 2 ulp of 1 absolute
+// (tests/host_device_math_main.cpp) at a quarter of its instructions; its
+// large-argument path, with a private array, is left to phases above 2^45.
+constexpr double PIO2_1 = 0x1.921fb54442d18p+0, PIO2_2 = 0x1.1a62633145c07p-54, PIO2_3 = -0x1.f1976b7ed8fbcp-110;
+ST_HD __forceinline__ void phase_sincos(double x, double& s, double& c) {
+    if (!(fabs(x) < 0x1p45)) {
+        sincos(x, &s, &c);
+        return;
+    }
+    const double n = rint(x * 0x1.45f306dc9c883p-1);
+    double r = __builtin_fma(-n, PIO2_1, x);
+    r = __builtin_fma(-n, PIO2_2, r);
+    r = __builtin_fma(-n, PIO2_3, r);
+    const double r2 = r * r;
+    const double cr = taylor_sum<0, 9>(r2), sr = r * taylor_sum<1, 9>(r2);
+    const int k = (int)(n - 4.0 * floor(0.25 * n));   // n mod 4
+    const double a = (k & 1) ? cr : sr, b = (k & 1) ? sr : cr;
+    s = (k & 2) ? -a : a;
+    c = ((k + 1) & 2) ? -b : b;
+}
+ST_HD __forceinline__ double phase_cos(double x) {
+    double s, c;
+    phase_sincos(x, s, c);
+    return c;
+}
+
 // Natural log and exp for the fast variant's step-size controllers, whose
 // factor (tol/err)^a (prev)^b only steers the step: a few ulp suffice, at a
 // third of the instructions of the library's correctly rounded forms.
@@ -662,19 +692,30 @@ ST_HD __forceinline__ double ctl_exp(double y) {
     return ldexp(taylor_sum<3, 14>(r), (int)n);
 }
 
-// gamma*B along a segment plus the pulse value pv (already scaled like the
-// polynomial), crossed with y
+// a x b with one rounding less per component (fast variant)
+ST_HD __forceinline__ d3 cross3_fma(const d3& a, const d3& b) {
+    return d3{__builtin_fma(a.y, b.z, -(a.z * b.y)), __builtin_fma(a.z, b.x, -(a.x * b.z)),
+              __builtin_fma(a.x, b.y, -(a.y * b.x))};
+}
+
+// gamma*B along a segment plus the pulse amp*cosv (amp already scaled like the
+// polynomial)
 template <bool PULSE = true>
-ST_HD __forceinline__ d3 poly_rhs(double tau, const d3& y, const Poly& q, double pv) {
+ST_HD __forceinline__ d3 poly_field(double tau, const Poly& q, double amp, double cosv) {
 #pragma clang fp contract(fast)
     d3 w{q.w0.x + tau * (q.w1.x + tau * q.w2.x), q.w0.y + tau * (q.w1.y + tau * q.w2.y),
          q.w0.z + tau * (q.w1.z + tau * q.w2.z)};
     if (PULSE && q.pon) {
-        if (q.paxis == 0) w.x += pv;
-        else if (q.paxis == 1) w.y += pv;
-        else w.z += pv;
+        if (q.paxis == 0) w.x = __builtin_fma(amp, cosv, w.x);
+        else if (q.paxis == 1) w.y = __builtin_fma(amp, cosv, w.y);
+        else w.z = __builtin_fma(amp, cosv, w.z);
     }
-    return cross3(y, w);
+    return w;
+}
+// ... crossed with y
+template <bool PULSE = true>
+ST_HD __forceinline__ d3 poly_rhs(double tau, const d3& y, const Poly& q, double amp, double cosv) {
+    return cross3_fma(y, poly_field<PULSE>(tau, q, amp, cosv));
 }
 
 ST_HD inline Poly make_poly(const SimParams& P, const Phys& F, const Seg& S) {
@@ -714,7 +755,7 @@ inline void set_poly_consts(Phys& F, bool gravity) {
 ST_HD __forceinline__ d3 rhs_fast(const SimParams& P, const Phys& F, double t, const d3& y, double t0,
                                        const Poly& q) {
 #pragma clang fp contract(fast)
-    return poly_rhs(t - t0, y, q, q.pon ? q.pag * cos(q.pw * t) : 0.0);
+    return poly_rhs(t - t0, y, q, q.pag, q.pon ? phase_cos(q.pw * t) : 0.0);
 }
 
 // gamma*B itself from the polynomial (plus the pulse when on)
@@ -724,7 +765,7 @@ ST_HD __forceinline__ d3 omega_fast(double t, double t0, const Poly& q) {
     d3 w{q.w0.x + tau * (q.w1.x + tau * q.w2.x), q.w0.y + tau * (q.w1.y + tau * q.w2.y),
          q.w0.z + tau * (q.w1.z + tau * q.w2.z)};
     if (q.pon) {
-        const double pv = q.pag * cos(q.pw * t);
+        const double pv = q.pag * phase_cos(q.pw * t);
         if (q.paxis == 0) w.x += pv;
         else if (q.paxis == 1) w.y += pv;
         else w.z += pv;

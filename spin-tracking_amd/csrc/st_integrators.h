@@ -266,6 +266,29 @@ __device__ __forceinline__ double fast_rsq(double x) {
 // x^(1/2) for x > 0
 __device__ __forceinline__ double fast_sqrt(double x) { return x * fast_rsq(x); }
 
+// Step factors of the DOP853 controller from the error norm: grow =
+// 1/max(facc2, min(facc1, fac11/safe)) after an accepted trial and shrink =
+// 1/min(facc1, fac11/safe) after a rejected one, fac11 = err^expo1 (over
+// facold^beta in grow).  With beta == 0, err^(-1/8) is three reciprocal
+// square roots, and the factors need no division.  (err == 0 or NaN: fac11 is
+// 0, as the power of a zero norm; an infinite norm leaves the clamp's bound.)
+__device__ __forceinline__ void dop_factors(const SimParams& P, double err, double facold, double& grow, double& shrink) {
+    if (!P.pow_beta_on && P.expo1 == 0.125) {
+        double inv = __builtin_inf();
+        if (err > 0.0) {
+            inv = fast_rsq(err);                                   // err^(-1/2)
+            inv = fast_sqrt(fast_sqrt(inv));                       // err^(-1/8)
+        }
+        shrink = __builtin_fmax(P.fac1, P.safe * inv);
+        grow = __builtin_fmin(P.fac2, shrink);
+    } else {
+        const double fac11 = pow(err, P.expo1);
+        const double fac = P.pow_beta_on ? fac11 / pow(facold, P.beta) : fac11;
+        grow = fast_rcp(__builtin_fmax(P.facc2, __builtin_fmin(P.facc1, fac / P.safe)));
+        shrink = 1.0 / min_d(P.facc1, fac11 / P.safe);
+    }
+}
+
 // Quadrature carried along an adjoint (backward) segment: moments
 // N_n = int u(s) s^n ds, n = 0, 1, 2, of the integrated vector over the
 // segment's own time s, by the step's 8th-order weights (b1, b6..b12) at the
@@ -292,18 +315,14 @@ ST_HD inline int dop_trial_fast_t(const SimParams& P, const Phys& F, DopState& D
     D.nstep++;
     const double x = D.x;
     const double tx = x - S.t0;
-    // Stages yield K = h*k.  Without a pulse, the field polynomial is scaled
-    // by h once per trial (hq); with one, the trial scales each k instead (3
-    // multiplies per stage), which keeps the 18 registers of the scaled copy
-    // free for the pulse's own state.
+    // Stages yield K = h*k: the field is scaled by h.  Without a pulse, the
+    // field polynomial is scaled once per trial (hq); with one, each stage
+    // scales its field instead (3 multiplies per stage), which keeps the 18
+    // registers of the scaled copy free for the pulse's own state.
     Poly hq = q;
     if constexpr (!PULSE)
         hq = Poly{d3{h * q.w0.x, h * q.w0.y, h * q.w0.z}, d3{h * q.w1.x, h * q.w1.y, h * q.w1.z},
                   d3{h * q.w2.x, h * q.w2.y, h * q.w2.z}, q.pag, q.pw, q.paxis, q.pon};
-    auto hk = [&](const d3& k) -> d3 {
-        if constexpr (PULSE) return d3{h * k.x, h * k.y, h * k.z};
-        else return k;
-    };
     const d3 K1{h * D.k1.x, h * D.k1.y, h * D.k1.z};
     // The pulse a*cos(w*t) at the stage times t = x + c*h (adjoint: at
     // t_end - (x + c*h), with the field negated): one sincos per trial at the
@@ -316,7 +335,7 @@ ST_HD inline int dop_trial_fast_t(const SimParams& P, const Phys& F, DopState& D
     const bool pon = PULSE && q.pon;
     if (pon) {
         hpag = ADJ ? -q.pag : q.pag;
-        sincos(q.pw * (ADJ ? (Q->t_end - x) : x), &pS, &pC);
+        phase_sincos(q.pw * (ADJ ? (Q->t_end - x) : x), pS, pC);
     }
     auto pcos = [&](double c) -> double {
         double a = q.pw * (c * h), sn, cs;
@@ -333,9 +352,14 @@ ST_HD inline int dop_trial_fast_t(const SimParams& P, const Phys& F, DopState& D
             cs = 1.0 - 2.0 * sn * sn;
             sn = s2;
         }
-        return ADJ ? pC * cs + pS * sn : pC * cs - pS * sn;
+        return __builtin_fma(pC, cs, ADJ ? pS * sn : -(pS * sn));
     };
-#define KR(C, YY) hk(poly_rhs<PULSE>(tx + (C) * h, (YY), hq, pon ? hpag * pcos(C) : 0.0))
+    auto rhs = [&](double tau, const d3& Y, double cosv) -> d3 {
+        d3 w = poly_field<PULSE>(tau, hq, hpag, cosv);
+        if constexpr (PULSE) w = d3{h * w.x, h * w.y, h * w.z};
+        return cross3_fma(Y, w);
+    };
+#define KR(C, YY) rhs(__builtin_fma((C), h, tx), (YY), pon ? pcos(C) : 0.0)
     // adjoint quadrature of this trial: sum_i b_i Y_i s_i^n
     d3 q0{0.0, 0.0, 0.0}, q1{0.0, 0.0, 0.0}, q2{0.0, 0.0, 0.0};
     auto quad = [&](double b, double si, const d3& Y) {
@@ -347,61 +371,54 @@ ST_HD inline int dop_trial_fast_t(const SimParams& P, const Phys& F, DopState& D
         }
     };
     quad(b1, tx, y);
-    d3 yy, K2, K3, K4, K5, K6, K7, K8, K9, K10, K11, K12;
-    ST_V3(yy, y.x + a21 * K1.x, y.y + a21 * K1.y, y.z + a21 * K1.z);
-    K2 = KR(c2, yy);
-    ST_V3(yy, y.x + (a31 * K1.x + a32 * K2.x), y.y + (a31 * K1.y + a32 * K2.y),
-          y.z + (a31 * K1.z + a32 * K2.z));
-    K3 = KR(c3, yy);
-    ST_V3(yy, y.x + (a41 * K1.x + a43 * K3.x), y.y + (a41 * K1.y + a43 * K3.y),
-          y.z + (a41 * K1.z + a43 * K3.z));
-    K4 = KR(c4, yy);
-    ST_V3(yy, y.x + (a51 * K1.x + a53 * K3.x + a54 * K4.x), y.y + (a51 * K1.y + a53 * K3.y + a54 * K4.y),
-          y.z + (a51 * K1.z + a53 * K3.z + a54 * K4.z));
-    K5 = KR(c5, yy);
-    ST_V3(yy, y.x + (a61 * K1.x + a64 * K4.x + a65 * K5.x), y.y + (a61 * K1.y + a64 * K4.y + a65 * K5.y),
-          y.z + (a61 * K1.z + a64 * K4.z + a65 * K5.z));
-    quad(b6, tx + c6 * h, yy);
-    K6 = KR(c6, yy);
-    ST_V3(yy, y.x + (a71 * K1.x + a74 * K4.x + a75 * K5.x + a76 * K6.x),
-          y.y + (a71 * K1.y + a74 * K4.y + a75 * K5.y + a76 * K6.y),
-          y.z + (a71 * K1.z + a74 * K4.z + a75 * K5.z + a76 * K6.z));
-    quad(b7, tx + c7 * h, yy);
-    K7 = KR(c7, yy);
-    ST_V3(yy, y.x + (a81 * K1.x + a84 * K4.x + a85 * K5.x + a86 * K6.x + a87 * K7.x),
-          y.y + (a81 * K1.y + a84 * K4.y + a85 * K5.y + a86 * K6.y + a87 * K7.y),
-          y.z + (a81 * K1.z + a84 * K4.z + a85 * K5.z + a86 * K6.z + a87 * K7.z));
-    quad(b8, tx + c8 * h, yy);
-    K8 = KR(c8, yy);
-    ST_V3(yy, y.x + (a91 * K1.x + a94 * K4.x + a95 * K5.x + a96 * K6.x + a97 * K7.x + a98 * K8.x),
-          y.y + (a91 * K1.y + a94 * K4.y + a95 * K5.y + a96 * K6.y + a97 * K7.y + a98 * K8.y),
-          y.z + (a91 * K1.z + a94 * K4.z + a95 * K5.z + a96 * K6.z + a97 * K7.z + a98 * K8.z));
-    quad(b9, tx + c9 * h, yy);
-    K9 = KR(c9, yy);
-    ST_V3(yy, y.x + (a101 * K1.x + a104 * K4.x + a105 * K5.x + a106 * K6.x + a107 * K7.x + a108 * K8.x + a109 * K9.x),
-          y.y + (a101 * K1.y + a104 * K4.y + a105 * K5.y + a106 * K6.y + a107 * K7.y + a108 * K8.y + a109 * K9.y),
-          y.z + (a101 * K1.z + a104 * K4.z + a105 * K5.z + a106 * K6.z + a107 * K7.z + a108 * K8.z + a109 * K9.z));
-    quad(b10, tx + c10 * h, yy);
-    K10 = KR(c10, yy);
-    ST_V3(yy,
-          y.x + (a111 * K1.x + a114 * K4.x + a115 * K5.x + a116 * K6.x + a117 * K7.x + a118 * K8.x + a119 * K9.x + a1110 * K10.x),
-          y.y + (a111 * K1.y + a114 * K4.y + a115 * K5.y + a116 * K6.y + a117 * K7.y + a118 * K8.y + a119 * K9.y + a1110 * K10.y),
-          y.z + (a111 * K1.z + a114 * K4.z + a115 * K5.z + a116 * K6.z + a117 * K7.z + a118 * K8.z + a119 * K9.z + a1110 * K10.z));
-    quad(b11, tx + c11 * h, yy);
-    K11 = KR(c11, yy);
+    // Each stage input is a chain of FMAs that starts from y, the weighted sums
+    // chains that start from their first product.
+    auto axpy = [](double a, const d3& K, const d3& s) -> d3 {
+        return d3{__builtin_fma(a, K.x, s.x), __builtin_fma(a, K.y, s.y), __builtin_fma(a, K.z, s.z)};
+    };
+    auto times = [](double a, const d3& K) -> d3 { return d3{a * K.x, a * K.y, a * K.z}; };
+    d3 yy;
+    yy = axpy(a21, K1, y);
+    const d3 K2 = KR(c2, yy);
+    yy = axpy(a31, K1, y); yy = axpy(a32, K2, yy);
+    const d3 K3 = KR(c3, yy);
+    yy = axpy(a41, K1, y); yy = axpy(a43, K3, yy);
+    const d3 K4 = KR(c4, yy);
+    yy = axpy(a51, K1, y); yy = axpy(a53, K3, yy); yy = axpy(a54, K4, yy);
+    const d3 K5 = KR(c5, yy);
+    yy = axpy(a61, K1, y); yy = axpy(a64, K4, yy); yy = axpy(a65, K5, yy);
+    quad(b6, __builtin_fma(c6, h, tx), yy);
+    const d3 K6 = KR(c6, yy);
+    yy = axpy(a71, K1, y); yy = axpy(a74, K4, yy); yy = axpy(a75, K5, yy); yy = axpy(a76, K6, yy);
+    quad(b7, __builtin_fma(c7, h, tx), yy);
+    const d3 K7 = KR(c7, yy);
+    yy = axpy(a81, K1, y); yy = axpy(a84, K4, yy); yy = axpy(a85, K5, yy); yy = axpy(a86, K6, yy);
+    yy = axpy(a87, K7, yy);
+    quad(b8, __builtin_fma(c8, h, tx), yy);
+    const d3 K8 = KR(c8, yy);
+    yy = axpy(a91, K1, y); yy = axpy(a94, K4, yy); yy = axpy(a95, K5, yy); yy = axpy(a96, K6, yy);
+    yy = axpy(a97, K7, yy); yy = axpy(a98, K8, yy);
+    quad(b9, __builtin_fma(c9, h, tx), yy);
+    const d3 K9 = KR(c9, yy);
+    yy = axpy(a101, K1, y); yy = axpy(a104, K4, yy); yy = axpy(a105, K5, yy); yy = axpy(a106, K6, yy);
+    yy = axpy(a107, K7, yy); yy = axpy(a108, K8, yy); yy = axpy(a109, K9, yy);
+    quad(b10, __builtin_fma(c10, h, tx), yy);
+    const d3 K10 = KR(c10, yy);
+    yy = axpy(a111, K1, y); yy = axpy(a114, K4, yy); yy = axpy(a115, K5, yy); yy = axpy(a116, K6, yy);
+    yy = axpy(a117, K7, yy); yy = axpy(a118, K8, yy); yy = axpy(a119, K9, yy); yy = axpy(a1110, K10, yy);
+    quad(b11, __builtin_fma(c11, h, tx), yy);
+    const d3 K11 = KR(c11, yy);
+    yy = axpy(a121, K1, y); yy = axpy(a124, K4, yy); yy = axpy(a125, K5, yy); yy = axpy(a126, K6, yy);
+    yy = axpy(a127, K7, yy); yy = axpy(a128, K8, yy); yy = axpy(a129, K9, yy); yy = axpy(a1210, K10, yy);
+    yy = axpy(a1211, K11, yy);
     const double xph = x + h;
-    ST_V3(yy,
-          y.x + (a121 * K1.x + a124 * K4.x + a125 * K5.x + a126 * K6.x + a127 * K7.x + a128 * K8.x + a129 * K9.x + a1210 * K10.x + a1211 * K11.x),
-          y.y + (a121 * K1.y + a124 * K4.y + a125 * K5.y + a126 * K6.y + a127 * K7.y + a128 * K8.y + a129 * K9.y + a1210 * K10.y + a1211 * K11.y),
-          y.z + (a121 * K1.z + a124 * K4.z + a125 * K5.z + a126 * K6.z + a127 * K7.z + a128 * K8.z + a129 * K9.z + a1210 * K10.z + a1211 * K11.z));
     quad(b12, tx + h, yy);
     const double c12 = pon ? pcos(1.0) : 0.0;
-    K12 = hk(poly_rhs<PULSE>(tx + h, yy, hq, hpag * c12));
+    const d3 K12 = rhs(tx + h, yy, c12);
 #undef KR
-    d3 bs;
-    ST_V3(bs, b1 * K1.x + b6 * K6.x + b7 * K7.x + b8 * K8.x + b9 * K9.x + b10 * K10.x + b11 * K11.x + b12 * K12.x,
-          b1 * K1.y + b6 * K6.y + b7 * K7.y + b8 * K8.y + b9 * K9.y + b10 * K10.y + b11 * K11.y + b12 * K12.y,
-          b1 * K1.z + b6 * K6.z + b7 * K7.z + b8 * K8.z + b9 * K9.z + b10 * K10.z + b11 * K11.z + b12 * K12.z);
+    d3 bs = times(b1, K1);
+    bs = axpy(b6, K6, bs); bs = axpy(b7, K7, bs); bs = axpy(b8, K8, bs); bs = axpy(b9, K9, bs);
+    bs = axpy(b10, K10, bs); bs = axpy(b11, K11, bs); bs = axpy(b12, K12, bs);
     d3 y1;
     ST_V3(y1, y.x + bs.x, y.y + bs.y, y.z + bs.z);
     // error norm: with K = h*k the reference's |h| * err / sqrt(n*deno)
@@ -409,36 +426,34 @@ ST_HD inline int dop_trial_fast_t(const SimParams& P, const Phys& F, DopState& D
     const double isx = fast_rcp(P.atol + P.rtol * __builtin_fmax(fabs(y.x), fabs(y1.x)));
     const double isy = fast_rcp(P.atol + P.rtol * __builtin_fmax(fabs(y.y), fabs(y1.y)));
     const double isz = fast_rcp(P.atol + P.rtol * __builtin_fmax(fabs(y.z), fabs(y1.z)));
-    double ex = (bs.x - bhh1 * K1.x - bhh2 * K9.x - bhh3 * K12.x) * isx;
-    double ey = (bs.y - bhh1 * K1.y - bhh2 * K9.y - bhh3 * K12.y) * isy;
-    double ez = (bs.z - bhh1 * K1.z - bhh2 * K9.z - bhh3 * K12.z) * isz;
-    const double err2 = ex * ex + ey * ey + ez * ez;
-    ex = (er1 * K1.x + er6 * K6.x + er7 * K7.x + er8 * K8.x + er9 * K9.x + er10 * K10.x + er11 * K11.x + er12 * K12.x) * isx;
-    ey = (er1 * K1.y + er6 * K6.y + er7 * K7.y + er8 * K8.y + er9 * K9.y + er10 * K10.y + er11 * K11.y + er12 * K12.y) * isy;
-    ez = (er1 * K1.z + er6 * K6.z + er7 * K7.z + er8 * K8.z + er9 * K9.z + er10 * K10.z + er11 * K11.z + er12 * K12.z) * isz;
-    const double e1 = ex * ex + ey * ey + ez * ez;
+    auto norm2 = [&](const d3& e) -> double {
+        const double ex = e.x * isx, ey = e.y * isy, ez = e.z * isz;
+        return __builtin_fma(ez, ez, __builtin_fma(ey, ey, ex * ex));
+    };
+    d3 e = axpy(-bhh1, K1, bs);
+    e = axpy(-bhh2, K9, e); e = axpy(-bhh3, K12, e);
+    const double err2 = norm2(e);
+    e = times(er1, K1);
+    e = axpy(er6, K6, e); e = axpy(er7, K7, e); e = axpy(er8, K8, e); e = axpy(er9, K9, e);
+    e = axpy(er10, K10, e); e = axpy(er11, K11, e); e = axpy(er12, K12, e);
+    const double e1 = norm2(e);
     const double deno = e1 + 0.01 * err2;
     const double err = (deno <= 0.0) ? 0.0 : e1 * fast_rsq(3.0 * deno);
-    double fac11;
-    if (!P.pow_beta_on && P.expo1 == 0.125)
-        fac11 = (err > 0.0) ? fast_sqrt(fast_sqrt(fast_sqrt(err))) : 0.0;
-    else
-        fac11 = pow(err, P.expo1);
-    double fac = P.pow_beta_on ? fac11 / pow(D.facold, P.beta) : fac11;
-    fac = __builtin_fmax(P.facc2, __builtin_fmin(P.facc1, fac / P.safe));
-    double hnew = h * fast_rcp(fac);
+    double grow, shrink;
+    dop_factors(P, err, D.facold, grow, shrink);
+    double hnew = h * grow;
     if (err <= 1.0 || P.fixed) {
         D.facold = max_d(err, 1.0E-4);
         nacc++;
         if constexpr (ADJ) {
             // derivative at the new point for the next trial (FSAL), and the
             // accepted step's quadrature
-            D.k1 = poly_rhs<PULSE>(tx + h, y1, q, -(q.pag * c12));
+            D.k1 = poly_rhs<PULSE>(tx + h, y1, q, -q.pag, c12);
             Q->n0 = d3{Q->n0.x + h * q0.x, Q->n0.y + h * q0.y, Q->n0.z + h * q0.z};
             Q->n1 = d3{Q->n1.x + h * q1.x, Q->n1.y + h * q1.y, Q->n1.z + h * q1.z};
             Q->n2 = d3{Q->n2.x + h * q2.x, Q->n2.y + h * q2.y, Q->n2.z + h * q2.z};
         } else {
-            D.k1 = poly_rhs<PULSE>(tx + h, y1, q, q.pag * c12);
+            D.k1 = poly_rhs<PULSE>(tx + h, y1, q, q.pag, c12);
         }
         y = y1;
         D.x = xph;
@@ -448,7 +463,7 @@ ST_HD inline int dop_trial_fast_t(const SimParams& P, const Phys& F, DopState& D
         D.reject = 0;
     } else {
         nrej++;
-        hnew = h / min_d(P.facc1, fac11 / P.safe);
+        hnew = h * shrink;
         D.reject = 1;
         D.last = 0;
     }
@@ -1151,7 +1166,7 @@ ST_HD inline int rk2_trial(const SimParams& P, const Phys& Fp, RkState& R, d3& y
             if (pon) {
                 const double X[5] = {X1, X2, X3, X4, X5};
 #pragma unroll
-                for (int i = 0; i < 5; ++i) hp[i] = h * (q.pag * cos(q.pw * (t + X[i] * h)));
+                for (int i = 0; i < 5; ++i) hp[i] = h * (q.pag * phase_cos(q.pw * (t + X[i] * h)));
             }
             auto expo = [&](int r) -> d3 {
 #if defined(__HIP_DEVICE_COMPILE__)
