@@ -30,6 +30,7 @@
 
 #include "../../include/spintrack.h"
 #include "st_adjoint.h"
+#include "st_quad.h"
 #include "st_analysis.h"
 #include "st_floquet.h"
 #include "st_fused.h"
@@ -215,6 +216,7 @@ struct st_handle {
     bool initialized = false;
     double last_target = 0.0;
     int grid_fused = 0, grid_spin = 0;
+    int n_simd = 0;                // SIMDs of the device (four per compute unit)
     // pipeline buffers
     char* d_recs = nullptr;
     uint32_t rec_cap = 0;          // C
@@ -453,6 +455,35 @@ static const void* spin_symbol(int variant, int integ, bool batch, bool pulse) {
     return batch ? spin_symbol_v<VAR_EXACT, true>(integ, pulse) : spin_symbol_v<VAR_EXACT, false>(integ, pulse);
 }
 
+// Four lanes per particle (st_quad.h) as long as all of the list is on the
+// chip at once: 16 quads in each of two waves per SIMD, 32,768 particles on
+// 256 compute units.  k_spin of one lane and of four, He-3 x 0.2 s: 1.82 and
+// 0.90 ms at 1,000, 1.96 and 1.27 ms at 16,384, 2.01 and 1.63 ms at 32,768,
+// 2.14 and 2.48 ms at 49,152 (neutrons x 0.5 s: 2.97 and 2.47 ms at 32,768,
+// 3.10 and 3.52 ms at 49,152).  0: the integrator has no such kernel.
+static uint32_t quad_limit(const st_handle* h) {
+    if (h->opt.integratorType != INT_DOP853 || h->ext.variant != ST_VARIANT_FAST) return 0;
+    return 32u * (uint32_t)h->n_simd;
+}
+template <bool BATCH, bool PULSE>
+static hipError_t launch_quad(st_handle* h, const PipeArgs& A) {
+    // one particle per wave until every SIMD has a wave, then up to 16
+    const uint32_t waves = (uint32_t)h->n_simd;
+    QuadArgs Q;
+    Q.P = h->P;
+    Q.D = h->D;
+    Q.A = A;
+    Q.ppw = 1;
+    while (Q.ppw < 16 && Q.ppw * waves < A.n_list) Q.ppw *= 2;
+    const uint32_t grid = (std::min(2 * waves, (A.n_list + Q.ppw - 1) / Q.ppw) + 3) / 4;
+    hipLaunchKernelGGL((k_spin_quad<BATCH, PULSE>), dim3(grid), dim3(256), 0, h->stream, Q);
+    return hipGetLastError();
+}
+static hipError_t spin_quad(st_handle* h, const PipeArgs& A) {
+    if (h->batch) return h->any_pulse ? launch_quad<true, true>(h, A) : launch_quad<true, false>(h, A);
+    return h->any_pulse ? launch_quad<false, true>(h, A) : launch_quad<false, false>(h, A);
+}
+
 static int persistent_grid(st_handle* h, const void* sym, int* cache) {
     if (*cache == 0) {
         int dev = 0, cus = 0, per_cu = 0;
@@ -460,6 +491,7 @@ static int persistent_grid(st_handle* h, const void* sym, int* cache) {
         HIPCHK(h, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
         HIPCHK(h, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, sym, 256, 0));
         *cache = cus * std::max(per_cu, 1);
+        h->n_simd = 4 * cus;
     }
     return ST_OK;
 }
@@ -687,7 +719,7 @@ static int run_pipeline(st_handle* h, RunArgs R) {
             // counts in d_small[1..2] and does not touch d_small[0]
             const int grid = std::min<int>(h->grid_spin, (int)((n_list + 255) / 256));
             if (h->ktime_on) HIPCHK(h, hipEventRecord(h->kev[2], h->stream));
-            HIPCHK(h, spin(h, dim3(grid), A));
+            HIPCHK(h, n_list <= quad_limit(h) ? spin_quad(h, A) : spin(h, dim3(grid), A));
             if (h->ktime_on) HIPCHK(h, hipEventRecord(h->kev[3], h->stream));
         } else if (spectral) {
             // one launch per register block of filters, each with its own queue

@@ -372,7 +372,8 @@ ST_HD inline int dop_trial_fast_t(const SimParams& P, const Phys& F, DopState& D
     };
     quad(b1, tx, y);
     // Each stage input is a chain of FMAs that starts from y, the weighted sums
-    // chains that start from their first product.
+    // chains that start from their first product (the quad kernel of
+    // st_quad.h forms every value by the same operations in the same order).
     auto axpy = [](double a, const d3& K, const d3& s) -> d3 {
         return d3{__builtin_fma(a, K.x, s.x), __builtin_fma(a, K.y, s.y), __builtin_fma(a, K.z, s.z)};
     };

@@ -1,0 +1,58 @@
+"""Four lanes per particle against one (csrc/st_quad.h): a small ensemble runs
+on the quad kernels, and the same particles as one configuration of a batch
+too large for them run on the one-lane kernels.  Both form every value by the
+same operations, so states, counters and snapshots are equal bit for bit."""
+import numpy as np
+import pytest
+
+import spintrack as st
+from spintrack import _lib, configs
+
+pytestmark = pytest.mark.gpu
+
+FILLER = 33000      # with it, the batch is past the quad kernels' 32,768
+
+
+def options(kind, n, seed):
+    if kind == "dressing":
+        o = configs.dressing(n=n, species="he3", tf=0.008, ioutInt=0.004, seed=seed)
+    elif kind == "he3":
+        o = configs.he3_thermal(n=n, tf=0.02, ioutInt=0.01, seed=seed)
+    else:
+        o = configs.neutron_cell(n=n, tf=0.06, ioutInt=0.03, seed=seed)
+        st.set_fields(o, yi=(0.0, 1.0, 0.0))
+    return o
+
+
+def run(p, times):
+    p.initParticles()
+    bb = p.block_bytes()
+    buf = _lib.DeviceBuffer(bb * len(times))
+    p.run(times, buf.ptr)
+    raw = p.copy_to_host(buf.ptr, bb * len(times))
+    buf.free()
+    return p.get_state(), p.particle_counters(), raw, bb
+
+
+# 1; a ragged wave; one particle past one per SIMD (two per wave)
+@pytest.mark.parametrize("n", [1, 17, 1025])
+@pytest.mark.parametrize("kind,variant", [("he3", st.VARIANT_FAST), ("dressing", st.VARIANT_FAST),
+                                          ("neutron", st.VARIANT_FAST)])
+def test_quad_equals_one_lane(kind, variant, n):
+    print(f"[quad] {kind} variant={variant} n={n}", flush=True)
+    axis = 1 if kind == "dressing" else 2
+    small, filler = options(kind, n, 11), options(kind, FILLER, 5000)
+    times = list(st.output_times(small))
+    with st.Particle(small, variant=variant, pulse_axis=axis) as p:
+        state, cnt, raw, bb = run(p, times)
+    with st.Particle.batch([small, filler], variant=variant, pulse_axis=axis, chunk_records=64) as b:
+        bstate, bcnt, braw, bbb = run(b, times)
+    for name in state.dtype.names:
+        assert state[name].tobytes() == bstate[:n][name].tobytes(), name
+    for name, v in cnt.items():
+        assert np.array_equal(v, bcnt[name][:n]), name
+    for k in range(len(times)):
+        x = raw[k * bb:(k + 1) * bb].view(st.snapshot_block_dtype(n))[0]
+        y = braw[k * bbb:(k + 1) * bbb].view(st.snapshot_block_dtype(n + FILLER))[0]
+        for name in x.dtype.names:
+            assert x[name].tobytes() == y[name][:n].tobytes(), (k, name)
