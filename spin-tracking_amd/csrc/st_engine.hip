@@ -465,23 +465,42 @@ static uint32_t quad_limit(const st_handle* h) {
     if (h->opt.integratorType != INT_DOP853 || h->ext.variant != ST_VARIANT_FAST) return 0;
     return 32u * (uint32_t)h->n_simd;
 }
+// particles per wave: one until every SIMD has a wave, then doubling to 16
+static uint32_t quad_ppw(const st_handle* h, uint32_t n) {
+    uint32_t ppw = 1;
+    while (ppw < 16 && ppw * (uint32_t)h->n_simd < n) ppw *= 2;
+    return ppw;
+}
+// workgroups of four waves, at most two waves per SIMD
+static uint32_t quad_grid(const st_handle* h, uint32_t n, uint32_t ppw) {
+    return (std::min(2 * (uint32_t)h->n_simd, (n + ppw - 1) / ppw) + 3) / 4;
+}
 template <bool BATCH, bool PULSE>
 static hipError_t launch_quad(st_handle* h, const PipeArgs& A) {
-    // one particle per wave until every SIMD has a wave, then up to 16
-    const uint32_t waves = (uint32_t)h->n_simd;
-    QuadArgs Q;
-    Q.P = h->P;
-    Q.D = h->D;
-    Q.A = A;
-    Q.ppw = 1;
-    while (Q.ppw < 16 && Q.ppw * waves < A.n_list) Q.ppw *= 2;
-    const uint32_t grid = (std::min(2 * waves, (A.n_list + Q.ppw - 1) / Q.ppw) + 3) / 4;
-    hipLaunchKernelGGL((k_spin_quad<BATCH, PULSE>), dim3(grid), dim3(256), 0, h->stream, Q);
+    QuadArgs Q{h->P, h->D, A, quad_ppw(h, A.n_list)};
+    hipLaunchKernelGGL((k_spin_quad<BATCH, PULSE>), dim3(quad_grid(h, A.n_list, Q.ppw)), dim3(256), 0, h->stream, Q);
     return hipGetLastError();
 }
 static hipError_t spin_quad(st_handle* h, const PipeArgs& A) {
     if (h->batch) return h->any_pulse ? launch_quad<true, true>(h, A) : launch_quad<true, false>(h, A);
     return h->any_pulse ? launch_quad<false, true>(h, A) : launch_quad<false, false>(h, A);
+}
+
+template <bool BATCH, bool PULSE>
+static hipError_t launch_adj(st_handle* h, const AdjArgs& J) {
+    if (J.n_list <= 32u * (uint32_t)h->n_simd) {
+        QuadAdjArgs Q{h->P, h->D, J, quad_ppw(h, J.n_list)};
+        hipLaunchKernelGGL((k_adj_quad<BATCH, PULSE>), dim3(quad_grid(h, J.n_list, Q.ppw)), dim3(256), 0, h->stream, Q);
+    } else {
+        // two waves per SIMD resident
+        const uint32_t grid = std::min((J.n_list + 255) / 256, 2u * (uint32_t)h->n_simd / 4);
+        hipLaunchKernelGGL((k_adj<BATCH, PULSE>), dim3(grid), dim3(256), 0, h->stream, h->P, h->D, J);
+    }
+    return hipGetLastError();
+}
+static hipError_t launch_adjoint(st_handle* h, const AdjArgs& J) {
+    if (h->batch) return h->any_pulse ? launch_adj<true, true>(h, J) : launch_adj<true, false>(h, J);
+    return h->any_pulse ? launch_adj<false, true>(h, J) : launch_adj<false, false>(h, J);
 }
 
 static int persistent_grid(st_handle* h, const void* sym, int* cache) {
@@ -1362,6 +1381,7 @@ ST_API int st_adjoint(st_handle* h, const void* blocks_dev, const double* seeds,
     J.seeds = d_seeds;
     J.n_targets = K;
     J.phys = h->d_phys;
+    J.queue = small + 3;      // zeroed with the replay's counters
     // Checkpoint groups: the replay runs G consecutive checkpoint chunks in one
     // stretch, from the first one's start state, into a window of G*C records
     // per particle (the same records the forward run wrote chunk by chunk:
@@ -1418,15 +1438,7 @@ ST_API int st_adjoint(st_handle* h, const void* blocks_dev, const double* seeds,
         J.n_list = c.n_list;
         J.C = A.C;   // the window's records per particle: bound and layout stride of both kernels
         J.ck = DevState{c.state, h->D.stride};
-        if (h->batch && h->any_pulse)
-            hipLaunchKernelGGL((k_adj<true, true>), grid, dim3(bs), 0, h->stream, h->P, h->D, J);
-        else if (h->batch)
-            hipLaunchKernelGGL((k_adj<true, false>), grid, dim3(bs), 0, h->stream, h->P, h->D, J);
-        else if (h->any_pulse)
-            hipLaunchKernelGGL((k_adj<false, true>), grid, dim3(bs), 0, h->stream, h->P, h->D, J);
-        else
-            hipLaunchKernelGGL((k_adj<false, false>), grid, dim3(bs), 0, h->stream, h->P, h->D, J);
-        HIPCHK(h, hipGetLastError());
+        HIPCHK(h, launch_adjoint(h, J));
         hi = lo;
     }
     // deterministic reduction: per-block partials per configuration, summed

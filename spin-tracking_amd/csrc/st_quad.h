@@ -86,10 +86,11 @@ __device__ __forceinline__ const ARGS& kernel_args() {
 // the tableau in registers
 // ---------------------------------------------------------------------------
 #define ST_DOP_RESIDENT(X)                                                                                          \
-    X(a61) X(a64) X(a65) X(a71) X(a74) X(a75) X(a76) X(a81) X(a84) X(a85) X(a86) X(a87) X(a91) X(a94) X(a95) X(a96) X(a97) X(a98) X(a101) X(a104) X(a105) X(a106) X(a107)   \
+    X(a81) X(a84) X(a85) X(a86) X(a87) X(a91) X(a94) X(a95) X(a96) X(a97) X(a98) X(a101) X(a104) X(a105) X(a106) X(a107)   \
     X(a108) X(a109) X(a111) X(a114) X(a115) X(a116) X(a117) X(a118) X(a119) X(a1110) X(a121) X(a124) X(a125)        \
     X(a126) X(a127) X(a128) X(a129) X(a1210) X(a1211) X(er1) X(er6) X(er7) X(er8) X(er9) X(er10) X(er11) X(er12)
 #define ST_DOP_LITERAL(X) X(a21) X(a31) X(a32) X(a41) X(a43) X(a51) X(a53) X(a54)
+#define ST_DOP_SPIN_RESIDENT(X) X(a61) X(a64) X(a65) X(a71) X(a74) X(a75) X(a76)
 #define ST_DOP_SCALAR(X)                                                                                            \
     X(c2) X(c3) X(c4) X(c5) X(c6) X(c7) X(c8) X(c9) X(c10) X(c11) X(b1) X(b6) X(b7) X(b8) X(b9) X(b10) X(b11)       \
     X(b12) X(bhh1) X(bhh2) X(bhh3)
@@ -98,17 +99,23 @@ __device__ __forceinline__ const ARGS& kernel_args() {
 // statements make each value opaque once per launch: the compiler would
 // otherwise rebuild it from literals at each use, two scalar moves that cost
 // as much as the product when the wave is alone on its SIMD.  (The first
-// stages' eight stay literals: 256 registers hold no more.)
+// stages' eight stay literals, fifteen in the adjoint, which carries the
+// quadrature: 256 registers hold no more.)
 struct DopTab {
 #define X(n) double n;
     ST_DOP_RESIDENT(X)
+    ST_DOP_SPIN_RESIDENT(X)
     ST_DOP_SCALAR(X)
     ST_DOP_LITERAL(X)
 #undef X
 };
+template <bool ADJ>
 __device__ __forceinline__ void dop_tab_load(DopTab& T) {
 #define X(n) T.n = dop::n; asm volatile("" : "+v"(T.n));
     ST_DOP_RESIDENT(X)
+#undef X
+#define X(n) T.n = dop::n; if constexpr (!ADJ) asm volatile("" : "+v"(T.n));
+    ST_DOP_SPIN_RESIDENT(X)
 #undef X
 #define X(n) T.n = dop::n; asm volatile("" : "+s"(T.n));
     ST_DOP_SCALAR(X)
@@ -157,17 +164,12 @@ struct QQuad {
     double n0, n1, n2, t_end;
 };
 
-// dop_trial_fast_t (st_integrators.h) on a quad.
-//
-// The trial is one chain: a stage's input, two quad moves, the cross product,
-// and the update of the next stage's input with it, each waiting for the one
-// before (an FP64 result is ready two issue slots after its instruction).
-// The products of older stages and the next stage's field fill those slots:
-// every stage sum is an accumulator that takes each K some stages before its
-// turn, and ST_KEEP pins the order the statements are written in (left
-// alone, the compiler, which schedules for registers here, issues each chain
-// back to back: 7.3 cycles per instruction).
-#define ST_KEEP __builtin_amdgcn_sched_barrier(0)
+// dop_trial_fast_t (st_integrators.h) on a quad.  About 250 vector
+// instructions and 60 quad moves without a pulse; alone on its SIMD a wave
+// takes 0.95 us for them, 7 cycles each (an FP64 instruction of a lone wave
+// takes 5.5 cycles, 9 when it needs the result before it).  Writing the stage
+// sums so that older products fill the waits of the newest one, with the
+// order pinned, measured the same (0.99 and 0.98 us on 1,000 neutrons).
 template <bool ADJ, bool PULSE>
 __device__ __forceinline__ int q_trial_fast(const SimParams& P, const DopTab& T, QDop& D, double& y, double& h,
                                             double seg_t0, const QPoly& q, const QPulse& pl,
@@ -212,21 +214,17 @@ __device__ __forceinline__ int q_trial_fast(const SimParams& P, const DopTab& T,
             hp2 = pcos(l == 0 ? T.c10 : l == 1 ? T.c11 : 1.0);
         }
     }
-    // the stage fields: a stage's is formed in five steps while the stage
-    // before it waits
-    double wa, wb, na, nb, tau;
-    auto pulse = [&](double p) {
+    auto stage = [&](double tau, double Y, double cosv) -> double {
+        double wa, wb;
+        q_field(tau, hq, wa, wb);
         if constexpr (PULSE) {
-            na = h * __builtin_fma(pl.ma, p, na);
-            nb = h * __builtin_fma(pl.mb, p, nb);
+            wa = h * __builtin_fma(pl.ma, cosv, wa);
+            wb = h * __builtin_fma(pl.mb, cosv, wb);
         }
+        return q_cross(Y, wa, wb);
     };
-#define QF1(C) tau = __builtin_fma((C), h, tx)
-#define QF2 na = hq.a1 + tau * hq.a2
-#define QF3 nb = hq.b1 + tau * hq.b2
-#define QF4 na = hq.a0 + tau * na
-#define QF5(LANE, HP) nb = hq.b0 + tau * nb; pulse(q_all<LANE>(HP))
-#define QFMA(S, A, K) S = __builtin_fma(T.A, K, S)
+#define QK(C, LANE, HP) stage(__builtin_fma(T.C, h, tx), yy, PULSE ? q_all<LANE>(HP) : 0.0)
+#define QF(S, A, K) S = __builtin_fma(T.A, K, S)
     double q0 = 0.0, q1 = 0.0, q2 = 0.0;
     auto quad = [&](double b, double si, double Y) {
         if constexpr (ADJ) {
@@ -237,63 +235,63 @@ __device__ __forceinline__ int q_trial_fast(const SimParams& P, const DopTab& T,
         }
     };
     const double K1 = h * D.k1;
-    QF1(T.c2); QF2; QF3; QF4; QF5(0, hp0);
     quad(T.b1, tx, y);
-    double ya, yb, t, yy = __builtin_fma(T.a21, K1, y);
-    double s3, s4, s5, s6, s7, s8, s9, s10, s11, s12, bs, er;
-    // one stage: moves | A | product | B | K | C | next input | D
-#define QSTAGE(N, A, B, C, CRIT, DD)                              \
-    wa = na; wb = nb;                                             \
-    ya = q_next1(yy); yb = q_next2(yy); ST_KEEP;                  \
-    A; ST_KEEP;                                                   \
-    t = yb * wa; ST_KEEP;                                         \
-    B; ST_KEEP;                                                   \
-    const double K##N = __builtin_fma(ya, wb, -t); ST_KEEP;       \
-    C; ST_KEEP;                                                   \
-    CRIT; ST_KEEP;                                                \
-    DD; ST_KEEP
-    QSTAGE(2, s3 = __builtin_fma(T.a31, K1, y); QF1(T.c3), QF2; s4 = __builtin_fma(T.a41, K1, y), QF3; QF4,
-           yy = __builtin_fma(T.a32, K2, s3), QF5(1, hp0); s5 = __builtin_fma(T.a51, K1, y);
-           s6 = __builtin_fma(T.a61, K1, y));
-    QSTAGE(3, QF1(T.c4); s7 = __builtin_fma(T.a71, K1, y), QF2; QF3, QF4; s8 = __builtin_fma(T.a81, K1, y),
-           yy = __builtin_fma(T.a43, K3, s4), QF5(2, hp0); QFMA(s5, a53, K3); s9 = __builtin_fma(T.a91, K1, y));
-    QSTAGE(4, QF1(T.c5); s10 = __builtin_fma(T.a101, K1, y), QF2; QF3, QF4; s11 = __builtin_fma(T.a111, K1, y),
-           yy = __builtin_fma(T.a54, K4, s5), QF5(3, hp0); QFMA(s6, a64, K4); QFMA(s7, a74, K4));
-    QSTAGE(5, QF1(T.c6); QFMA(s8, a84, K4), QF2; QF3, QF4; QFMA(s9, a94, K4),
-           yy = __builtin_fma(T.a65, K5, s6), QF5(0, hp1); QFMA(s7, a75, K5); QFMA(s8, a85, K5));
+    double yy = __builtin_fma(T.a21, K1, y);
+    const double K2 = QK(c2, 0, hp0);
+    yy = y;
+    QF(yy, a31, K1); QF(yy, a32, K2);
+    const double K3 = QK(c3, 1, hp0);
+    yy = y;
+    QF(yy, a41, K1); QF(yy, a43, K3);
+    const double K4 = QK(c4, 2, hp0);
+    yy = y;
+    QF(yy, a51, K1); QF(yy, a53, K3); QF(yy, a54, K4);
+    const double K5 = QK(c5, 3, hp0);
+    yy = y;
+    QF(yy, a61, K1); QF(yy, a64, K4); QF(yy, a65, K5);
     quad(T.b6, __builtin_fma(T.c6, h, tx), yy);
-    QSTAGE(6, QF1(T.c7); QFMA(s9, a95, K5), QF2; QF3, QF4; QFMA(s10, a104, K4),
-           yy = __builtin_fma(T.a76, K6, s7), QF5(1, hp1); QFMA(s8, a86, K6); QFMA(s9, a96, K6));
+    const double K6 = QK(c6, 0, hp1);
+    yy = y;
+    QF(yy, a71, K1); QF(yy, a74, K4); QF(yy, a75, K5); QF(yy, a76, K6);
     quad(T.b7, __builtin_fma(T.c7, h, tx), yy);
-    QSTAGE(7, QF1(T.c8); QFMA(s10, a105, K5), QF2; QF3, QF4; QFMA(s10, a106, K6),
-           yy = __builtin_fma(T.a87, K7, s8), QF5(2, hp1); QFMA(s9, a97, K7); QFMA(s11, a114, K4));
+    const double K7 = QK(c7, 1, hp1);
+    yy = y;
+    QF(yy, a81, K1); QF(yy, a84, K4); QF(yy, a85, K5); QF(yy, a86, K6); QF(yy, a87, K7);
     quad(T.b8, __builtin_fma(T.c8, h, tx), yy);
-    QSTAGE(8, QF1(T.c9); QFMA(s10, a107, K7), QF2; QF3; QFMA(s11, a115, K5), QF4; s12 = __builtin_fma(T.a121, K1, y),
-           yy = __builtin_fma(T.a98, K8, s9), QF5(3, hp1); QFMA(s10, a108, K8); QFMA(s11, a116, K6));
+    const double K8 = QK(c8, 2, hp1);
+    yy = y;
+    QF(yy, a91, K1); QF(yy, a94, K4); QF(yy, a95, K5); QF(yy, a96, K6); QF(yy, a97, K7); QF(yy, a98, K8);
     quad(T.b9, __builtin_fma(T.c9, h, tx), yy);
-    QSTAGE(9, QF1(T.c10); QFMA(s11, a117, K7), QF2; QF3; QFMA(s12, a124, K4), QF4; bs = T.b1 * K1; er = T.er1 * K1,
-           yy = __builtin_fma(T.a109, K9, s10), QF5(0, hp2); QFMA(s11, a118, K8); QFMA(s12, a125, K5));
+    const double K9 = QK(c9, 3, hp1);
+    yy = y;
+    QF(yy, a101, K1); QF(yy, a104, K4); QF(yy, a105, K5); QF(yy, a106, K6); QF(yy, a107, K7); QF(yy, a108, K8);
+    QF(yy, a109, K9);
     quad(T.b10, __builtin_fma(T.c10, h, tx), yy);
-    QSTAGE(10, QF1(T.c11); QFMA(s11, a119, K9), QF2; QF3; QFMA(s12, a126, K6), QF4; QFMA(bs, b6, K6); QFMA(er, er6, K6),
-           yy = __builtin_fma(T.a1110, K10, s11), QF5(1, hp2); QFMA(s12, a127, K7); QFMA(bs, b7, K7));
+    const double K10 = QK(c10, 0, hp2);
+    yy = y;
+    QF(yy, a111, K1); QF(yy, a114, K4); QF(yy, a115, K5); QF(yy, a116, K6); QF(yy, a117, K7); QF(yy, a118, K8);
+    QF(yy, a119, K9); QF(yy, a1110, K10);
     quad(T.b11, __builtin_fma(T.c11, h, tx), yy);
-    QSTAGE(11, tau = tx + h; QFMA(s12, a128, K8), QF2; QF3; QFMA(s12, a129, K9), QF4; QFMA(s12, a1210, K10),
-           yy = __builtin_fma(T.a1211, K11, s12), QF5(2, hp2); QFMA(er, er7, K7); QFMA(bs, b8, K8));
+    const double K11 = QK(c11, 1, hp2);
+    yy = y;
+    QF(yy, a121, K1); QF(yy, a124, K4); QF(yy, a125, K5); QF(yy, a126, K6); QF(yy, a127, K7); QF(yy, a128, K8);
+    QF(yy, a129, K9); QF(yy, a1210, K10); QF(yy, a1211, K11);
     quad(T.b12, tx + h, yy);
-    QSTAGE(12, QFMA(er, er8, K8); QFMA(bs, b9, K9), QFMA(er, er9, K9); QFMA(bs, b10, K10),
-           QFMA(er, er10, K10); QFMA(bs, b11, K11), QFMA(bs, b12, K12), QFMA(er, er11, K11); QFMA(er, er12, K12));
-#undef QSTAGE
-#undef QF1
-#undef QF2
-#undef QF3
-#undef QF4
-#undef QF5
+    const double c12 = PULSE ? q_all<2>(hp2) : 0.0;
+    const double K12 = stage(tx + h, yy, c12);
+    double bs = T.b1 * K1;
+    QF(bs, b6, K6); QF(bs, b7, K7); QF(bs, b8, K8); QF(bs, b9, K9); QF(bs, b10, K10); QF(bs, b11, K11); QF(bs, b12, K12);
+    double er = T.er1 * K1;
+    QF(er, er6, K6); QF(er, er7, K7); QF(er, er8, K8); QF(er, er9, K9); QF(er, er10, K10); QF(er, er11, K11);
+    QF(er, er12, K12);
+#undef QK
+#undef QF
     const double xph = x + h;
     const double y1 = y + bs;
     double e = __builtin_fma(-T.bhh1, K1, bs);
     // the derivative at the new point (used when the trial is accepted),
     // formed while the error norm's chain waits
-    const double c12 = PULSE ? q_all<2>(hp2) : 0.0;
+    double na, nb;
     q_field(tx + h, q, na, nb);
     if constexpr (PULSE) {
         na = __builtin_fma(pl.ma, c12, na);
@@ -306,7 +304,6 @@ __device__ __forceinline__ int q_trial_fast(const SimParams& P, const DopTab& T,
     const d3 v2 = q_vec(e * is), v1 = q_vec(er * is);
     const double err2 = __builtin_fma(v2.z, v2.z, __builtin_fma(v2.y, v2.y, v2.x * v2.x));
     const double e1 = __builtin_fma(v1.z, v1.z, __builtin_fma(v1.y, v1.y, v1.x * v1.x));
-#undef QFMA
     const double deno = e1 + 0.01 * err2;
     const double err = (deno <= 0.0) ? 0.0 : e1 * fast_rsq(3.0 * deno);
     double grow, shrink;
@@ -384,7 +381,7 @@ __device__ __forceinline__ void quad_spin_fast() {
     const bool first = (lane >> 2) < ppw;
     const bool lead = first && (lane & 3u) == 0u, owner = first && (lane & 3u) != 3u;
     DopTab T;
-    dop_tab_load(T);
+    dop_tab_load<false>(T);
     // a plain handle's physics in LDS, one copy per workgroup
     __shared__ Phys shared_phys;
     if constexpr (!BATCH) {
@@ -514,6 +511,172 @@ __device__ __forceinline__ void quad_spin_fast() {
 template <bool BATCH, bool PULSE>
 __global__ __launch_bounds__(256, 2) void k_spin_quad(const QuadArgs) {
     quad_spin_fast<BATCH, PULSE>();
+}
+
+// ---------------------------------------------------------------------------
+// the adjoint's walk back on quads (k_adj, st_adjoint.h)
+// ---------------------------------------------------------------------------
+struct QuadAdjArgs {
+    SimParams P;
+    DevState D;
+    AdjArgs A;
+    uint32_t ppw;
+};
+// The lane of component c carries u_c, its moments and its share of the
+// gradient sums: u_c r_j (3), (u x v)_c and u_c.
+template <bool BATCH, bool PULSE>
+__global__ __launch_bounds__(256, 2) void k_adj_quad(const QuadAdjArgs) {
+#pragma clang fp contract(fast)
+    auto args = []() -> const QuadAdjArgs& { return kernel_args<QuadAdjArgs>(); };
+    const uint32_t lane = __lane_id();
+    const uint32_t c = (lane & 3u) == 3u ? 0u : (lane & 3u);
+    const uint32_t ppw = args().ppw;
+    const bool first = (lane >> 2) < ppw;
+    const bool lead = first && (lane & 3u) == 0u, owner = first && (lane & 3u) != 3u;
+    DopTab T;
+    dop_tab_load<true>(T);
+    __shared__ Phys shared_phys;
+    // per lane: its gradient sums, and p0 and v0 of the segment being
+    // integrated (registers go to the tableau)
+    __shared__ double sums[5][256], pv[6][256];
+    if constexpr (!BATCH) {
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(args().A.phys);
+        for (uint32_t i = threadIdx.x; i < sizeof(Phys) / 4; i += blockDim.x) reinterpret_cast<uint32_t*>(&shared_phys)[i] = src[i];
+        __syncthreads();
+    }
+    QPulse pl;
+    if constexpr (PULSE && !BATCH) q_pulse_load(pl, shared_phys, c, -1.0);
+    uint32_t pid = 0, cfg = 0;
+    double u = 0.0, h = 0.0;
+    int32_t kb = 0, fail = 0, j = -1;
+    SegRec nxt;                 // record j, loaded while record j + 1 is integrated,
+    double nxt_t0 = 0.0;        // and its start time
+    QPoly q;
+    QQuad Q;
+    QDop dop;
+    uint32_t nacc = 0, nrej = 0;
+    enum { S_DONE = 0, S_NEXT = 1, S_INT = 2 };
+    int phase = S_DONE;
+    // record i and its start time
+    auto load = [&](const AdjArgs& A, int32_t i) {
+        if (i < 0) return;
+        nxt = get_rec(A.recs, A.C, pid, (uint32_t)i);
+        nxt_t0 = i > 0 ? get_rec(A.recs, A.C, pid, (uint32_t)(i - 1)).t : A.ck.ld(F_T, pid * 8u);
+    };
+    auto take = [&]() {
+        const AdjArgs& A = args().A;
+        const uint32_t i = quad_acquire(A.queue, ppw);
+        if (i >= A.n_list) return;
+        pid = A.list[i];
+        const uint32_t o = pid * 8u;
+        u = A.adj.ld(A_UX + (int)c, o);
+        h = A.adj.ld(A_H, o);
+        kb = (int32_t)A.adj.ld<int64_t>(A_K, o);
+        fail = (int32_t)A.adj.ld<int64_t>(A_FAIL, o);
+        if constexpr (BATCH) {
+            const DevState& D = args().D;
+            cfg = (uint32_t)*(D.template f<uint64_t>(F_CFG) + pid);
+        }
+        if constexpr (PULSE && BATCH) q_pulse_load(pl, A.phys[cfg], c, -1.0);
+        for (int k = 0; k < 3; ++k) sums[k][threadIdx.x] = A.adj.ld(A_G0 + 3 * (int)c + k, o);
+        sums[3][threadIdx.x] = A.adj.ld(A_G0 + 9 + (int)c, o);
+        sums[4][threadIdx.x] = A.adj.ld(A_G0 + 12 + (int)c, o);
+        j = (int32_t)A.seg_count[pid] - 1;
+        load(A, j);
+        phase = S_NEXT;
+    };
+    take();
+    while (phase != S_DONE) {
+        while (phase == S_NEXT) {
+            const AdjArgs& A = args().A;
+            if (j < 0) {
+                const uint32_t o = pid * 8u;
+                if (owner) {
+                    A.adj.st(A_UX + (int)c, o, u);
+                    for (int k = 0; k < 3; ++k) A.adj.st(A_G0 + 3 * (int)c + k, o, sums[k][threadIdx.x]);
+                    A.adj.st(A_G0 + 9 + (int)c, o, sums[3][threadIdx.x]);
+                    A.adj.st(A_G0 + 12 + (int)c, o, sums[4][threadIdx.x]);
+                }
+                if (lead) {
+                    A.adj.st(A_H, o, h);
+                    A.adj.st<int64_t>(A_K, o, kb);
+                    A.adj.st<int64_t>(A_FAIL, o, fail);
+                }
+                phase = S_DONE;
+                take();
+                continue;
+            }
+            const SegRec rec = nxt;
+            const double t0 = nxt_t0;
+            load(A, j - 1);
+            if ((rec.flags & R_IEND) && kb >= 0) {
+                const double* Sk = reinterpret_cast<const double*>(A.blocks + (uint64_t)kb * A.block_bytes + 56ull * A.n) +
+                                   3ull * pid;
+                const double* gp = A.seeds + 3 * ((uint64_t)cfg * A.n_targets + (uint64_t)kb);
+                const double gc = gp[c], Sc = Sk[c];
+                u = u + __builtin_fma(q_next1(gc), q_next2(Sc), -(q_next2(gc) * q_next1(Sc)));
+                --kb;
+                const d3 all = q_vec(u);
+                if (!(__builtin_isfinite(all.x) && __builtin_isfinite(all.y) && __builtin_isfinite(all.z))) fail = -3;
+            }
+            const double Ts = rec.t - t0;
+            if (!(rec.flags & R_INTEGRATE) || fail || !(Ts > 0.0)) {
+                --j;
+                continue;
+            }
+            QPoly f;
+            q_make_poly(f, BATCH ? A.phys[cfg] : shared_phys, d3{rec.px, rec.py, rec.pz}, d3{rec.vx, rec.vy, rec.vz}, c);
+            q.a0 = -(f.a0 + Ts * (f.a1 + Ts * f.a2));
+            q.b0 = -(f.b0 + Ts * (f.b1 + Ts * f.b2));
+            q.a1 = f.a1 + 2.0 * Ts * f.a2;
+            q.b1 = f.b1 + 2.0 * Ts * f.b2;
+            q.a2 = -f.a2;
+            q.b2 = -f.b2;
+            pv[0][threadIdx.x] = rec.px; pv[1][threadIdx.x] = rec.py; pv[2][threadIdx.x] = rec.pz;
+            pv[3][threadIdx.x] = rec.vx; pv[4][threadIdx.x] = rec.vy; pv[5][threadIdx.x] = rec.vz;
+            Q.n0 = Q.n1 = Q.n2 = 0.0;
+            Q.t_end = rec.t;
+            dop.x = 0.0;
+            dop.xf = Ts;
+            dop.facold = 1.0E-4;
+            dop.last = 0;
+            dop.reject = 0;
+            dop.nstep = 0;
+            double wa = q.a0, wb = q.b0;
+            if constexpr (PULSE) {
+                const double cosv = pl.on ? phase_cos(pl.pw * rec.t) : 0.0;
+                wa = __builtin_fma(pl.ma, cosv, wa);
+                wb = __builtin_fma(pl.mb, cosv, wb);
+            }
+            dop.k1 = q_cross(u, wa, wb);
+            phase = S_INT;
+        }
+        if (phase == S_INT) {
+            const int st = q_trial_fast<true, PULSE>(args().P, T, dop, u, h, 0.0, q, pl, nacc, nrej, &Q);
+            if (st < 0) {
+                fail = st;
+                --j;
+                phase = S_NEXT;
+            } else if (st > 0) {
+                const double ay = args().P.gravity ? G_CONST : 0.0;
+                const AdjMoments M = adj_moments(dop.xf, Q.n0, Q.n1, Q.n2);
+                const uint32_t i = threadIdx.x;
+                const d3 v{pv[3][i], pv[4][i], pv[5][i]};
+                const double vc = q_pick(v, c);
+                // (u x v)_c plus -int u_z tau ay dt for x, +int u_x tau ay dt for z
+                const double uv = __builtin_fma(q_next1(M.m0), q_next2(vc), -(q_next2(M.m0) * q_next1(vc)));
+                const double mz = q_next2(M.m1), mx = q_next1(M.m1);
+                const double uva = c == 0 ? __builtin_fma(mz, -ay, uv) : (c == 2 ? __builtin_fma(mx, ay, uv) : uv);
+                sums[0][i] += adj_ur(M, pv[0][i], v.x, 0.0);
+                sums[1][i] += adj_ur(M, pv[1][i], v.y, 0.5 * ay);
+                sums[2][i] += adj_ur(M, pv[2][i], v.z, 0.0);
+                sums[3][i] += uva;
+                sums[4][i] += M.m0;
+                --j;
+                phase = S_NEXT;
+            }
+        }
+    }
 }
 
 }  // namespace st

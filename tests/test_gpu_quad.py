@@ -56,3 +56,29 @@ def test_quad_equals_one_lane(kind, variant, n):
         y = braw[k * bbb:(k + 1) * bbb].view(st.snapshot_block_dtype(n + FILLER))[0]
         for name in x.dtype.names:
             assert x[name].tobytes() == y[name][:n].tobytes(), (k, name)
+
+
+# the walk back (k_adj_quad against k_adj): gradients of one configuration
+@pytest.mark.parametrize("kind,n", [("neutron", 1), ("neutron", 70), ("dressing", 17)])
+def test_quad_adjoint_equals_one_lane(kind, n):
+    print(f"[quad adjoint] {kind} n={n}", flush=True)
+    axis = 1 if kind == "dressing" else 2
+    small, filler = options(kind, n, 11), options(kind, FILLER, 5000)
+    times = list(st.output_times(small))
+    seeds = np.linspace(-1.0, 1.0, 3 * len(times)).reshape(1, len(times), 3)
+
+    def gradient(p, s):
+        p.set_checkpointing(True)
+        p.initParticles()
+        buf = _lib.DeviceBuffer(p.block_bytes() * len(times))
+        p.run(times, buf.ptr)
+        g = p.adjoint(buf.ptr, s)
+        buf.free()
+        return g
+
+    with st.Particle(small, variant=st.VARIANT_FAST, pulse_axis=axis, chunk_records=8) as p:
+        g = gradient(p, seeds)
+    with st.Particle.batch([small, filler], variant=st.VARIANT_FAST, pulse_axis=axis, chunk_records=8) as b:
+        gb = gradient(b, np.concatenate([seeds, seeds]))
+    assert np.all(np.isfinite(g)) and np.any(g != 0.0)
+    assert g[0].tobytes() == gb[0].tobytes()
