@@ -460,9 +460,11 @@ static const void* spin_symbol(int variant, int integ, bool batch, bool pulse) {
 // 256 compute units.  k_spin of one lane and of four, He-3 x 0.2 s: 1.82 and
 // 0.90 ms at 1,000, 1.96 and 1.27 ms at 16,384, 2.01 and 1.63 ms at 32,768,
 // 2.14 and 2.48 ms at 49,152 (neutrons x 0.5 s: 2.97 and 2.47 ms at 32,768,
-// 3.10 and 3.52 ms at 49,152).  0: the integrator has no such kernel.
+// 3.10 and 3.52 ms at 49,152).  The exact variant on the same He-3: 4.32 and
+// 1.96 ms, 4.41 and 2.33 ms, 4.50 and 3.54 ms, 4.55 and 4.58 ms.  0: the
+// integrator has no such kernel, or the field hooks have their own form.
 static uint32_t quad_limit(const st_handle* h) {
-    if (h->opt.integratorType != INT_DOP853 || h->ext.variant != ST_VARIANT_FAST) return 0;
+    if (h->opt.integratorType != INT_DOP853 || !ST_FIELDS_POLYNOMIAL) return 0;
     return 32u * (uint32_t)h->n_simd;
 }
 // particles per wave: one until every SIMD has a wave, then doubling to 16
@@ -475,15 +477,19 @@ static uint32_t quad_ppw(const st_handle* h, uint32_t n) {
 static uint32_t quad_grid(const st_handle* h, uint32_t n, uint32_t ppw) {
     return (std::min(2 * (uint32_t)h->n_simd, (n + ppw - 1) / ppw) + 3) / 4;
 }
-template <bool BATCH, bool PULSE>
+template <int VAR, bool BATCH, bool PULSE>
 static hipError_t launch_quad(st_handle* h, const PipeArgs& A) {
     QuadArgs Q{h->P, h->D, A, quad_ppw(h, A.n_list)};
-    hipLaunchKernelGGL((k_spin_quad<BATCH, PULSE>), dim3(quad_grid(h, A.n_list, Q.ppw)), dim3(256), 0, h->stream, Q);
+    hipLaunchKernelGGL((k_spin_quad<VAR, BATCH, PULSE>), dim3(quad_grid(h, A.n_list, Q.ppw)), dim3(256), 0, h->stream, Q);
     return hipGetLastError();
 }
+template <int VAR>
+static hipError_t spin_quad_v(st_handle* h, const PipeArgs& A) {
+    if (h->batch) return h->any_pulse ? launch_quad<VAR, true, true>(h, A) : launch_quad<VAR, true, false>(h, A);
+    return h->any_pulse ? launch_quad<VAR, false, true>(h, A) : launch_quad<VAR, false, false>(h, A);
+}
 static hipError_t spin_quad(st_handle* h, const PipeArgs& A) {
-    if (h->batch) return h->any_pulse ? launch_quad<true, true>(h, A) : launch_quad<true, false>(h, A);
-    return h->any_pulse ? launch_quad<false, true>(h, A) : launch_quad<false, false>(h, A);
+    return h->ext.variant == ST_VARIANT_FAST ? spin_quad_v<VAR_FAST>(h, A) : spin_quad_v<VAR_EXACT>(h, A);
 }
 
 template <bool BATCH, bool PULSE>

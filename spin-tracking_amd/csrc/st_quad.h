@@ -2,23 +2,26 @@
 // that do not fill the chip.
 //
 // What bounds a small ensemble is one lane's chain of trial steps: with one
-// wave per SIMD nothing else can issue, so every instruction of the trial,
-// scalar ones included, costs its own issue slot (about 800 vector and 1,300
-// scalar instructions per one-lane fast trial, most of the scalar ones moves
-// of 64-bit tableau literals: 3.8 us per trial, against 1.7 us when three
-// waves share the SIMD).  Here a particle takes a quad of lanes, one spin
-// component each (lane 3 repeats lane 0):
+// wave per SIMD nothing else can issue, and a lone wave needs 5.5 cycles for
+// an FP64 instruction and 9 for one that waits for the result before it.  A
+// one-lane trial is about 1,000 instructions, the segment set-up that some
+// lane of a wave needs on most trips included (fast: 2.1 us on neutrons,
+// 3.2 us on He-3, whose segments are short; exact 5.4 and 7.1 us; 1.6 us per
+// fast trial when three waves share the SIMD).  Here a particle takes a quad
+// of lanes, one spin component each (lane 3 repeats lane 0):
 //   * the stage sums, two thirds of the trial's operations, run once per quad
 //     instead of once per component;
 //   * the components meet in the cross products and the error norm, through
 //     quad-permute moves (no LDS, no waits);
-//   * the tableau stays in vector registers for the whole launch (the
-//     one-lane kernel needs them for its state; a lane of a quad holds a third
-//     of that state);
-//   * the next segment record is loaded while the current one is integrated.
+//   * the tableau stays in registers for the whole launch (the one-lane kernel
+//     needs them for its state; a lane of a quad holds a third of that state);
+//   * the next segment record is loaded while the current one is integrated;
+//   * the pulse's stage cosines are split over the quad.
+// Per trial 1.0 us on neutrons and 1.5 us on He-3 (1,000 particles, fast),
+// 2.4 and 3.2 us exact.
 // Every value is formed by the one-lane trial's operations in its order, so
-// accept/reject decisions and results are those of the one-lane kernels; a
-// quad's four lanes always agree on the control flow.
+// accept/reject decisions and results are those of the one-lane kernels bit
+// for bit; a quad's four lanes always agree on the control flow.
 #pragma once
 
 #include "st_adjoint.h"
@@ -142,7 +145,7 @@ struct QPulse {
 
 // Loop state of a segment: DopState with the lane's component of k1.
 struct QDop {
-    double x, xf, facold, k1;
+    double x, xf, facold, k1, posneg;   // (posneg: exact variant)
     int32_t reject, last;
     uint32_t nstep;
 };
@@ -334,6 +337,138 @@ __device__ __forceinline__ int q_trial_fast(const SimParams& P, const DopTab& T,
     return 0;
 }
 
+// ---------------------------------------------------------------------------
+// the exact trial, one component per lane
+// ---------------------------------------------------------------------------
+// What omega_exact reads for one component, and the segment's start state of
+// that component.  hg and gg: half the gravity and the gravity along the
+// component (0 across it, where (0*d)*d and 0*d are the +0 the one-lane form
+// adds).
+struct QExact {
+    double p0, v0, hg, gg;
+    double G0, G1, G2, B0, Ea, Eb, gamma;
+    double pa, pw;
+    int32_t axis;        // the pulse's axis; -1: none on this particle
+    bool mine;           // it is the lane's component
+};
+__device__ __forceinline__ void q_exact_load(QExact& X, const SimParams& P, const Phys& F, uint32_t c) {
+    const uint32_t a = c == 2 ? 0u : c + 1, b = c == 0 ? 2u : c - 1;
+    X.G0 = F.G[3 * c]; X.G1 = F.G[3 * c + 1]; X.G2 = F.G[3 * c + 2];
+    X.B0 = (&F.B0x)[c];
+    X.Ea = (&F.Ex)[a];
+    X.Eb = (&F.Ex)[b];
+    X.gamma = F.gamma;
+    X.pa = F.pa;
+    X.pw = F.pw;
+    X.axis = F.pulse_on ? F.pulse_axis : -1;
+    X.mine = X.axis == (int32_t)c;
+    X.hg = P.gravity && c == 1 ? HALF_G : 0.0;
+    X.gg = P.gravity && c == 1 ? G_CONST : 0.0;
+}
+// the pulse at time t (whole field hook, its one nonzero component)
+__device__ __forceinline__ double q_pulse_exact(const QExact& X, double t) {
+    double pl[3] = {0.0, 0.0, 0.0};
+    st_field_pulse(t, X.pa, X.pw, X.axis, pl);
+    return X.axis == 0 ? pl[0] : (X.axis == 1 ? pl[1] : pl[2]);
+}
+// Bloch's y x omega at time t, component c (rhs_exact, st_device.h); pulse:
+// the pulse's value at t
+__device__ __forceinline__ double q_rhs_exact(const QExact& X, bool gravity, double t, double t0, double y, double pulse) {
+    const double d = t - t0;
+    double p = X.p0 + X.v0 * d, v = X.v0;
+    if (gravity) {
+        p = p + (X.hg * d) * d;
+        v = v + X.gg * d;
+    }
+    const d3 r = q_vec(p);
+    const double g = r.x * X.G0 + r.y * X.G1 + r.z * X.G2;
+    const double cr = q_next1(v) * X.Eb - q_next2(v) * X.Ea;
+    const double B = (((X.mine ? pulse : 0.0) + X.B0) + cr * IC2) + g;
+    const double w = B * X.gamma;
+    return q_next1(y) * q_next2(w) - q_next2(y) * q_next1(w);
+}
+// dop_trial_exact (st_integrators.h) on a quad.  The pulse's cosines are
+// split over the quad as in q_trial_fast.
+template <bool PULSE>
+__device__ __forceinline__ int q_trial_exact(const SimParams& P, const DopTab& T, QDop& D, double& y, double& h,
+                                             double t0, const QExact& X, uint32_t& nacc, uint32_t& nrej) {
+    if (D.nstep > P.nmax) return -1;
+    if ((D.x + 1.01 * h - D.xf) * D.posneg > 0.0) {
+        h = D.xf - D.x;
+        D.last = 1;
+    }
+    if (h < P.hmin && D.last != 1) h = P.hmin;
+    D.nstep++;
+    const double x = D.x, xph = x + h;
+    const bool gravity = P.gravity;
+    double hp0 = 0.0, hp1 = 0.0, hp2 = 0.0;
+    if constexpr (PULSE) {
+        if (X.axis >= 0) {
+            const uint32_t l = __lane_id() & 3u;
+            hp0 = q_pulse_exact(X, x + (l == 0 ? T.c2 : l == 1 ? T.c3 : l == 2 ? T.c4 : T.c5) * h);
+            hp1 = q_pulse_exact(X, x + (l == 0 ? T.c6 : l == 1 ? T.c7 : l == 2 ? T.c8 : T.c9) * h);
+            hp2 = q_pulse_exact(X, l == 0 ? x + T.c10 * h : l == 1 ? x + T.c11 * h : xph);
+        }
+    }
+#define QX(TT, LANE, HP) q_rhs_exact(X, gravity, (TT), t0, yy, PULSE ? q_all<LANE>(HP) : 0.0)
+    const double k1 = D.k1;
+    double yy = y + k1 * (h * T.a21);
+    const double k2 = QX(x + T.c2 * h, 0, hp0);
+    yy = y + h * (T.a31 * k1 + T.a32 * k2);
+    const double k3 = QX(x + T.c3 * h, 1, hp0);
+    yy = y + h * (T.a41 * k1 + T.a43 * k3);
+    const double k4 = QX(x + T.c4 * h, 2, hp0);
+    yy = y + h * (T.a51 * k1 + T.a53 * k3 + T.a54 * k4);
+    const double k5 = QX(x + T.c5 * h, 3, hp0);
+    yy = y + h * (T.a61 * k1 + T.a64 * k4 + T.a65 * k5);
+    const double k6 = QX(x + T.c6 * h, 0, hp1);
+    yy = y + h * (T.a71 * k1 + T.a74 * k4 + T.a75 * k5 + T.a76 * k6);
+    const double k7 = QX(x + T.c7 * h, 1, hp1);
+    yy = y + h * (T.a81 * k1 + T.a84 * k4 + T.a85 * k5 + T.a86 * k6 + T.a87 * k7);
+    const double k8 = QX(x + T.c8 * h, 2, hp1);
+    yy = y + h * (T.a91 * k1 + T.a94 * k4 + T.a95 * k5 + T.a96 * k6 + T.a97 * k7 + T.a98 * k8);
+    const double k9 = QX(x + T.c9 * h, 3, hp1);
+    yy = y + h * (T.a101 * k1 + T.a104 * k4 + T.a105 * k5 + T.a106 * k6 + T.a107 * k7 + T.a108 * k8 + T.a109 * k9);
+    const double k10 = QX(x + T.c10 * h, 0, hp2);
+    yy = y + h * (T.a111 * k1 + T.a114 * k4 + T.a115 * k5 + T.a116 * k6 + T.a117 * k7 + T.a118 * k8 + T.a119 * k9 + T.a1110 * k10);
+    const double k11 = QX(x + T.c11 * h, 1, hp2);
+    yy = y + h * (T.a121 * k1 + T.a124 * k4 + T.a125 * k5 + T.a126 * k6 + T.a127 * k7 + T.a128 * k8 + T.a129 * k9 + T.a1210 * k10 + T.a1211 * k11);
+    const double k12 = QX(xph, 2, hp2);
+#undef QX
+    const double b = T.b1 * k1 + T.b6 * k6 + T.b7 * k7 + T.b8 * k8 + T.b9 * k9 + T.b10 * k10 + T.b11 * k11 + T.b12 * k12;
+    const double y1 = y + h * b;
+    const double sk = P.atol + P.rtol * max_d(fabs(y), fabs(y1));
+    d3 e = q_vec((b - T.bhh1 * k1 - T.bhh2 * k9 - T.bhh3 * k12) / sk);
+    const double err2 = 0.0 + (e.x * e.x + e.y * e.y + e.z * e.z);
+    e = q_vec((T.er1 * k1 + T.er6 * k6 + T.er7 * k7 + T.er8 * k8 + T.er9 * k9 + T.er10 * k10 + T.er11 * k11 + T.er12 * k12) / sk);
+    double err = 0.0 + (e.x * e.x + e.y * e.y + e.z * e.z);
+    double deno = err + 0.01 * err2;
+    if (deno <= 0.0) deno = 1.0;
+    err = fabs(h) * err * sqrt(1.0 / (deno * 3.0));
+    const double fac11 = pow(err, P.expo1);
+    double fac = P.pow_beta_on ? fac11 / pow(D.facold, P.beta) : fac11 / 1.0;
+    fac = max_d(P.facc2, min_d(P.facc1, fac / P.safe));
+    double hnew = h / fac;
+    if (err <= 1.0 || P.fixed) {
+        D.facold = max_d(err, 1.0E-4);
+        nacc++;
+        D.k1 = q_rhs_exact(X, gravity, xph, t0, y1, PULSE ? q_all<2>(hp2) : 0.0);
+        y = y1;
+        D.x = xph;
+        if (D.last) return 1;
+        if (fabs(hnew) > P.hmax) hnew = D.posneg * P.hmax;
+        if (D.reject) hnew = D.posneg * min_d(fabs(hnew), fabs(h));
+        D.reject = 0;
+    } else {
+        nrej++;
+        hnew = h / min_d(P.facc1, fac11 / P.safe);
+        D.reject = 1;
+        D.last = 0;
+    }
+    if (!P.fixed) h = hnew;
+    return 0;
+}
+
 // The products make_poly reads, for the lane's components a = c+1 and b = c+2.
 __device__ __forceinline__ void q_pulse_load(QPulse& pl, const Phys& F, uint32_t c, double sign = 1.0) {
     const int32_t a = c == 2 ? 0 : (int32_t)c + 1, b = c == 0 ? 2 : (int32_t)c - 1;
@@ -372,8 +507,8 @@ __device__ __forceinline__ void q_make_poly(QPoly& q, const Phys& F, const d3& p
 __device__ __forceinline__ void quad_block(const RunArgs& R, uint32_t pid, int32_t k, uint32_t c, double y) {
     if (R.blocks) reinterpret_cast<double*>(R.blocks + (uint64_t)k * R.block_bytes + 56 * (uint64_t)R.n)[3 * (uint64_t)pid + c] = y;
 }
-template <bool BATCH, bool PULSE>
-__device__ __forceinline__ void quad_spin_fast() {
+template <int VAR, bool BATCH, bool PULSE>
+__device__ __forceinline__ void quad_spin() {
     auto args = []() -> const QuadArgs& { return kernel_args<QuadArgs>(); };
     const uint32_t lane = __lane_id();
     const uint32_t c = (lane & 3u) == 3u ? 0u : (lane & 3u);   // lane 3 repeats lane 0
@@ -390,7 +525,12 @@ __device__ __forceinline__ void quad_spin_fast() {
         __syncthreads();
     }
     QPulse pl;
-    if constexpr (PULSE && !BATCH) q_pulse_load(pl, shared_phys, c);
+    QExact X;
+    auto physics = [&](const Phys& F) {
+        if constexpr (VAR == VAR_EXACT) q_exact_load(X, args().P, F, c);
+        else if constexpr (PULSE) q_pulse_load(pl, F, c);
+    };
+    if constexpr (!BATCH) physics(shared_phys);
     SpinLane L;      // (S unused: the lane's component is y)
     double y = 0.0;
     QDop dop;
@@ -409,7 +549,7 @@ __device__ __forceinline__ void quad_spin_fast() {
         if (i >= n_list) return;
         spin_load<BATCH>(D, A, A.list[i], L);
         y = q_pick(L.S, c);
-        if constexpr (PULSE && BATCH) q_pulse_load(pl, A.phys[L.cfg], c);
+        if constexpr (BATCH) physics(A.phys[L.cfg]);
         if (L.nrec > 0) nxt = load_rec(rec_at_seq(A, L.pid, 0, L.page));
         phase = S_NEXT;
     };
@@ -437,20 +577,29 @@ __device__ __forceinline__ void quad_spin_fast() {
                 if (rec.flags & R_FIRST) L.tempH = L.h;
                 if ((rec.flags & R_INTEGRATE) && !L.stopped) {
                     seg_t0 = L.t_spin;
-                    q_make_poly(q, BATCH ? A.phys[L.cfg] : shared_phys, d3{rec.px, rec.py, rec.pz}, d3{rec.vx, rec.vy, rec.vz}, c);
                     dop.x = seg_t0;
                     dop.xf = rec.t;
                     dop.facold = 1.0E-4;
                     dop.last = 0;
                     dop.reject = 0;
                     dop.nstep = 0;
-                    double wa = q.a0, wb = q.b0;
-                    if constexpr (PULSE) {
-                        const double cosv = pl.on ? phase_cos(pl.pw * seg_t0) : 0.0;
-                        wa = __builtin_fma(pl.ma, cosv, wa);
-                        wb = __builtin_fma(pl.mb, cosv, wb);
+                    if constexpr (VAR == VAR_EXACT) {
+                        dop.posneg = sign_d(1.0, rec.t - seg_t0);
+                        X.p0 = q_pick(d3{rec.px, rec.py, rec.pz}, c);
+                        X.v0 = q_pick(d3{rec.vx, rec.vy, rec.vz}, c);
+                        dop.k1 = q_rhs_exact(X, args().P.gravity, seg_t0, seg_t0, y,
+                                             PULSE && X.axis >= 0 ? q_pulse_exact(X, seg_t0) : 0.0);
+                    } else {
+                        q_make_poly(q, BATCH ? A.phys[L.cfg] : shared_phys, d3{rec.px, rec.py, rec.pz},
+                                    d3{rec.vx, rec.vy, rec.vz}, c);
+                        double wa = q.a0, wb = q.b0;
+                        if constexpr (PULSE) {
+                            const double cosv = pl.on ? phase_cos(pl.pw * seg_t0) : 0.0;
+                            wa = __builtin_fma(pl.ma, cosv, wa);
+                            wb = __builtin_fma(pl.mb, cosv, wb);
+                        }
+                        dop.k1 = q_cross(y, wa, wb);
                     }
-                    dop.k1 = q_cross(y, wa, wb);
                     L.seg++;
                     if (R.trace && L.pid == R.trace_pid) {
                         const d3 S = q_vec(y);
@@ -471,7 +620,9 @@ __device__ __forceinline__ void quad_spin_fast() {
             }
         }
         if (phase == S_INT) {
-            const int st = q_trial_fast<false, PULSE>(args().P, T, dop, y, L.tempH, seg_t0, q, pl, L.acc, L.rej, nullptr);
+            int st;
+            if constexpr (VAR == VAR_EXACT) st = q_trial_exact<PULSE>(args().P, T, dop, y, L.tempH, seg_t0, X, L.acc, L.rej);
+            else st = q_trial_fast<false, PULSE>(args().P, T, dop, y, L.tempH, seg_t0, q, pl, L.acc, L.rej, nullptr);
             if (st != 0) {
                 const PipeArgs& A = args().A;
                 const RunArgs& R = A.R;
@@ -508,9 +659,9 @@ __device__ __forceinline__ void quad_spin_fast() {
     flush_counters(args().A.R.work, sum);
 }
 
-template <bool BATCH, bool PULSE>
+template <int VAR, bool BATCH, bool PULSE>
 __global__ __launch_bounds__(256, 2) void k_spin_quad(const QuadArgs) {
-    quad_spin_fast<BATCH, PULSE>();
+    quad_spin<VAR, BATCH, PULSE>();
 }
 
 // ---------------------------------------------------------------------------

@@ -37,7 +37,8 @@ def run(p, times):
 # 1; a ragged wave; one particle past one per SIMD (two per wave)
 @pytest.mark.parametrize("n", [1, 17, 1025])
 @pytest.mark.parametrize("kind,variant", [("he3", st.VARIANT_FAST), ("dressing", st.VARIANT_FAST),
-                                          ("neutron", st.VARIANT_FAST)])
+                                          ("neutron", st.VARIANT_FAST), ("he3", st.VARIANT_EXACT),
+                                          ("dressing", st.VARIANT_EXACT), ("neutron", st.VARIANT_EXACT)])
 def test_quad_equals_one_lane(kind, variant, n):
     print(f"[quad] {kind} variant={variant} n={n}", flush=True)
     axis = 1 if kind == "dressing" else 2
