@@ -129,10 +129,23 @@ ST_HD __forceinline__ uint64_t xo_next(Rng& s) {
     s.w = (s.z << 45) | (s.z >> 19);
     return r;
 }
-// src/particle.cpp:72-83 (53-bit integer -> double is exact)
-ST_HD __forceinline__ double uni(Rng& s) { return (double)(xo_next(s) >> 11) * 0x1.0p-53; }
+// src/particle.cpp:72-83 (53-bit integer -> double is exact, so its halves may
+// be scaled and added instead: every step of either form is exact)
+ST_HD __forceinline__ double uni(Rng& s) {
+    const uint64_t r = xo_next(s);
+    const uint32_t hi = (uint32_t)(r >> 43), lo = (uint32_t)(r >> 11);
+    return __builtin_fma((double)lo, 0x1.0p-53, (double)hi * 0x1.0p-21);
+}
 // src/particle.cpp:85-87
 ST_HD __forceinline__ double uni_lh(Rng& s, double lo, double hi) { return uni(s) * (hi - lo) + lo; }
+
+// uni_lh(s, -1, 1): u*2 and the two halves are exact, so the one rounding of
+// u*2 - 1 is that of the last FMA
+ST_HD __forceinline__ double uni_pm1(Rng& s) {
+    const uint64_t r = xo_next(s);
+    const uint32_t hi = (uint32_t)(r >> 43), lo = (uint32_t)(r >> 11);
+    return __builtin_fma((double)lo, 0x1.0p-52, __builtin_fma((double)hi, 0x1.0p-20, -1.0));
+}
 
 // src/particle.cpp:89-107: Marsaglia polar method, spare cached in the state
 ST_HD inline double normal(Rng& s, double mean, double sd) {
@@ -142,8 +155,8 @@ ST_HD inline double normal(Rng& s, double mean, double sd) {
     }
     double ts, tu, tv;
     do {
-        tu = uni_lh(s, -1.0, 1.0);
-        tv = uni_lh(s, -1.0, 1.0);
+        tu = uni_pm1(s);
+        tv = uni_pm1(s);
         ts = tu * tu + tv * tv;
     } while (ts >= 1.0 || ts == 0.0);
     ts = sqrt(-2.0 * log(ts) / ts);
@@ -157,8 +170,8 @@ ST_HD __forceinline__ double maxboltz(Rng& s, double sqrtkT_m) { return normal(s
 ST_HD __forceinline__ void polar_pair(Rng& s, double& first, double& second) {
     double ts, tu, tv;
     do {
-        tu = uni_lh(s, -1.0, 1.0);
-        tv = uni_lh(s, -1.0, 1.0);
+        tu = uni_pm1(s);
+        tv = uni_pm1(s);
         ts = tu * tu + tv * tv;
     } while (ts >= 1.0 || ts == 0.0);
     ts = sqrt(-2.0 * log(ts) / ts);
@@ -384,18 +397,10 @@ ST_HD __forceinline__ void flip_v(d3& v, char wh) {
 // same operations, same operands, same stream order.
 enum { JOB_NONE = 0, JOB_GAS = 1, JOB_DIFFUSE = 2 };
 
-// src/particle.cpp:306-328: Lambertian re-emission from wall wh at the
-// post-flight speed Vel (v: the post-flight velocity, for the signs); the
-// reference draws phi and theta before it looks at the wall id, and stops the
-// particle on an edge or corner.
-ST_HD inline void diffuse_job(d3& v, bool& stop, char wh, double Vel, Rng& rng) {
-    const double phi = acos(sqrt(uni(rng)));
-    const double theta = unif02pi(rng);
-    // sincos shares one argument reduction between the two values
-    // (each equals the separate sin / cos of the device libm)
-    double sp, cp, sth, cth;
-    sincos(phi, &sp, &cp);
-    sincos(theta, &sth, &cth);
+// The re-emitted velocity from the sine and cosine of phi (sp, cp) and theta
+// (sth, cth).
+ST_HD __forceinline__ void diffuse_emit(d3& v, bool& stop, char wh, double Vel, double sp, double cp, double sth,
+                                        double cth) {
     if (wh == 'x') {
         v.x = -1.0 * psgn(v.x) * Vel * cp;
         v.y = -Vel * sp * cth;
@@ -411,6 +416,20 @@ ST_HD inline void diffuse_job(d3& v, bool& stop, char wh, double Vel, Rng& rng) 
     } else {
         stop = true;
     }
+}
+// src/particle.cpp:306-328: Lambertian re-emission from wall wh at the
+// post-flight speed Vel (v: the post-flight velocity, for the signs); the
+// reference draws phi and theta before it looks at the wall id, and stops the
+// particle on an edge or corner.
+ST_HD inline void diffuse_job(d3& v, bool& stop, char wh, double Vel, Rng& rng) {
+    const double phi = acos(sqrt(uni(rng)));
+    const double theta = unif02pi(rng);
+    // sincos shares one argument reduction between the two values
+    // (each equals the separate sin / cos of the device libm)
+    double sp, cp, sth, cth;
+    sincos(phi, &sp, &cp);
+    sincos(theta, &sth, &cth);
+    diffuse_emit(v, stop, wh, Vel, sp, cp, sth, cth);
 }
 
 // A gas collision: the next gas time when it was deferred from
@@ -482,6 +501,13 @@ ST_HD inline void move_and_collide(const SimParams& P, const Phys& F, Kin& K, Rn
 // src/particle.cpp:412-444
 ST_HD inline void sanity(const SimParams& P, Kin& K) {
     const double tol = 1.0e-15;
+    // All tests at once for the particle that passes them: a position within
+    // the walls is no NaN, and a finite sum has no infinite or NaN term.  (A
+    // sum that is not finite for another reason goes through the tests below.)
+    if (fabs(K.pos.x) <= P.Lx / 2.0 + tol && fabs(K.pos.y) <= P.Ly / 2.0 + tol && fabs(K.pos.z) <= P.Lz / 2.0 + tol &&
+        __builtin_isfinite(((K.t_old + K.t) + (K.pos_old.x + K.pos_old.y)) + ((K.pos_old.z + K.v.x) + (K.v.y + K.v.z)) +
+                           (K.v_old.x + (K.v_old.y + K.v_old.z))))
+        return;
     if (fabs(K.pos.x) > P.Lx / 2.0 + tol || fabs(K.pos.y) > P.Ly / 2.0 + tol ||
         fabs(K.pos.z) > P.Lz / 2.0 + tol) {
         K.stop = true; K.failure = 1; return;

@@ -216,7 +216,7 @@ struct st_handle {
     bool initialized = false;
     double last_target = 0.0;
     int grid_fused = 0, grid_spin = 0;
-    int n_simd = 0;                // SIMDs of the device (four per compute unit)
+    int n_simd = 1024;             // SIMDs of the device (four per compute unit)
     // pipeline buffers
     char* d_recs = nullptr;
     uint32_t rec_cap = 0;          // C
@@ -516,7 +516,6 @@ static int persistent_grid(st_handle* h, const void* sym, int* cache) {
         HIPCHK(h, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
         HIPCHK(h, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, sym, 256, 0));
         *cache = cus * std::max(per_cu, 1);
-        h->n_simd = 4 * cus;
     }
     return ST_OK;
 }
@@ -623,11 +622,21 @@ static int save_ckpt(st_handle* h, const uint32_t* list, uint32_t n_list) {
 // (k_kin over all n lanes, k_spin over its persistent grid, k_fixup over 64
 // groups); each reads this chunk's list length and failure count on the
 // device.  The graph holds the run's arguments, so it is captured per call.
-// The kinematics kernel over n_lanes lanes, kbs lanes per workgroup.
-static void launch_kin(st_handle* h, const DevState& D, const PipeArgs& A, uint32_t n_lanes, int kbs) {
-    const dim3 grid((n_lanes + kbs - 1) / kbs);
-    if (h->batch) hipLaunchKernelGGL(k_kin<true>, grid, dim3(kbs), 0, h->stream, h->P, D, A);
-    else hipLaunchKernelGGL(k_kin<false>, grid, dim3(kbs), 0, h->stream, h->P, D, A);
+// The kinematics kernel over a list of n particles, kbs lanes per workgroup.
+// Up to 32 particles per SIMD a wave takes as few of them (a power of two) as
+// leave one wave per SIMD; the measured line is at k_kin.
+template <bool BATCH>
+static void launch_kin_b(st_handle* h, const DevState& D, const PipeArgs& A, uint32_t n, int kbs) {
+    uint32_t ppw = 1;
+    while (ppw < 64 && ppw * (uint32_t)h->n_simd < n) ppw *= 2;
+    const uint32_t per_group = ppw * (uint32_t)(kbs / 64);
+    const dim3 grid((n + per_group - 1) / per_group);
+    if (ppw < 64) hipLaunchKernelGGL((k_kin<BATCH, true>), grid, dim3(kbs), 0, h->stream, h->P, D, A, ppw);
+    else hipLaunchKernelGGL((k_kin<BATCH, false>), grid, dim3(kbs), 0, h->stream, h->P, D, A, ppw);
+}
+static void launch_kin(st_handle* h, const DevState& D, const PipeArgs& A, uint32_t n, int kbs) {
+    if (h->batch) launch_kin_b<true>(h, D, A, n, kbs);
+    else launch_kin_b<false>(h, D, A, n, kbs);
 }
 
 static int run_pipeline_graph(st_handle* h, PipeArgs A, SpinFn spin, int kbs) {
@@ -985,6 +994,9 @@ static int create_common(const st_options& opt, const st_ext& x, uint32_t n, st_
     h->any_pulse = h->P.ph.pulse_on != 0;
     h->state_bytes = (size_t)field_stride(h->n) * F_COUNT;
     if (hipGetDevice(&h->device) != hipSuccess) h->device = -1;
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, std::max(h->device, 0)) == hipSuccess)
+        h->n_simd = 4 * cus;
     hipError_t e = hipMalloc(&h->state, h->state_bytes);
     if (e == hipSuccess) e = hipMalloc(&h->d_work, N_WORK * sizeof(unsigned long long));
     if (e == hipSuccess) e = hipMalloc(&h->d_small, 256);

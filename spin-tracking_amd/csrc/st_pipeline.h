@@ -202,14 +202,15 @@ __device__ __forceinline__ void put_rec(char* at, double t, const d3& p, const d
 //   kin_end    sanity check, watchdog, record flags, interval close.
 struct KinEvent {
     bool first;      // the event opened an interval
-    bool empty;      // no event: the interval closes at once (rt/rp/rv, flags set)
+    bool empty;      // no event: the interval closes at once
     bool gas_draw;   // the gas job draws the next gas time first
     int job;         // JOB_NONE / JOB_GAS / JOB_DIFFUSE
     double Vel;      // post-flight speed (the re-emissions' input)
 };
 
+// (store: this lane writes the particle's snapshot entries)
 __device__ __forceinline__ void kin_begin(const SimParams& P, const Phys& F, const RunArgs& R, KinLane& L, KinEvent& E,
-                                          double& rt, d3& rp, d3& rv) {
+                                          bool store = true) {
     E.first = false;
     E.empty = false;
     E.gas_draw = false;
@@ -229,10 +230,7 @@ __device__ __forceinline__ void kin_begin(const SimParams& P, const Phys& F, con
         if (!moves || L.K.stop) {
             // the reference's loop body never runs this interval
             if (moves) L.tf = tgt;
-            rt = L.K.t;
-            rp = L.K.pos;
-            rv = L.K.v;
-            kin_block(R, L);
+            if (store) kin_block(R, L);
             L.k++;
             if (L.k >= R.n_targets) L.done = true;
             E.empty = true;
@@ -250,8 +248,13 @@ __device__ __forceinline__ void kin_begin(const SimParams& P, const Phys& F, con
 }
 
 __device__ __forceinline__ uint64_t kin_end(const SimParams& P, const RunArgs& R, int32_t integ, KinLane& L,
-                                            const KinEvent& E, double& rt, d3& rp, d3& rv) {
-    if (E.empty) return R_EMPTY | R_IEND;
+                                            const KinEvent& E, double& rt, d3& rp, d3& rv, bool store = true) {
+    if (E.empty) {
+        rt = L.K.t;
+        rp = L.K.pos;
+        rv = L.K.v;
+        return R_EMPTY | R_IEND;
+    }
     // src/particle.cpp:757
     sanity(P, L.K);
     if (++L.n_events > R.max_events && L.K.failure == 0) {
@@ -274,7 +277,7 @@ __device__ __forceinline__ uint64_t kin_end(const SimParams& P, const RunArgs& R
     L.n_steps += 1;
     if (L.K.finished || L.K.stop) {
         fl |= R_IEND;
-        kin_block(R, L);
+        if (store) kin_block(R, L);
         L.k++;
         L.open = false;
         if (L.k >= R.n_targets) L.done = true;
@@ -290,7 +293,7 @@ __device__ __forceinline__ void run_job(const Phys& F, KinLane& L, const KinEven
 __device__ __forceinline__ uint64_t kin_step(const SimParams& P, const Phys& F, const RunArgs& R, int32_t integ, KinLane& L,
                                              double& rt, d3& rp, d3& rv) {
     KinEvent E;
-    kin_begin(P, F, R, L, E, rt, rp, rv);
+    kin_begin(P, F, R, L, E);
     if (!E.empty) run_job(F, L, E);
     return kin_end(P, R, integ, L, E, rt, rp, rv);
 }
@@ -309,32 +312,207 @@ __global__ __launch_bounds__(256) void k_begin_run(const DevState D, uint32_t n,
     list[i] = i;
 }
 
-// waiting lanes that start a wave's diffuse re-emissions (He-3, 1M, 4 x 0.5 s:
-// k_kin 105 ms at 4, 106 at 8, 114 at 16, 108 without the wait); a particle
-// whose walls are mostly diffuse takes its re-emission at once
+// ---------------------------------------------------------------------------
+// k_kin: the event loop, in two forms
+// ---------------------------------------------------------------------------
+// What bounds it is the vector issue rate, and in a wave of 64 particles most
+// of it goes to the union of their branches: of 64 He-3 lanes about 25 have a
+// gas collision and 2 a diffuse wall on nearly every trip.  SPREAD = false,
+// for lists that fill the chip: 64 particles a wave, each lane calling for
+// itself, only the diffuse re-emissions held back for four waiting lanes.
+//
+// SPREAD = true, for lists of at most 32 particles per SIMD: a wave holds ppw
+// particles (a power of two), so that fewer particles' branches meet in it.
+// Its lanes beyond them repeat the first ones (slot = lane % ppw) and store
+// nothing; with those lanes masked off the vector instructions would run at
+// half rate (FMAs under fixed masks, four waves on a compute unit: 5.6 cycles
+// each with 10 to 64 active lanes, 10-14 with 1 to 8).  The idle lanes also
+// take over calls: those of a trip that need a logarithm (or a sincos) post
+// their arguments to consecutive places of an LDS array, all 64 lanes
+// evaluate one each, and the owners pick up their results.  Draws, operations
+// and operands are those of kin_step, in its order per particle.
+// He-3 (gas, 5% diffuse walls), us per event against 64 a wave: 1,000
+// particles 3.3 and 6.3 (one a wave), 2,047 3.9 and 6.3, 8,192 5.2 and 6.6,
+// 16,384 5.7 and 6.4 (sixteen a wave), 32,768 6.3 and 6.8; with 64 particles a
+// wave the shared calls are the slower form (1M: 46.0 and 42.9 ns).
+struct WaveSlots {
+    uint32_t slot;    // the lane's particle within the wave
+    bool real;        // the lane that stores for it
+    __device__ __forceinline__ uint32_t rank(uint64_t mask) const {
+        return (uint32_t)__popcll(mask & ((1ull << slot) - 1ull));
+    }
+};
+// LDS operations of one wave execute in order; this keeps the compiler from
+// moving them across an exchange
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+constexpr uint32_t KIN_EXCHANGE = 256;   // doubles per wave: 192 logarithms, or 64 pairs of sincos
+
+// The accepted polar-method candidates (polar_pair, st_device.h) of the lanes
+// with `left` of them to draw, one or two each, all lanes active throughout:
+// a lane goes on to its second pair at once, so the wave runs as many trips as
+// its lane with the most attempts in all.  as = 1 where none was drawn.
+__device__ __forceinline__ void wave_polar(Rng& rng, int left, double& au, double& av, double& as, double& bu,
+                                           double& bv, double& bs) {
+    au = av = bu = bv = 0.0;
+    as = bs = 1.0;
+    while (__any(left > 0)) {
+        Rng r = rng;
+        const double u = uni_pm1(r), v = uni_pm1(r);
+        const double q = u * u + v * v;
+        if (left > 0) {
+            rng.x = r.x; rng.y = r.y; rng.z = r.z; rng.w = r.w;
+            // the newest candidate in b; an accepted first one moves to a
+            const bool ok = q < 1.0 && q != 0.0;
+            if (ok) {
+                au = bu; av = bv; as = bs;
+                bu = u; bv = v; bs = q;
+                --left;
+            }
+        }
+    }
+}
+
+// gas_job (st_device.h) for the lanes with `need`.
+__device__ __forceinline__ void wave_gas(KinLane& L, const KinEvent& E, const Phys& F, bool need, const WaveSlots& W,
+                                         double* buf) {
+    const uint32_t lane = __lane_id();
+    const bool polar = need && (F.dist == 'M' || F.dist == 'C');
+    const bool draw = need && E.gas_draw;
+    const bool had = L.rng.has;
+    double ue = 1.0;
+    if (draw) ue = 1.0 - uni(L.rng);
+    const bool two = polar && !had;
+    // (a lane with one pair has it in b)
+    double au, av, as, bu, bv, bs;
+    wave_polar(L.rng, polar ? (had ? 1 : 2) : 0, au, av, as, bu, bv, bs);
+    // post the arguments: gas times, last pairs, first pairs of two
+    const uint64_t m0 = __ballot(draw && W.real), m1 = __ballot(polar && W.real), m2 = __ballot(two && W.real);
+    const uint32_t n0 = (uint32_t)__popcll(m0), n1 = n0 + (uint32_t)__popcll(m1), n2 = n1 + (uint32_t)__popcll(m2);
+    const uint32_t i0 = W.rank(m0), i1 = n0 + W.rank(m1), i2 = n1 + W.rank(m2);
+    if (W.real) {
+        if (draw) buf[i0] = ue;
+        if (polar) buf[i1] = bs;
+        if (two) buf[i2] = as;
+    }
+    wave_fence();
+    for (uint32_t base = 0; base < n2; base += 64) {
+        const uint32_t i = base + lane;
+        const double x = i < n2 ? buf[i] : 1.0;
+        const double l = log(x);
+        const double f = sqrt(-2.0 * l / x);
+        if (i < n2) buf[i] = i < n0 ? l : f;
+    }
+    wave_fence();
+    if (draw) L.K.next_gas += -F.tc * buf[i0];
+    if (polar) {
+        // the last pair drawn, and its factor
+        const double fb = buf[i1], b0 = 0.0 + 1.0 * bu * fb, b1 = bv * fb, sp = L.rng.spare;
+        double n0_, n1_, n2_;
+        if (had) {
+            n0_ = sp * 1.0 + 0.0;
+            n1_ = b0;
+            n2_ = b1 * 1.0 + 0.0;
+        } else {
+            const double fa = buf[i2];
+            n0_ = 0.0 + 1.0 * au * fa;
+            n1_ = (av * fa) * 1.0 + 0.0;
+            n2_ = b0;
+        }
+        L.rng.spare = b1;
+        L.rng.has = !had;
+        if (F.dist == 'M') {
+            L.K.v = d3{n0_ * F.sqrtKT_m, n1_ * F.sqrtKT_m, n2_ * F.sqrtKT_m};
+        } else {
+            const double vn = len3(d3{n0_, n1_, n2_});
+            const double Vel = len3(L.K.v);
+            L.K.v = d3{(Vel * n0_) / vn, (Vel * n1_) / vn, (Vel * n2_) / vn};
+        }
+    }
+    wave_fence();
+}
+
+// diffuse_job (st_device.h) for the lanes with `need`.
+__device__ __forceinline__ void wave_diffuse(KinLane& L, bool need, const WaveSlots& W, double* buf) {
+    const uint32_t lane = __lane_id();
+    double u1 = 0.5, theta = 0.0;
+    if (need) {
+        u1 = uni(L.rng);
+        theta = unif02pi(L.rng);
+    }
+    const double phi = acos(sqrt(u1)), Vel = len3(L.K.v);
+    const uint64_t m = __ballot(need && W.real);
+    const uint32_t w = (uint32_t)__popcll(m), i = W.rank(m);
+    if (need && W.real) {
+        buf[i] = phi;
+        buf[w + i] = theta;
+    }
+    wave_fence();
+    for (uint32_t base = 0; base < 2 * w; base += 64) {
+        const uint32_t k = base + lane;
+        double sn, cs;
+        sincos(k < 2 * w ? buf[k] : 0.0, &sn, &cs);
+        if (k < 2 * w) {
+            buf[k] = sn;
+            buf[128 + k] = cs;
+        }
+    }
+    wave_fence();
+    if (need) {
+        const double sp = buf[i], cp = buf[128 + i], sth = buf[w + i], cth = buf[128 + w + i];
+        diffuse_emit(L.K.v, L.K.stop, L.K.wall_hit, Vel, sp, cp, sth, cth);
+    }
+    wave_fence();
+}
+
+// waiting lanes that start a wave's diffuse re-emissions; a particle whose
+// walls are mostly diffuse takes its re-emission at once
 constexpr int DIFFUSE_BATCH = 4;
-template <bool BATCH>
-__global__ __launch_bounds__(256) void k_kin(const SimParams P, const DevState D, const PipeArgs A) {
-    const uint32_t li = blockIdx.x * blockDim.x + threadIdx.x;
+template <bool BATCH, bool SPREAD>
+__global__ __launch_bounds__(256, 3) void k_kin(const SimParams P, const DevState D, const PipeArgs A, uint32_t ppw) {
+    __shared__ double exchange[SPREAD ? 4 : 1][SPREAD ? KIN_EXCHANGE : 1];
+    double* const buf = exchange[SPREAD ? threadIdx.x >> 6 : 0];
+    if constexpr (!SPREAD) ppw = 64;
+    const uint32_t n_list = list_len(A);
+    const uint32_t base = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * ppw;
+    if (base >= n_list) return;   // (a whole wave)
     unsigned long long cnt[2] = {0, 0};   // events, trips
-    if (li < list_len(A)) {
+    WaveSlots W;
+    bool live = true;
+    {
+        const uint32_t lane = __lane_id();
+        W.slot = lane & (ppw - 1u);
+        if constexpr (SPREAD) {
+            if (base + W.slot >= n_list) W.slot = 0;   // the lanes past the list repeat the first particle
+            W.real = W.slot == lane;
+        } else {
+            live = base + lane < n_list;
+            W.slot = live ? lane : 0;
+            W.real = true;
+        }
+    }
+    if (live) {
         KinLane L;
-        kin_load(D, A.list[li], L);
+        kin_load(D, A.list[base + W.slot], L);
         const Phys& F = lane_phys<BATCH>(P, D, A.phys, L.pid);
         // back up the kinematic state for a possible spin-failure replay
-        const uint32_t o = L.pid * 8u;
-        const DevState B{A.backup, D.stride};
+        if (!SPREAD || W.real) {
+            const uint32_t o = L.pid * 8u;
+            const DevState B{A.backup, D.stride};
 #pragma unroll
-        for (int f = 0; f < N_KIN_FIELDS; ++f) B.st<uint64_t>(KIN_FIELDS[f], o, D.ld<uint64_t>(KIN_FIELDS[f], o));
+            for (int f = 0; f < N_KIN_FIELDS; ++f) B.st<uint64_t>(KIN_FIELDS[f], o, D.ld<uint64_t>(KIN_FIELDS[f], o));
+        }
         uint32_t j = 0, lim = A.no_recs ? 0xffffffffu : A.C, page = OVF_NONE, rpage = OVF_NONE;
         const double t0 = L.K.t;
         KinEvent E;
+        E.empty = true;
         bool pend = false;   // the event's diffuse re-emission waits for more lanes
-        const int batch = F.diffuse < 0.5 ? DIFFUSE_BATCH : 1;
-        double rt;
-        d3 rp, rv;
-        while (!L.done) {
-            if (!pend && j == lim) {
+        bool run = !L.done;  // the particle has events left in this chunk
+        const int batch = F.diffuse < 0.5 ? max(1, (int)(DIFFUSE_BATCH * ppw / 64u)) : 1;
+        for (;;) {
+            if (run && !pend && j == lim) {
                 // Chunk depth used up: continue on an overflow page if one is
                 // left and the particle is near its end -- its remaining time
                 // to the last output under twice what this chunk has covered
@@ -345,48 +523,67 @@ __global__ __launch_bounds__(256) void k_kin(const SimParams P, const DevState D
                 // chunk for their lanes (He-3, 1M, 20 x 0.5 s at the default
                 // depth: 1,432 ms with this rule, 1,455 ms taking pages for
                 // any particle, 1,538 ms with four times the covered time).
-                if (A.ovf_pages == 0) break;
-                double t_last = target_of(A.R, A.R.n_targets - 1);
-                if (A.R.stop_at) t_last = fmin(t_last, A.R.stop_at[L.pid]);
-                if (A.R.n_targets > 1 && !(t_last - L.K.t <= 2.0 * (L.K.t - t0))) break;
-                const uint32_t p = atomicAdd(A.ovf_head, 1u);
-                if (p >= A.ovf_pages) break;
-                if (page == OVF_NONE) A.ovf_first[L.pid] = p;
-                else A.ovf_link[page] = p;
-                page = p;
-                lim += OVF_PAGE;
-            }
-            if (!pend) {
-                kin_begin(P, F, A.R, L, E, rt, rp, rv);
-                if (!E.empty) {
-                    if (E.job == JOB_GAS)
-                        gas_job(L.K.v, L.K.next_gas, E.gas_draw, E.Vel, F.tc, F.sqrtKT_m, F.dist, L.rng);
-                    pend = E.job == JOB_DIFFUSE;
+                run = A.ovf_pages != 0;
+                if (run) {
+                    double t_last = target_of(A.R, A.R.n_targets - 1);
+                    if (A.R.stop_at) t_last = fmin(t_last, A.R.stop_at[L.pid]);
+                    if (A.R.n_targets > 1 && !(t_last - L.K.t <= 2.0 * (L.K.t - t0))) run = false;
+                }
+                if (run) {
+                    uint32_t p = 0;
+                    if (!SPREAD || W.real) p = atomicAdd(A.ovf_head, 1u);
+                    if constexpr (SPREAD) p = __shfl(p, W.slot);   // (a particle's lanes are here together)
+                    run = p < A.ovf_pages;
+                    if (run) {
+                        if (!SPREAD || W.real) {
+                            if (page == OVF_NONE) A.ovf_first[L.pid] = p;
+                            else A.ovf_link[page] = p;
+                        }
+                        page = p;
+                        lim += OVF_PAGE;
+                    }
                 }
             }
-            // The diffuse re-emission (acos and two sincos; about a sixth of
-            // this kernel's time, for ~3% of He-3 events) would run on almost
-            // every trip for a lane or two.  It runs once `batch` lanes of the
-            // wave wait for it, or when no running lane has other work;
-            // a waiting lane idles, its random stream untouched meanwhile, so
-            // every lane's events and draws are those of kin_step.
-            {
-                const uint64_t waiting = __ballot(pend), running = __ballot(1);
-                if (pend && (__popcll(waiting) >= batch || waiting == running)) {
-                    diffuse_job(L.K.v, L.K.stop, L.K.wall_hit, E.Vel, L.rng);
-                    pend = false;
-                }
+            const uint64_t running = __ballot(run && (!SPREAD || W.real));
+            if (running == 0) break;
+            bool gas = false;
+            if (run && !pend) {
+                kin_begin(P, F, A.R, L, E, !SPREAD || W.real);
+                gas = !E.empty && E.job == JOB_GAS;
+                pend = !E.empty && E.job == JOB_DIFFUSE;
+                // (the post-flight speed only where the re-emission keeps it)
+                if (!SPREAD && gas)
+                    gas_job(L.K.v, L.K.next_gas, E.gas_draw, F.dist == 'C' ? len3(L.K.v) : 0.0, F.tc, F.sqrtKT_m,
+                            F.dist, L.rng);
             }
-            if (pend) continue;
-            const uint64_t fl = kin_end(P, A.R, A.integ, L, E, rt, rp, rv);
-            if (!A.no_recs) put_rec(rec_at_seq(A, L.pid, j, rpage), rt, rp, rv, fl);
-            ++j;
-            cnt[0] += (fl & R_EMPTY) ? 0 : 1;
+            if (SPREAD && __any(gas)) wave_gas(L, E, F, gas, W, buf);
+            // The diffuse re-emissions run once `batch` lanes of the wave wait
+            // for them, or when no running lane has other work; a waiting lane
+            // idles, its random stream untouched meanwhile.
+            const uint64_t waiting = __ballot(pend && (!SPREAD || W.real));
+            if (waiting != 0 && (waiting == running || __any(pend && __popcll(waiting) >= batch))) {
+                if constexpr (SPREAD) wave_diffuse(L, pend, W, buf);
+                else if (pend) diffuse_job(L.K.v, L.K.stop, L.K.wall_hit, len3(L.K.v), L.rng);
+                pend = false;
+            }
+            if (run && !pend) {
+                double rt;
+                d3 rp, rv;
+                const uint64_t fl = kin_end(P, A.R, A.integ, L, E, rt, rp, rv, !SPREAD || W.real);
+                if (!SPREAD || W.real) {
+                    if (!A.no_recs) put_rec(rec_at_seq(A, L.pid, j, rpage), rt, rp, rv, fl);
+                    cnt[0] += (fl & R_EMPTY) ? 0 : 1;
+                }
+                ++j;
+                run = !L.done;
+            }
         }
-        cnt[1] = j;
-        A.seg_count[L.pid] = j;
-        kin_store(D, L);
-        if (!L.done) A.next_list[atomicAdd(A.next_count, 1u)] = L.pid;
+        if (!SPREAD || W.real) {
+            cnt[1] = j;
+            A.seg_count[L.pid] = j;
+            kin_store(D, L);
+            if (!L.done) A.next_list[atomicAdd(A.next_count, 1u)] = L.pid;
+        }
     }
     flush_counters(A.R.work + 4, cnt);
 }
