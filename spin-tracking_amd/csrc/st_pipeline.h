@@ -732,7 +732,9 @@ __device__ __forceinline__ void spin_body(const SimParams& P, const DevState& D,
                         const double nan = __builtin_nan("");
                         L.S = d3{nan, nan, nan};
                     }
-                    if (rec.flags & R_IEND) {
+                    // (after an integrator failure k_fixup writes the blocks:
+                    // the kinematics' later intervals are not the particle's)
+                    if ((rec.flags & R_IEND) && !L.stopped) {
                         spin_block(R, L);
                         L.k++;
                     }
@@ -774,8 +776,7 @@ __device__ __forceinline__ void spin_body(const SimParams& P, const DevState& D,
                     const double nan = __builtin_nan("");
                     L.S = d3{nan, nan, nan};
                 }
-                if ((rec.flags & R_IEND) || st < 0) {
-                    // (a failing particle's later blocks are written by k_fixup)
+                if ((rec.flags & R_IEND) && !L.stopped) {
                     spin_block(R, L);
                     L.k++;
                 }
