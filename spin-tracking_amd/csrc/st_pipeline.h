@@ -732,9 +732,7 @@ __device__ __forceinline__ void spin_body(const SimParams& P, const DevState& D,
                         const double nan = __builtin_nan("");
                         L.S = d3{nan, nan, nan};
                     }
-                    // (after an integrator failure k_fixup writes the blocks:
-                    // the kinematics' later intervals are not the particle's)
-                    if ((rec.flags & R_IEND) && !L.stopped) {
+                    if (rec.flags & R_IEND) {
                         spin_block(R, L);
                         L.k++;
                     }
@@ -771,12 +769,14 @@ __device__ __forceinline__ void spin_body(const SimParams& P, const DevState& D,
                         A.fail_list[3 * slot + 2] = (uint32_t)st;
                     }
                     L.stopped = true;
+                    L.nrec = 0;   // the later records are not the particle's
                 }
                 if (L.stopped || (rec.flags & R_STOP)) {
                     const double nan = __builtin_nan("");
                     L.S = d3{nan, nan, nan};
                 }
-                if ((rec.flags & R_IEND) && !L.stopped) {
+                // (k_fixup writes the blocks from a failing interval on)
+                if ((rec.flags & R_IEND) && st > 0) {
                     spin_block(R, L);
                     L.k++;
                 }

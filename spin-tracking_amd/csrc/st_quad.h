@@ -610,7 +610,7 @@ __device__ __forceinline__ void quad_spin() {
                     phase = S_INT;
                 } else {
                     if (rec.flags & R_STOP) y = __builtin_nan("");
-                    if ((rec.flags & R_IEND) && !L.stopped) {   // (spin_body: the blocks after a failure)
+                    if (rec.flags & R_IEND) {
                         if (owner) quad_block(R, L.pid, L.k, c, y);
                         L.k++;
                     }
@@ -644,9 +644,10 @@ __device__ __forceinline__ void quad_spin() {
                         }
                     }
                     L.stopped = true;
+                    L.nrec = 0;   // (spin_body: the records after a failure)
                 }
                 if (L.stopped || (cur_flags & R_STOP)) y = __builtin_nan("");
-                if ((cur_flags & R_IEND) && !L.stopped) {
+                if ((cur_flags & R_IEND) && st > 0) {
                     if (owner) quad_block(R, L.pid, L.k, c, y);
                     L.k++;
                 }
