@@ -461,10 +461,13 @@ static const void* spin_symbol(int variant, int integ, bool batch, bool pulse) {
 // 0.90 ms at 1,000, 1.96 and 1.27 ms at 16,384, 2.01 and 1.63 ms at 32,768,
 // 2.14 and 2.48 ms at 49,152 (neutrons x 0.5 s: 2.97 and 2.47 ms at 32,768,
 // 3.10 and 3.52 ms at 49,152).  The exact variant on the same He-3: 4.32 and
-// 1.96 ms, 4.41 and 2.33 ms, 4.50 and 3.54 ms, 4.55 and 4.58 ms.  0: the
-// integrator has no such kernel, or the field hooks have their own form.
+// 1.96 ms, 4.41 and 2.33 ms, 4.50 and 3.54 ms, 4.55 and 4.58 ms.  RK45,
+// neutrons x 0.5 ms: 10.7 and 8.2 ms at 16,384, 10.8 and 10.4 ms at 32,768,
+// 10.8 and 16.5 ms at 49,152 (exact 27.3 and 14.8, 27.4 and 23.6, 27.4 and
+// 32.5 ms).  0: the integrator has no such kernel, or the field hooks have
+// their own form.
 static uint32_t quad_limit(const st_handle* h) {
-    if (h->opt.integratorType != INT_DOP853 || !ST_FIELDS_POLYNOMIAL) return 0;
+    if ((h->opt.integratorType != INT_DOP853 && h->opt.integratorType != INT_RK45) || !ST_FIELDS_POLYNOMIAL) return 0;
     return 32u * (uint32_t)h->n_simd;
 }
 // particles per wave: one until every SIMD has a wave, then doubling to 16
@@ -477,19 +480,22 @@ static uint32_t quad_ppw(const st_handle* h, uint32_t n) {
 static uint32_t quad_grid(const st_handle* h, uint32_t n, uint32_t ppw) {
     return (std::min(2 * (uint32_t)h->n_simd, (n + ppw - 1) / ppw) + 3) / 4;
 }
-template <int VAR, bool BATCH, bool PULSE>
+template <int VAR, int INTEG, bool BATCH, bool PULSE>
 static hipError_t launch_quad(st_handle* h, const PipeArgs& A) {
     QuadArgs Q{h->P, h->D, A, quad_ppw(h, A.n_list)};
-    hipLaunchKernelGGL((k_spin_quad<VAR, BATCH, PULSE>), dim3(quad_grid(h, A.n_list, Q.ppw)), dim3(256), 0, h->stream, Q);
+    hipLaunchKernelGGL((k_spin_quad<VAR, INTEG, BATCH, PULSE>), dim3(quad_grid(h, A.n_list, Q.ppw)), dim3(256), 0, h->stream, Q);
     return hipGetLastError();
 }
-template <int VAR>
+template <int VAR, int INTEG>
 static hipError_t spin_quad_v(st_handle* h, const PipeArgs& A) {
-    if (h->batch) return h->any_pulse ? launch_quad<VAR, true, true>(h, A) : launch_quad<VAR, true, false>(h, A);
-    return h->any_pulse ? launch_quad<VAR, false, true>(h, A) : launch_quad<VAR, false, false>(h, A);
+    if (h->batch) return h->any_pulse ? launch_quad<VAR, INTEG, true, true>(h, A) : launch_quad<VAR, INTEG, true, false>(h, A);
+    return h->any_pulse ? launch_quad<VAR, INTEG, false, true>(h, A) : launch_quad<VAR, INTEG, false, false>(h, A);
 }
 static hipError_t spin_quad(st_handle* h, const PipeArgs& A) {
-    return h->ext.variant == ST_VARIANT_FAST ? spin_quad_v<VAR_FAST>(h, A) : spin_quad_v<VAR_EXACT>(h, A);
+    const bool fast = h->ext.variant == ST_VARIANT_FAST;
+    if (h->opt.integratorType == INT_RK45)
+        return fast ? spin_quad_v<VAR_FAST, INT_RK45>(h, A) : spin_quad_v<VAR_EXACT, INT_RK45>(h, A);
+    return fast ? spin_quad_v<VAR_FAST, INT_DOP853>(h, A) : spin_quad_v<VAR_EXACT, INT_DOP853>(h, A);
 }
 
 template <bool BATCH, bool PULSE>

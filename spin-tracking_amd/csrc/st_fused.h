@@ -226,7 +226,7 @@ __global__ __launch_bounds__(256) void k_engine(const SimParams P, const DevStat
                 if (VAR == VAR_EXACT) st = dop_trial_exact(P, F, dop, L.S, L.tempH, seg, L.acc, L.rej);
                 else st = dop_trial_fast<PULSE>(P, F, dop, L.S, L.tempH, seg, poly, L.acc, L.rej);
             } else if (INTEG == INT_RK45) {
-                st = rk_trial<VAR>(P, F, rk, L.S, L.tempH, seg, poly, L.acc, L.rej);
+                st = rk_any_trial<VAR, INT_RK45>(P, F, rk, L.S, L.tempH, seg, poly, L.acc, L.rej);
             } else {
                 st = 1;  // unreachable: without an integrator no lane enters PH_INT
             }

@@ -518,17 +518,105 @@ ST_HD __forceinline__ void rk_begin(RkState& R, const Seg& S, double t_end, doub
     R.prev_lr = 0.0;
 }
 
+// Step-size head of an iteration (:268-297): 0, or the reference's error return.
+ST_HD __forceinline__ int rk_bounds(const SimParams& P, double t, double tf, double& lastH, bool& stop, int32_t& nstep,
+                                    double& h) {
+    nstep++;
+    if ((uint32_t)nstep > P.nmax) return -2;
+    const double endDt = tf - t;
+    lastH = h;
+    if (P.fixed) {
+        h = P.h0;
+    } else {
+        if (h > P.hmax) {
+            h = std_min(h, P.hmax);
+        } else if (h < P.hmin) {
+            return -1;
+        }
+    }
+    if (h >= endDt) {
+        h = endDt;
+        stop = true;
+    } else {
+        lastH = h;
+        stop = false;
+    }
+    return 0;
+}
+// Controller factor and accept test of the fast variant from the squared error
+// norm: ratio^0.1 * prev^(-0.4/7) as one exp of a sum of logs, the previous
+// trial's log carried over (no square root, no division): one ctl_log and one
+// ctl_exp instead of two pows.
+ST_HD __forceinline__ double rk_factor_fast(double tol, double e2_in, double& prev_lr, bool& small) {
+    const double e2 = std_max(e2_in, 1.0E-32);
+    const double lr = 0.5 * ctl_log(tol * tol * fast_rcp(e2));
+    const double q = ctl_exp(__builtin_fma(-0.4 / 7.0, prev_lr, (0.7 / 7.0) * lr));
+    prev_lr = lr;
+    small = e2 < 4.0 * tol * tol;
+    return q;
+}
+
+// Fast variant of one iteration: h is folded into the field polynomial, so
+// stages yield K = h*k and every stage input, the step and the error are
+// chains of FMAs from y or from their first product (the quad kernel of
+// st_quad.h forms every value by the same operations in the same order).
+// Weights of zero (the second stage's) are left out.
+ST_HD inline int rk_trial_fast(const SimParams& P, RkState& R, d3& y, double& h, const Seg& S, const Poly& q,
+                               uint32_t& nacc, uint32_t& nrej) {
+    using namespace rk;
+    if (const int b = rk_bounds(P, R.t, R.tf, R.lastH, R.stop, R.nstep, h)) return b;
+    const double t = R.t, hpag = h * q.pag;
+    const Poly hq{d3{h * q.w0.x, h * q.w0.y, h * q.w0.z}, d3{h * q.w1.x, h * q.w1.y, h * q.w1.z},
+                  d3{h * q.w2.x, h * q.w2.y, h * q.w2.z}, q.pag, q.pw, q.paxis, q.pon};
+    auto K = [&](double tt, const d3& yy) -> d3 {
+        return cross3_fma(yy, poly_field<true>(tt - S.t0, hq, hpag, q.pon ? phase_cos(q.pw * tt) : 0.0));
+    };
+    auto axpy = [](double a, const d3& k, const d3& s) -> d3 {
+        return d3{__builtin_fma(a, k.x, s.x), __builtin_fma(a, k.y, s.y), __builtin_fma(a, k.z, s.z)};
+    };
+    const d3 K1 = K(t, R.yy1);
+    d3 yy = axpy(B21, K1, y);
+    const d3 K2 = K(__builtin_fma(A2, h, t), yy);
+    yy = axpy(B31, K1, y); yy = axpy(B32, K2, yy);
+    const d3 K3 = K(__builtin_fma(A3, h, t), yy);
+    yy = axpy(B41, K1, y); yy = axpy(B42, K2, yy); yy = axpy(B43, K3, yy);
+    const d3 K4 = K(__builtin_fma(A4, h, t), yy);
+    yy = axpy(B51, K1, y); yy = axpy(B52, K2, yy); yy = axpy(B53, K3, yy); yy = axpy(B54, K4, yy);
+    const d3 K5 = K(__builtin_fma(A5, h, t), yy);
+    yy = axpy(B61, K1, y); yy = axpy(B62, K2, yy); yy = axpy(B63, K3, yy); yy = axpy(B64, K4, yy); yy = axpy(B65, K5, yy);
+    const d3 K6 = K(__builtin_fma(A6, h, t), yy);
+    R.yy1 = yy;
+    d3 ws = axpy(CH1, K1, y);
+    ws = axpy(CH3, K3, ws); ws = axpy(CH4, K4, ws); ws = axpy(CH5, K5, ws); ws = axpy(CH6, K6, ws);
+    d3 te{CT1 * K1.x, CT1 * K1.y, CT1 * K1.z};
+    te = axpy(CT3, K3, te); te = axpy(CT4, K4, te); te = axpy(CT5, K5, te); te = axpy(CT6, K6, te);
+    bool small;
+    double q_ = rk_factor_fast(P.rtol, __builtin_fma(te.z, te.z, __builtin_fma(te.y, te.y, te.x * te.x)), R.prev_lr, small);
+    q_ = std_min(q_, 4.0);
+    if ((q_ > 0.81 && small) || P.fixed) {
+        nacc++;
+        y = ws;
+        R.t += h;
+        if (R.stop) {
+            h = R.lastH;
+            return 1;
+        }
+    } else {
+        nrej++;
+        if (R.stop) R.stop = false;
+    }
+    if (!P.fixed) h = h * q_;
+    return 0;
+}
+
 // One iteration of the reference's while(1) (:267-335).  Returns 0 to
 // continue, 1 when the call returns 0 (done), -1 / -2 for the reference's
 // error returns.
-template <int VAR>
-ST_HD inline int rk_trial(const SimParams& P, const Phys& Fp, RkState& R, d3& y, double& h, const Seg& S,
-                               const Poly& q, uint32_t& nacc, uint32_t& nrej) {
+ST_HD inline int rk_trial_exact(const SimParams& P, const Phys& Fp, RkState& R, d3& y, double& h, const Seg& S,
+                                uint32_t& nacc, uint32_t& nrej) {
     using namespace rk;
-    auto F = [&](double tt, const d3& yy) -> d3 {
-        if (VAR == VAR_EXACT) return rhs_exact(P, Fp, tt, yy, S);
-        return rhs_fast(P, Fp, tt, yy, S.t0, q);
-    };
+    auto F = [&](double tt, const d3& yy) -> d3 { return rhs_exact(P, Fp, tt, yy, S); };
+    // rk_bounds, written out (through the call: 22 more scalar spills, 2 % slower)
     R.nstep++;
     if ((uint32_t)R.nstep > P.nmax) return -2;
     const double endDt = R.tf - R.t;
@@ -591,25 +679,12 @@ ST_HD inline int rk_trial(const SimParams& P, const Phys& Fp, RkState& R, d3& y,
           h * (CT1 * k1.y + CT2 * k2.y + CT3 * k3.y + CT4 * k4.y + CT5 * k5.y + CT6 * k6.y),
           h * (CT1 * k1.z + CT2 * k2.z + CT3 * k3.z + CT4 * k4.z + CT5 * k5.z + CT6 * k6.z));
     const double tol = P.rtol;
-    double q_;
-    bool small;   // error < 2 tol
-    if constexpr (VAR == VAR_FAST) {
-        // ratio^0.1 * prev^(-0.4/7) as one exp of a sum of logs, the previous
-        // trial's log carried over, from the squared norm (no square root,
-        // no division): one ctl_log and one ctl_exp instead of two pows
-        const double e2 = std_max(te.x * te.x + te.y * te.y + te.z * te.z, 1.0E-32);
-        const double lr = 0.5 * ctl_log(tol * tol * fast_rcp(e2));
-        q_ = ctl_exp((0.7 / 7.0) * lr + (-0.4 / 7.0) * R.prev_lr);
-        R.prev_lr = lr;
-        small = e2 < 4.0 * tol * tol;
-    } else {
-        double error = len3(te);
-        error = std_max(error, 1.0E-16);
-        const double ratio = tol / error;
-        q_ = pow(ratio, 0.7 / 7.0) * pow(R.prev_ratio, -0.4 / 7.0);
-        small = error < 2 * tol;
-        R.prev_ratio = ratio;
-    }
+    double error = len3(te);
+    error = std_max(error, 1.0E-16);
+    const double ratio = tol / error;
+    double q_ = pow(ratio, 0.7 / 7.0) * pow(R.prev_ratio, -0.4 / 7.0);
+    const bool small = error < 2 * tol;
+    R.prev_ratio = ratio;
     q_ = std_min(q_, 4.0);
     if ((q_ > 0.81 && small) || P.fixed) {
         nacc++;
@@ -981,11 +1056,7 @@ ST_HD __forceinline__ int control_v2(const SimParams& P, RkState& R, d3& y, cons
     double q_;
     bool small;   // error < 2 tol
     if constexpr (VAR == VAR_FAST) {
-        const double e2 = std_max(err_in, 1.0E-32);
-        const double lr = 0.5 * ctl_log(tol * tol * fast_rcp(e2));
-        q_ = ctl_exp((0.7 / 7.0) * lr + (-0.4 / 7.0) * R.prev_lr);
-        R.prev_lr = lr;
-        small = e2 < 4.0 * tol * tol;
+        q_ = rk_factor_fast(tol, err_in, R.prev_lr, small);
     } else {
         const double error = std_max(err_in, 1.0E-16);
         const double ratio = tol / error;
@@ -1238,7 +1309,7 @@ template <int VAR, int INTEG>
 ST_HD __forceinline__ int rk_any_trial(const SimParams& P, const Phys& Fp, RkState& R, d3& y, double& h,
                                        const Seg& S, const Poly& q, uint32_t& nacc, uint32_t& nrej) {
     if constexpr (INTEG == INT_RK45)
-        return rk_trial<VAR>(P, Fp, R, y, h, S, q, nacc, nrej);
+        return VAR == VAR_FAST ? rk_trial_fast(P, R, y, h, S, q, nacc, nrej) : rk_trial_exact(P, Fp, R, y, h, S, nacc, nrej);
     else
         return rk2_trial<VAR, INTEG>(P, Fp, R, y, h, S, q, nacc, nrej);
 }

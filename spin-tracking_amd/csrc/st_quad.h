@@ -1,5 +1,5 @@
-// st_quad.h -- DOP853 spin kernels with four lanes per particle, for ensembles
-// that do not fill the chip.
+// st_quad.h -- spin kernels with four lanes per particle, for ensembles that do
+// not fill the chip.
 //
 // What bounds a small ensemble is one lane's chain of trial steps: with one
 // wave per SIMD nothing else can issue, and a lone wave needs 5.5 cycles for
@@ -18,7 +18,10 @@
 //   * the next segment record is loaded while the current one is integrated;
 //   * the pulse's stage cosines are split over the quad.
 // Per trial 1.0 us on neutrons and 1.5 us on He-3 (1,000 particles, fast),
-// 2.4 and 3.2 us exact.
+// 2.4 and 3.2 us exact.  RK45 (half the stages, and a controller that is a
+// chain of 60 dependent operations, a logarithm and an exponential): 0.88 us
+// fast, of one lane 1.15 (and 1.40 before its sums were chains of FMAs);
+// exact 1.60 and 2.92 us.
 // Every value is formed by the one-lane trial's operations in its order, so
 // accept/reject decisions and results are those of the one-lane kernels bit
 // for bit; a quad's four lanes always agree on the control flow.
@@ -469,6 +472,159 @@ __device__ __forceinline__ int q_trial_exact(const SimParams& P, const DopTab& T
     return 0;
 }
 
+// ---------------------------------------------------------------------------
+// RK45 (integratorType 1), one component per lane
+// ---------------------------------------------------------------------------
+#define ST_RK_RESIDENT(X)                                                                                            \
+    X(A2) X(A3) X(A4) X(A6) X(B21) X(B31) X(B32) X(B41) X(B42) X(B43) X(B51) X(B52) X(B53) X(B54) X(B61) X(B62) X(B63) \
+    X(B64) X(B65) X(CH1) X(CH3) X(CH4) X(CH5) X(CH6) X(CT1) X(CT3) X(CT4) X(CT5) X(CT6)
+struct RkTab {
+#define X(n) double n;
+    ST_RK_RESIDENT(X)
+#undef X
+};
+__device__ __forceinline__ void rk_tab_load(RkTab& T) {
+#define X(n) T.n = rk::n; asm volatile("" : "+v"(T.n));
+    ST_RK_RESIDENT(X)
+#undef X
+}
+// RkState with the lane's component of yy1
+struct QRk {
+    double t, tf, lastH, prev_ratio, prev_lr, yy1;
+    int32_t nstep;
+    bool stop;
+};
+__device__ __forceinline__ void q_rk_begin(QRk& R, double t0, double t_end, double h) {
+    R.t = t0;
+    R.tf = t_end;
+    R.stop = false;
+    R.nstep = 0;
+    R.lastH = h;
+    R.yy1 = 0.0;
+    R.prev_ratio = 1.0;
+    R.prev_lr = 0.0;
+}
+// end of an iteration: accept or reject, next step size
+__device__ __forceinline__ int q_rk_end(const SimParams& P, QRk& R, double& y, double ws, double& h, double q_, bool small,
+                                        uint32_t& nacc, uint32_t& nrej) {
+    q_ = std_min(q_, 4.0);
+    if ((q_ > 0.81 && small) || P.fixed) {
+        nacc++;
+        y = ws;
+        R.t += h;
+        if (R.stop) {
+            h = R.lastH;
+            return 1;
+        }
+    } else {
+        nrej++;
+        if (R.stop) R.stop = false;
+    }
+    if (!P.fixed) h = h * q_;
+    return 0;
+}
+// rk_trial_fast (st_integrators.h) on a quad; the pulse's cosines at the six
+// stage times are split over the quad.
+template <bool PULSE>
+__device__ __forceinline__ int q_trial_rk_fast(const SimParams& P, const RkTab& T, QRk& R, double& y, double& h,
+                                               double t0, const QPoly& q, const QPulse& pl, uint32_t& nacc,
+                                               uint32_t& nrej) {
+    if (const int b = rk_bounds(P, R.t, R.tf, R.lastH, R.stop, R.nstep, h)) return b;
+    const double t = R.t;
+    const QPoly hq{h * q.a0, h * q.a1, h * q.a2, h * q.b0, h * q.b1, h * q.b2};
+    const double t2 = __builtin_fma(T.A2, h, t), t3 = __builtin_fma(T.A3, h, t), t4 = __builtin_fma(T.A4, h, t),
+                 t5 = __builtin_fma(rk::A5, h, t), t6 = __builtin_fma(T.A6, h, t);
+    double hp0 = 0.0, hp1 = 0.0, ha = 0.0, hb = 0.0;
+    if constexpr (PULSE) {
+        if (pl.on) {
+            const uint32_t l = __lane_id() & 3u;
+            hp0 = phase_cos(pl.pw * (l == 0 ? t : l == 1 ? t2 : l == 2 ? t3 : t4));
+            hp1 = phase_cos(pl.pw * (l == 0 ? t5 : t6));
+            ha = h * pl.ma;
+            hb = h * pl.mb;
+        }
+    }
+    auto K = [&](double tt, double yy, double cosv) -> double {
+        double wa, wb;
+        q_field(tt - t0, hq, wa, wb);
+        if constexpr (PULSE) {
+            wa = __builtin_fma(ha, cosv, wa);
+            wb = __builtin_fma(hb, cosv, wb);
+        }
+        return q_cross(yy, wa, wb);
+    };
+#define QF(S, A, K) S = __builtin_fma(T.A, K, S)
+    const double K1 = K(t, R.yy1, q_all<0>(hp0));
+    double yy = y;
+    QF(yy, B21, K1);
+    const double K2 = K(t2, yy, q_all<1>(hp0));
+    yy = y;
+    QF(yy, B31, K1); QF(yy, B32, K2);
+    const double K3 = K(t3, yy, q_all<2>(hp0));
+    yy = y;
+    QF(yy, B41, K1); QF(yy, B42, K2); QF(yy, B43, K3);
+    const double K4 = K(t4, yy, q_all<3>(hp0));
+    yy = y;
+    QF(yy, B51, K1); QF(yy, B52, K2); QF(yy, B53, K3); QF(yy, B54, K4);
+    const double K5 = K(t5, yy, q_all<0>(hp1));
+    yy = y;
+    QF(yy, B61, K1); QF(yy, B62, K2); QF(yy, B63, K3); QF(yy, B64, K4); QF(yy, B65, K5);
+    const double K6 = K(t6, yy, q_all<1>(hp1));
+    R.yy1 = yy;
+    double ws = y;
+    QF(ws, CH1, K1); QF(ws, CH3, K3); QF(ws, CH4, K4); QF(ws, CH5, K5); QF(ws, CH6, K6);
+    double te = T.CT1 * K1;
+    QF(te, CT3, K3); QF(te, CT4, K4); QF(te, CT5, K5); QF(te, CT6, K6);
+#undef QF
+    const d3 e = q_vec(te);
+    bool small;
+    const double f = rk_factor_fast(P.rtol, __builtin_fma(e.z, e.z, __builtin_fma(e.y, e.y, e.x * e.x)), R.prev_lr, small);
+    return q_rk_end(P, R, y, ws, h, f, small, nacc, nrej);
+}
+// rk_trial_exact on a quad
+template <bool PULSE>
+__device__ __forceinline__ int q_trial_rk_exact(const SimParams& P, const RkTab& T, QRk& R, double& y, double& h,
+                                                double t0, const QExact& X, uint32_t& nacc, uint32_t& nrej) {
+    if (const int b = rk_bounds(P, R.t, R.tf, R.lastH, R.stop, R.nstep, h)) return b;
+    const bool gravity = P.gravity;
+    const double t = R.t, t2 = t + T.A2 * h, t3 = t + T.A3 * h, t4 = t + T.A4 * h, t5 = t + rk::A5 * h, t6 = t + T.A6 * h;
+    double hp0 = 0.0, hp1 = 0.0;
+    if constexpr (PULSE) {
+        if (X.axis >= 0) {
+            const uint32_t l = __lane_id() & 3u;
+            hp0 = q_pulse_exact(X, l == 0 ? t : l == 1 ? t2 : l == 2 ? t3 : t4);
+            hp1 = q_pulse_exact(X, l == 0 ? t5 : t6);
+        }
+    }
+#define QX(TT, LANE, HP) q_rhs_exact(X, gravity, (TT), t0, yy, PULSE ? q_all<LANE>(HP) : 0.0)
+    double yy = R.yy1;
+    const double k1 = QX(t, 0, hp0);
+    yy = y + (h * T.B21) * k1;
+    const double k2 = QX(t2, 1, hp0);
+    yy = y + (h * T.B31) * k1 + (h * T.B32) * k2;
+    const double k3 = QX(t3, 2, hp0);
+    yy = y + (h * T.B41) * k1 + (h * T.B42) * k2 + (h * T.B43) * k3;
+    const double k4 = QX(t4, 3, hp0);
+    yy = y + (h * T.B51) * k1 + (h * T.B52) * k2 + (h * T.B53) * k3 + (h * T.B54) * k4;
+    const double k5 = QX(t5, 0, hp1);
+    yy = y + (h * T.B61) * k1 + (h * T.B62) * k2 + (h * T.B63) * k3 + (h * T.B64) * k4 + (h * T.B65) * k5;
+    const double k6 = QX(t6, 1, hp1);
+#undef QX
+    R.yy1 = yy;
+    const double ws = y + h * (k1 * T.CH1 + k2 * rk::CH2 + k3 * T.CH3 + k4 * T.CH4 + k5 * T.CH5 + k6 * T.CH6);
+    const double te = h * (T.CT1 * k1 + rk::CT2 * k2 + T.CT3 * k3 + T.CT4 * k4 + T.CT5 * k5 + T.CT6 * k6);
+    const double tol = P.rtol;
+    double error = len3(q_vec(te));
+    error = std_max(error, 1.0E-16);
+    const double ratio = tol / error;
+    // both powers at once: lanes 0 and 1 of the quad take the first, 2 and 3 the other
+    const bool low = (__lane_id() & 2u) == 0u;
+    const double p = pow(low ? ratio : R.prev_ratio, low ? 0.7 / 7.0 : -0.4 / 7.0);
+    const double f = q_all<0>(p) * q_all<2>(p);
+    R.prev_ratio = ratio;
+    return q_rk_end(P, R, y, ws, h, f, error < 2 * tol, nacc, nrej);
+}
+
 // The products make_poly reads, for the lane's components a = c+1 and b = c+2.
 __device__ __forceinline__ void q_pulse_load(QPulse& pl, const Phys& F, uint32_t c, double sign = 1.0) {
     const int32_t a = c == 2 ? 0 : (int32_t)c + 1, b = c == 0 ? 2 : (int32_t)c - 1;
@@ -507,7 +663,7 @@ __device__ __forceinline__ void q_make_poly(QPoly& q, const Phys& F, const d3& p
 __device__ __forceinline__ void quad_block(const RunArgs& R, uint32_t pid, int32_t k, uint32_t c, double y) {
     if (R.blocks) reinterpret_cast<double*>(R.blocks + (uint64_t)k * R.block_bytes + 56 * (uint64_t)R.n)[3 * (uint64_t)pid + c] = y;
 }
-template <int VAR, bool BATCH, bool PULSE>
+template <int VAR, int INTEG, bool BATCH, bool PULSE>
 __device__ __forceinline__ void quad_spin() {
     auto args = []() -> const QuadArgs& { return kernel_args<QuadArgs>(); };
     const uint32_t lane = __lane_id();
@@ -515,8 +671,11 @@ __device__ __forceinline__ void quad_spin() {
     const uint32_t ppw = args().ppw;
     const bool first = (lane >> 2) < ppw;
     const bool lead = first && (lane & 3u) == 0u, owner = first && (lane & 3u) != 3u;
+    constexpr bool DOP = INTEG == INT_DOP853;
     DopTab T;
-    dop_tab_load<false>(T);
+    RkTab TR;
+    if constexpr (DOP) dop_tab_load<false>(T);
+    else rk_tab_load(TR);
     // a plain handle's physics in LDS, one copy per workgroup
     __shared__ Phys shared_phys;
     if constexpr (!BATCH) {
@@ -534,7 +693,9 @@ __device__ __forceinline__ void quad_spin() {
     SpinLane L;      // (S unused: the lane's component is y)
     double y = 0.0;
     QDop dop;
+    QRk rk;
     QPoly q;
+    auto seg_end = [&]() { return DOP ? dop.xf : rk.tf; };
     double seg_t0 = 0.0;
     SegRec nxt;      // record L.j, loaded while record L.j - 1 is integrated
     uint32_t cur_flags = 0;
@@ -575,30 +736,37 @@ __device__ __forceinline__ void quad_spin() {
                 if (L.j + 1 < L.nrec) nxt = load_rec(rec_at_seq(A, L.pid, L.j + 1, L.page));
                 cur_flags = (uint32_t)rec.flags;
                 if (rec.flags & R_FIRST) L.tempH = L.h;
-                if ((rec.flags & R_INTEGRATE) && !L.stopped) {
+                if (rec.flags & R_INTEGRATE) {
                     seg_t0 = L.t_spin;
-                    dop.x = seg_t0;
-                    dop.xf = rec.t;
-                    dop.facold = 1.0E-4;
-                    dop.last = 0;
-                    dop.reject = 0;
-                    dop.nstep = 0;
                     if constexpr (VAR == VAR_EXACT) {
-                        dop.posneg = sign_d(1.0, rec.t - seg_t0);
                         X.p0 = q_pick(d3{rec.px, rec.py, rec.pz}, c);
                         X.v0 = q_pick(d3{rec.vx, rec.vy, rec.vz}, c);
-                        dop.k1 = q_rhs_exact(X, args().P.gravity, seg_t0, seg_t0, y,
-                                             PULSE && X.axis >= 0 ? q_pulse_exact(X, seg_t0) : 0.0);
                     } else {
                         q_make_poly(q, BATCH ? A.phys[L.cfg] : shared_phys, d3{rec.px, rec.py, rec.pz},
                                     d3{rec.vx, rec.vy, rec.vz}, c);
-                        double wa = q.a0, wb = q.b0;
-                        if constexpr (PULSE) {
-                            const double cosv = pl.on ? phase_cos(pl.pw * seg_t0) : 0.0;
-                            wa = __builtin_fma(pl.ma, cosv, wa);
-                            wb = __builtin_fma(pl.mb, cosv, wb);
+                    }
+                    if constexpr (DOP) {
+                        dop.x = seg_t0;
+                        dop.xf = rec.t;
+                        dop.facold = 1.0E-4;
+                        dop.last = 0;
+                        dop.reject = 0;
+                        dop.nstep = 0;
+                        if constexpr (VAR == VAR_EXACT) {
+                            dop.posneg = sign_d(1.0, rec.t - seg_t0);
+                            dop.k1 = q_rhs_exact(X, args().P.gravity, seg_t0, seg_t0, y,
+                                                 PULSE && X.axis >= 0 ? q_pulse_exact(X, seg_t0) : 0.0);
+                        } else {
+                            double wa = q.a0, wb = q.b0;
+                            if constexpr (PULSE) {
+                                const double cosv = pl.on ? phase_cos(pl.pw * seg_t0) : 0.0;
+                                wa = __builtin_fma(pl.ma, cosv, wa);
+                                wb = __builtin_fma(pl.mb, cosv, wb);
+                            }
+                            dop.k1 = q_cross(y, wa, wb);
                         }
-                        dop.k1 = q_cross(y, wa, wb);
+                    } else {
+                        q_rk_begin(rk, seg_t0, rec.t, L.tempH);
                     }
                     L.seg++;
                     if (R.trace && L.pid == R.trace_pid) {
@@ -621,19 +789,22 @@ __device__ __forceinline__ void quad_spin() {
         }
         if (phase == S_INT) {
             int st;
-            if constexpr (VAR == VAR_EXACT) st = q_trial_exact<PULSE>(args().P, T, dop, y, L.tempH, seg_t0, X, L.acc, L.rej);
-            else st = q_trial_fast<false, PULSE>(args().P, T, dop, y, L.tempH, seg_t0, q, pl, L.acc, L.rej, nullptr);
+            const SimParams& P = args().P;
+            if constexpr (DOP && VAR == VAR_EXACT) st = q_trial_exact<PULSE>(P, T, dop, y, L.tempH, seg_t0, X, L.acc, L.rej);
+            else if constexpr (DOP) st = q_trial_fast<false, PULSE>(P, T, dop, y, L.tempH, seg_t0, q, pl, L.acc, L.rej, nullptr);
+            else if constexpr (VAR == VAR_EXACT) st = q_trial_rk_exact<PULSE>(P, TR, rk, y, L.tempH, seg_t0, X, L.acc, L.rej);
+            else st = q_trial_rk_fast<PULSE>(P, TR, rk, y, L.tempH, seg_t0, q, pl, L.acc, L.rej);
             if (st != 0) {
                 const PipeArgs& A = args().A;
                 const RunArgs& R = A.R;
                 if (R.trace && L.pid == R.trace_pid) {
                     const d3 S = q_vec(y);
                     if (lead)
-                        ST_TRACE(R, 2, L.t_spin, dop.xf, d3{0, 0, 0}, d3{0, 0, 0}, S, L.tempH, L.acc, L.rej,
+                        ST_TRACE(R, 2, L.t_spin, seg_end(), d3{0, 0, 0}, d3{0, 0, 0}, S, L.tempH, L.acc, L.rej,
                                  (char)(cur_flags >> 8), (char)(cur_flags >> 16), st, 0, 0);
                 }
                 if (args().P.keep) L.h = L.tempH;
-                L.t_spin = dop.xf;
+                L.t_spin = seg_end();
                 if (st < 0) {
                     if (lead) {
                         const uint32_t slot = atomicAdd(A.fail_count, 1u);
@@ -643,10 +814,9 @@ __device__ __forceinline__ void quad_spin() {
                             A.fail_list[3 * slot + 2] = (uint32_t)st;
                         }
                     }
-                    L.stopped = true;
                     L.nrec = 0;   // (spin_body: the records after a failure)
                 }
-                if (L.stopped || (cur_flags & R_STOP)) y = __builtin_nan("");
+                if (st < 0 || (cur_flags & R_STOP)) y = __builtin_nan("");
                 if ((cur_flags & R_IEND) && st > 0) {
                     if (owner) quad_block(R, L.pid, L.k, c, y);
                     L.k++;
@@ -660,9 +830,9 @@ __device__ __forceinline__ void quad_spin() {
     flush_counters(args().A.R.work, sum);
 }
 
-template <int VAR, bool BATCH, bool PULSE>
+template <int VAR, int INTEG, bool BATCH, bool PULSE>
 __global__ __launch_bounds__(256, 2) void k_spin_quad(const QuadArgs) {
-    quad_spin<VAR, BATCH, PULSE>();
+    quad_spin<VAR, INTEG, BATCH, PULSE>();
 }
 
 // ---------------------------------------------------------------------------

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 FILLER = 33000      # with it, the batch is past the quad kernels' 32,768
 
 
-def options(kind, n, seed):
+def options(kind, n, seed, integ=0):
     if kind == "dressing":
         o = configs.dressing(n=n, species="he3", tf=0.008, ioutInt=0.004, seed=seed)
     elif kind == "he3":
@@ -21,6 +21,8 @@ def options(kind, n, seed):
     else:
         o = configs.neutron_cell(n=n, tf=0.06, ioutInt=0.03, seed=seed)
         st.set_fields(o, yi=(0.0, 1.0, 0.0))
+    if integ == 1:      # RK45: far more steps per second at a loose tolerance already
+        st.set_fields(o, integratorType=1, rtol=1e-9, tf=o.tf / 20.0, ioutInt=o.ioutInt / 20.0)
     return o
 
 
@@ -39,10 +41,11 @@ def run(p, times):
 @pytest.mark.parametrize("kind,variant", [("he3", st.VARIANT_FAST), ("dressing", st.VARIANT_FAST),
                                           ("neutron", st.VARIANT_FAST), ("he3", st.VARIANT_EXACT),
                                           ("dressing", st.VARIANT_EXACT), ("neutron", st.VARIANT_EXACT)])
-def test_quad_equals_one_lane(kind, variant, n):
-    print(f"[quad] {kind} variant={variant} n={n}", flush=True)
+@pytest.mark.parametrize("integ", [0, 1])
+def test_quad_equals_one_lane(kind, variant, n, integ):
+    print(f"[quad] {kind} variant={variant} n={n} integratorType={integ}", flush=True)
     axis = 1 if kind == "dressing" else 2
-    small, filler = options(kind, n, 11), options(kind, FILLER, 5000)
+    small, filler = options(kind, n, 11, integ), options(kind, FILLER, 5000, integ)
     times = list(st.output_times(small))
     with st.Particle(small, variant=variant, pulse_axis=axis) as p:
         state, cnt, raw, bb = run(p, times)
