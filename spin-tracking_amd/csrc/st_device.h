@@ -608,6 +608,25 @@ constexpr double TAYLOR_HOST[4][14] = {{ST_TAYLOR_COS}, {ST_TAYLOR_SINC}, {ST_TA
 #undef ST_TAYLOR_ATANH
 #undef ST_TAYLOR_EXP
 
+// Puts the instructions after the one that forms v on 8-byte boundaries (one
+// s_nop where they are not), and lets none of those that use v move ahead.
+// A lone wave issues one instruction in 4.3 cycles, whether or not it waits
+// for the result before it; 8-byte instructions one after another that lie
+// across the boundaries take 5.3, and code without FMA contraction is little
+// else (products and sums of doubles have no 4-byte form).  In the exact
+// trials, after each stage: k_spin_quad on 64 neutrons x 0.5 s took 3.27 or
+// 3.62 ms, as the trial happened to lie, and takes 3.30.  The one-lane DOP853
+// kernel, whose stages the scheduler no longer mixes, needs 225 registers in
+// place of 344, two waves per SIMD (1,048,576 neutrons x 0.2 s: 50.1 and
+// 35.5 ms; 131,072: 6.26 and 4.81 ms).  In the rotations of the MagnusCFET
+// and quaternion trials it gains nothing (their library calls are aligned
+// by themselves; 2 % slower) and is not used.
+#if defined(__HIP_DEVICE_COMPILE__)
+#define ST_CODE_ALIGN(v) asm(".p2align 3" : "+v"(v))
+#else
+#define ST_CODE_ALIGN(v) ((void)(v))
+#endif
+
 // sum_{k<N} TAYLOR[row][k] x2^k by Horner, one FMA per term
 template <int ROW, int N>
 ST_HD __forceinline__ double taylor_sum(double x2) {

@@ -142,48 +142,59 @@ ST_HD inline int dop_trial_exact(const SimParams& P, const Phys& F, DopState& D,
         ST_V3(yy, y.x + k1.x * ha, y.y + k1.y * ha, y.z + k1.z * ha);
     }
     k2 = rhs_exact(P, F, x + c2 * h, yy, S);
+    ST_CODE_ALIGN(k2.x);
     ST_V3(yy, y.x + h * (a31 * k1.x + a32 * k2.x), y.y + h * (a31 * k1.y + a32 * k2.y),
           y.z + h * (a31 * k1.z + a32 * k2.z));
     k3 = rhs_exact(P, F, x + c3 * h, yy, S);
+    ST_CODE_ALIGN(k3.x);
     ST_V3(yy, y.x + h * (a41 * k1.x + a43 * k3.x), y.y + h * (a41 * k1.y + a43 * k3.y),
           y.z + h * (a41 * k1.z + a43 * k3.z));
     k4 = rhs_exact(P, F, x + c4 * h, yy, S);
+    ST_CODE_ALIGN(k4.x);
     ST_V3(yy, y.x + h * (a51 * k1.x + a53 * k3.x + a54 * k4.x),
           y.y + h * (a51 * k1.y + a53 * k3.y + a54 * k4.y),
           y.z + h * (a51 * k1.z + a53 * k3.z + a54 * k4.z));
     k5 = rhs_exact(P, F, x + c5 * h, yy, S);
+    ST_CODE_ALIGN(k5.x);
     ST_V3(yy, y.x + h * (a61 * k1.x + a64 * k4.x + a65 * k5.x),
           y.y + h * (a61 * k1.y + a64 * k4.y + a65 * k5.y),
           y.z + h * (a61 * k1.z + a64 * k4.z + a65 * k5.z));
     k6 = rhs_exact(P, F, x + c6 * h, yy, S);
+    ST_CODE_ALIGN(k6.x);
     ST_V3(yy, y.x + h * (a71 * k1.x + a74 * k4.x + a75 * k5.x + a76 * k6.x),
           y.y + h * (a71 * k1.y + a74 * k4.y + a75 * k5.y + a76 * k6.y),
           y.z + h * (a71 * k1.z + a74 * k4.z + a75 * k5.z + a76 * k6.z));
     k7 = rhs_exact(P, F, x + c7 * h, yy, S);
+    ST_CODE_ALIGN(k7.x);
     ST_V3(yy, y.x + h * (a81 * k1.x + a84 * k4.x + a85 * k5.x + a86 * k6.x + a87 * k7.x),
           y.y + h * (a81 * k1.y + a84 * k4.y + a85 * k5.y + a86 * k6.y + a87 * k7.y),
           y.z + h * (a81 * k1.z + a84 * k4.z + a85 * k5.z + a86 * k6.z + a87 * k7.z));
     k8 = rhs_exact(P, F, x + c8 * h, yy, S);
+    ST_CODE_ALIGN(k8.x);
     ST_V3(yy, y.x + h * (a91 * k1.x + a94 * k4.x + a95 * k5.x + a96 * k6.x + a97 * k7.x + a98 * k8.x),
           y.y + h * (a91 * k1.y + a94 * k4.y + a95 * k5.y + a96 * k6.y + a97 * k7.y + a98 * k8.y),
           y.z + h * (a91 * k1.z + a94 * k4.z + a95 * k5.z + a96 * k6.z + a97 * k7.z + a98 * k8.z));
     k9 = rhs_exact(P, F, x + c9 * h, yy, S);
+    ST_CODE_ALIGN(k9.x);
     ST_V3(yy,
           y.x + h * (a101 * k1.x + a104 * k4.x + a105 * k5.x + a106 * k6.x + a107 * k7.x + a108 * k8.x + a109 * k9.x),
           y.y + h * (a101 * k1.y + a104 * k4.y + a105 * k5.y + a106 * k6.y + a107 * k7.y + a108 * k8.y + a109 * k9.y),
           y.z + h * (a101 * k1.z + a104 * k4.z + a105 * k5.z + a106 * k6.z + a107 * k7.z + a108 * k8.z + a109 * k9.z));
     k10 = rhs_exact(P, F, x + c10 * h, yy, S);
+    ST_CODE_ALIGN(k10.x);
     ST_V3(yy,
           y.x + h * (a111 * k1.x + a114 * k4.x + a115 * k5.x + a116 * k6.x + a117 * k7.x + a118 * k8.x + a119 * k9.x + a1110 * k10.x),
           y.y + h * (a111 * k1.y + a114 * k4.y + a115 * k5.y + a116 * k6.y + a117 * k7.y + a118 * k8.y + a119 * k9.y + a1110 * k10.y),
           y.z + h * (a111 * k1.z + a114 * k4.z + a115 * k5.z + a116 * k6.z + a117 * k7.z + a118 * k8.z + a119 * k9.z + a1110 * k10.z));
     k2 = rhs_exact(P, F, x + c11 * h, yy, S);
+    ST_CODE_ALIGN(k2.x);
     const double xph = x + h;
     ST_V3(yy,
           y.x + h * (a121 * k1.x + a124 * k4.x + a125 * k5.x + a126 * k6.x + a127 * k7.x + a128 * k8.x + a129 * k9.x + a1210 * k10.x + a1211 * k2.x),
           y.y + h * (a121 * k1.y + a124 * k4.y + a125 * k5.y + a126 * k6.y + a127 * k7.y + a128 * k8.y + a129 * k9.y + a1210 * k10.y + a1211 * k2.y),
           y.z + h * (a121 * k1.z + a124 * k4.z + a125 * k5.z + a126 * k6.z + a127 * k7.z + a128 * k8.z + a129 * k9.z + a1210 * k10.z + a1211 * k2.z));
     k3 = rhs_exact(P, F, xph, yy, S);
+    ST_CODE_ALIGN(k3.x);
     ST_V3(k4, b1 * k1.x + b6 * k6.x + b7 * k7.x + b8 * k8.x + b9 * k9.x + b10 * k10.x + b11 * k2.x + b12 * k3.x,
           b1 * k1.y + b6 * k6.y + b7 * k7.y + b8 * k8.y + b9 * k9.y + b10 * k10.y + b11 * k2.y + b12 * k3.y,
           b1 * k1.z + b6 * k6.z + b7 * k7.z + b8 * k8.z + b9 * k9.z + b10 * k10.z + b11 * k2.z + b12 * k3.z);
@@ -639,37 +650,43 @@ ST_HD inline int rk_trial_exact(const SimParams& P, const Phys& Fp, RkState& R, 
     }
     const double t = R.t;
     d3 yy1 = R.yy1;
-    const d3 k1 = F(t, yy1);
+    d3 k1 = F(t, yy1);
+    ST_CODE_ALIGN(k1.x);
     {
         const double c = h * B21;
         ST_V3(yy1, y.x + c * k1.x, y.y + c * k1.y, y.z + c * k1.z);
     }
-    const d3 k2 = F(t + A2 * h, yy1);
+    d3 k2 = F(t + A2 * h, yy1);
+    ST_CODE_ALIGN(k2.x);
     {
         const double c1 = h * B31, c2_ = h * B32;
         ST_V3(yy1, y.x + c1 * k1.x + c2_ * k2.x, y.y + c1 * k1.y + c2_ * k2.y, y.z + c1 * k1.z + c2_ * k2.z);
     }
-    const d3 k3 = F(t + A3 * h, yy1);
+    d3 k3 = F(t + A3 * h, yy1);
+    ST_CODE_ALIGN(k3.x);
     {
         const double c1 = h * B41, c2_ = h * B42, c3_ = h * B43;
         ST_V3(yy1, y.x + c1 * k1.x + c2_ * k2.x + c3_ * k3.x, y.y + c1 * k1.y + c2_ * k2.y + c3_ * k3.y,
               y.z + c1 * k1.z + c2_ * k2.z + c3_ * k3.z);
     }
-    const d3 k4 = F(t + A4 * h, yy1);
+    d3 k4 = F(t + A4 * h, yy1);
+    ST_CODE_ALIGN(k4.x);
     {
         const double c1 = h * B51, c2_ = h * B52, c3_ = h * B53, c4_ = h * B54;
         ST_V3(yy1, y.x + c1 * k1.x + c2_ * k2.x + c3_ * k3.x + c4_ * k4.x,
               y.y + c1 * k1.y + c2_ * k2.y + c3_ * k3.y + c4_ * k4.y,
               y.z + c1 * k1.z + c2_ * k2.z + c3_ * k3.z + c4_ * k4.z);
     }
-    const d3 k5 = F(t + A5 * h, yy1);
+    d3 k5 = F(t + A5 * h, yy1);
+    ST_CODE_ALIGN(k5.x);
     {
         const double c1 = h * B61, c2_ = h * B62, c3_ = h * B63, c4_ = h * B64, c5_ = h * B65;
         ST_V3(yy1, y.x + c1 * k1.x + c2_ * k2.x + c3_ * k3.x + c4_ * k4.x + c5_ * k5.x,
               y.y + c1 * k1.y + c2_ * k2.y + c3_ * k3.y + c4_ * k4.y + c5_ * k5.y,
               y.z + c1 * k1.z + c2_ * k2.z + c3_ * k3.z + c4_ * k4.z + c5_ * k5.z);
     }
-    const d3 k6 = F(t + A6 * h, yy1);
+    d3 k6 = F(t + A6 * h, yy1);
+    ST_CODE_ALIGN(k6.x);
     R.yy1 = yy1;
     d3 ws, te;
     ST_V3(ws, y.x + h * (k1.x * CH1 + k2.x * CH2 + k3.x * CH3 + k4.x * CH4 + k5.x * CH5 + k6.x * CH6),
@@ -1161,37 +1178,43 @@ ST_HD inline int rk2_trial(const SimParams& P, const Phys& Fp, RkState& R, d3& y
         using namespace rkf;
         auto F = [&](double tt, const d3& yy) -> d3 { return cross3(yy, W(tt)); };
         d3 yy1 = R.yy1;
-        const d3 k1 = F(t, yy1);
+        d3 k1 = F(t, yy1);
+        if constexpr (VAR == VAR_EXACT) ST_CODE_ALIGN(k1.x);
         {
             const double c = h * B21;
             ST_V3(yy1, y.x + c * k1.x, y.y + c * k1.y, y.z + c * k1.z);
         }
-        const d3 k2 = F(t + A2 * h, yy1);
+        d3 k2 = F(t + A2 * h, yy1);
+        if constexpr (VAR == VAR_EXACT) ST_CODE_ALIGN(k2.x);
         {
             const double c1 = h * B31, c2_ = h * B32;
             ST_V3(yy1, y.x + c1 * k1.x + c2_ * k2.x, y.y + c1 * k1.y + c2_ * k2.y, y.z + c1 * k1.z + c2_ * k2.z);
         }
-        const d3 k3 = F(t + A3 * h, yy1);
+        d3 k3 = F(t + A3 * h, yy1);
+        if constexpr (VAR == VAR_EXACT) ST_CODE_ALIGN(k3.x);
         {
             const double c1 = h * B41, c2_ = h * B42, c3_ = h * B43;
             ST_V3(yy1, y.x + c1 * k1.x + c2_ * k2.x + c3_ * k3.x, y.y + c1 * k1.y + c2_ * k2.y + c3_ * k3.y,
                   y.z + c1 * k1.z + c2_ * k2.z + c3_ * k3.z);
         }
-        const d3 k4 = F(t + A4 * h, yy1);
+        d3 k4 = F(t + A4 * h, yy1);
+        if constexpr (VAR == VAR_EXACT) ST_CODE_ALIGN(k4.x);
         {
             const double c1 = h * B51, c2_ = h * B52, c3_ = h * B53, c4_ = h * B54;
             ST_V3(yy1, y.x + c1 * k1.x + c2_ * k2.x + c3_ * k3.x + c4_ * k4.x,
                   y.y + c1 * k1.y + c2_ * k2.y + c3_ * k3.y + c4_ * k4.y,
                   y.z + c1 * k1.z + c2_ * k2.z + c3_ * k3.z + c4_ * k4.z);
         }
-        const d3 k5 = F(t + A5 * h, yy1);
+        d3 k5 = F(t + A5 * h, yy1);
+        if constexpr (VAR == VAR_EXACT) ST_CODE_ALIGN(k5.x);
         {
             const double c1 = h * B61, c2_ = h * B62, c3_ = h * B63, c4_ = h * B64, c5_ = h * B65;
             ST_V3(yy1, y.x + c1 * k1.x + c2_ * k2.x + c3_ * k3.x + c4_ * k4.x + c5_ * k5.x,
                   y.y + c1 * k1.y + c2_ * k2.y + c3_ * k3.y + c4_ * k4.y + c5_ * k5.y,
                   y.z + c1 * k1.z + c2_ * k2.z + c3_ * k3.z + c4_ * k4.z + c5_ * k5.z);
         }
-        const d3 k6 = F(t + A6 * h, yy1);
+        d3 k6 = F(t + A6 * h, yy1);
+        if constexpr (VAR == VAR_EXACT) ST_CODE_ALIGN(k6.x);
         R.yy1 = yy1;
         d3 ws, te;
         ST_V3(ws, y.x + h * (k1.x * W1 + k2.x * W2 + k3.x * W3 + k4.x * W4 + k5.x * W5 + k6.x * W6),

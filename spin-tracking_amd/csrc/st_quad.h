@@ -416,27 +416,38 @@ __device__ __forceinline__ int q_trial_exact(const SimParams& P, const DopTab& T
 #define QX(TT, LANE, HP) q_rhs_exact(X, gravity, (TT), t0, yy, PULSE ? q_all<LANE>(HP) : 0.0)
     const double k1 = D.k1;
     double yy = y + k1 * (h * T.a21);
-    const double k2 = QX(x + T.c2 * h, 0, hp0);
+    double k2 = QX(x + T.c2 * h, 0, hp0);
+    ST_CODE_ALIGN(k2);
     yy = y + h * (T.a31 * k1 + T.a32 * k2);
-    const double k3 = QX(x + T.c3 * h, 1, hp0);
+    double k3 = QX(x + T.c3 * h, 1, hp0);
+    ST_CODE_ALIGN(k3);
     yy = y + h * (T.a41 * k1 + T.a43 * k3);
-    const double k4 = QX(x + T.c4 * h, 2, hp0);
+    double k4 = QX(x + T.c4 * h, 2, hp0);
+    ST_CODE_ALIGN(k4);
     yy = y + h * (T.a51 * k1 + T.a53 * k3 + T.a54 * k4);
-    const double k5 = QX(x + T.c5 * h, 3, hp0);
+    double k5 = QX(x + T.c5 * h, 3, hp0);
+    ST_CODE_ALIGN(k5);
     yy = y + h * (T.a61 * k1 + T.a64 * k4 + T.a65 * k5);
-    const double k6 = QX(x + T.c6 * h, 0, hp1);
+    double k6 = QX(x + T.c6 * h, 0, hp1);
+    ST_CODE_ALIGN(k6);
     yy = y + h * (T.a71 * k1 + T.a74 * k4 + T.a75 * k5 + T.a76 * k6);
-    const double k7 = QX(x + T.c7 * h, 1, hp1);
+    double k7 = QX(x + T.c7 * h, 1, hp1);
+    ST_CODE_ALIGN(k7);
     yy = y + h * (T.a81 * k1 + T.a84 * k4 + T.a85 * k5 + T.a86 * k6 + T.a87 * k7);
-    const double k8 = QX(x + T.c8 * h, 2, hp1);
+    double k8 = QX(x + T.c8 * h, 2, hp1);
+    ST_CODE_ALIGN(k8);
     yy = y + h * (T.a91 * k1 + T.a94 * k4 + T.a95 * k5 + T.a96 * k6 + T.a97 * k7 + T.a98 * k8);
-    const double k9 = QX(x + T.c9 * h, 3, hp1);
+    double k9 = QX(x + T.c9 * h, 3, hp1);
+    ST_CODE_ALIGN(k9);
     yy = y + h * (T.a101 * k1 + T.a104 * k4 + T.a105 * k5 + T.a106 * k6 + T.a107 * k7 + T.a108 * k8 + T.a109 * k9);
-    const double k10 = QX(x + T.c10 * h, 0, hp2);
+    double k10 = QX(x + T.c10 * h, 0, hp2);
+    ST_CODE_ALIGN(k10);
     yy = y + h * (T.a111 * k1 + T.a114 * k4 + T.a115 * k5 + T.a116 * k6 + T.a117 * k7 + T.a118 * k8 + T.a119 * k9 + T.a1110 * k10);
-    const double k11 = QX(x + T.c11 * h, 1, hp2);
+    double k11 = QX(x + T.c11 * h, 1, hp2);
+    ST_CODE_ALIGN(k11);
     yy = y + h * (T.a121 * k1 + T.a124 * k4 + T.a125 * k5 + T.a126 * k6 + T.a127 * k7 + T.a128 * k8 + T.a129 * k9 + T.a1210 * k10 + T.a1211 * k11);
-    const double k12 = QX(xph, 2, hp2);
+    double k12 = QX(xph, 2, hp2);
+    ST_CODE_ALIGN(k12);
 #undef QX
     const double b = T.b1 * k1 + T.b6 * k6 + T.b7 * k7 + T.b8 * k8 + T.b9 * k9 + T.b10 * k10 + T.b11 * k11 + T.b12 * k12;
     const double y1 = y + h * b;
@@ -598,17 +609,23 @@ __device__ __forceinline__ int q_trial_rk_exact(const SimParams& P, const RkTab&
     }
 #define QX(TT, LANE, HP) q_rhs_exact(X, gravity, (TT), t0, yy, PULSE ? q_all<LANE>(HP) : 0.0)
     double yy = R.yy1;
-    const double k1 = QX(t, 0, hp0);
+    double k1 = QX(t, 0, hp0);
+    ST_CODE_ALIGN(k1);
     yy = y + (h * T.B21) * k1;
-    const double k2 = QX(t2, 1, hp0);
+    double k2 = QX(t2, 1, hp0);
+    ST_CODE_ALIGN(k2);
     yy = y + (h * T.B31) * k1 + (h * T.B32) * k2;
-    const double k3 = QX(t3, 2, hp0);
+    double k3 = QX(t3, 2, hp0);
+    ST_CODE_ALIGN(k3);
     yy = y + (h * T.B41) * k1 + (h * T.B42) * k2 + (h * T.B43) * k3;
-    const double k4 = QX(t4, 3, hp0);
+    double k4 = QX(t4, 3, hp0);
+    ST_CODE_ALIGN(k4);
     yy = y + (h * T.B51) * k1 + (h * T.B52) * k2 + (h * T.B53) * k3 + (h * T.B54) * k4;
-    const double k5 = QX(t5, 0, hp1);
+    double k5 = QX(t5, 0, hp1);
+    ST_CODE_ALIGN(k5);
     yy = y + (h * T.B61) * k1 + (h * T.B62) * k2 + (h * T.B63) * k3 + (h * T.B64) * k4 + (h * T.B65) * k5;
-    const double k6 = QX(t6, 1, hp1);
+    double k6 = QX(t6, 1, hp1);
+    ST_CODE_ALIGN(k6);
 #undef QX
     R.yy1 = yy;
     const double ws = y + h * (k1 * T.CH1 + k2 * rk::CH2 + k3 * T.CH3 + k4 * T.CH4 + k5 * T.CH5 + k6 * T.CH6);
