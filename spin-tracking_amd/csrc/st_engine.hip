@@ -458,13 +458,13 @@ static const void* spin_symbol(int variant, int integ, bool batch, bool pulse) {
 // Four lanes per particle (st_quad.h) as long as all of the list is on the
 // chip at once: 16 quads in each of two waves per SIMD, 32,768 particles on
 // 256 compute units.  k_spin of one lane and of four, He-3 x 0.2 s: 1.82 and
-// 0.90 ms at 1,000, 1.96 and 1.27 ms at 16,384, 2.01 and 1.63 ms at 32,768,
-// 2.14 and 2.48 ms at 49,152 (neutrons x 0.5 s: 2.97 and 2.47 ms at 32,768,
+// 0.79 ms at 1,000, 1.96 and 1.20 ms at 16,384, 2.01 and 1.59 ms at 32,768,
+// 2.14 and 2.48 ms at 49,152 (neutrons x 0.5 s: 2.97 and 2.42 ms at 32,768,
 // 3.10 and 3.52 ms at 49,152).  The exact variant on the same He-3: 4.32 and
-// 1.96 ms, 4.41 and 2.33 ms, 4.50 and 3.54 ms, 4.55 and 4.58 ms.  RK45,
-// neutrons x 0.5 ms: 10.7 and 8.2 ms at 16,384, 10.8 and 10.4 ms at 32,768,
-// 10.8 and 16.5 ms at 49,152 (exact 27.3 and 14.8, 27.4 and 23.6, 27.4 and
-// 32.5 ms).  0: the integrator has no such kernel, or the field hooks have
+// 1.86 ms, 4.41 and 2.35 ms, 4.50 and 3.59 ms, 4.55 and 4.58 ms.  RK45,
+// neutrons x 0.5 ms: 10.7 and 4.8 ms at 8,192, 10.8 and 7.7 ms at 32,768
+// 10.8 and 10.6 ms at 49,152 (exact 27.2 and 13.1, 27.4 and 22.0, 27.4 and
+// 30.7 ms).  0: the integrator has no such kernel, or the field hooks have
 // their own form.
 static uint32_t quad_limit(const st_handle* h) {
     if ((h->opt.integratorType != INT_DOP853 && h->opt.integratorType != INT_RK45) || !ST_FIELDS_POLYNOMIAL) return 0;

@@ -563,7 +563,7 @@ ST_HD __forceinline__ double rk_factor_fast(double tol, double e2_in, double& pr
     const double lr = 0.5 * ctl_log(tol * tol * fast_rcp(e2));
     const double q = ctl_exp(__builtin_fma(-0.4 / 7.0, prev_lr, (0.7 / 7.0) * lr));
     prev_lr = lr;
-    small = e2 < 4.0 * tol * tol;
+    small = e2 < 4.0 * (tol * tol);
     return q;
 }
 
@@ -576,26 +576,27 @@ ST_HD inline int rk_trial_fast(const SimParams& P, RkState& R, d3& y, double& h,
                                uint32_t& nacc, uint32_t& nrej) {
     using namespace rk;
     if (const int b = rk_bounds(P, R.t, R.tf, R.lastH, R.stop, R.nstep, h)) return b;
-    const double t = R.t, hpag = h * q.pag;
+    const double t = R.t, tx = t - S.t0, hpag = h * q.pag;
     const Poly hq{d3{h * q.w0.x, h * q.w0.y, h * q.w0.z}, d3{h * q.w1.x, h * q.w1.y, h * q.w1.z},
                   d3{h * q.w2.x, h * q.w2.y, h * q.w2.z}, q.pag, q.pw, q.paxis, q.pon};
-    auto K = [&](double tt, const d3& yy) -> d3 {
-        return cross3_fma(yy, poly_field<true>(tt - S.t0, hq, hpag, q.pon ? phase_cos(q.pw * tt) : 0.0));
+    auto K = [&](double c, const d3& yy) -> d3 {
+        return cross3_fma(yy, poly_field<true>(__builtin_fma(c, h, tx), hq, hpag,
+                                               q.pon ? phase_cos(q.pw * __builtin_fma(c, h, t)) : 0.0));
     };
     auto axpy = [](double a, const d3& k, const d3& s) -> d3 {
         return d3{__builtin_fma(a, k.x, s.x), __builtin_fma(a, k.y, s.y), __builtin_fma(a, k.z, s.z)};
     };
-    const d3 K1 = K(t, R.yy1);
+    const d3 K1 = cross3_fma(R.yy1, poly_field<true>(tx, hq, hpag, q.pon ? phase_cos(q.pw * t) : 0.0));
     d3 yy = axpy(B21, K1, y);
-    const d3 K2 = K(__builtin_fma(A2, h, t), yy);
+    const d3 K2 = K(A2, yy);
     yy = axpy(B31, K1, y); yy = axpy(B32, K2, yy);
-    const d3 K3 = K(__builtin_fma(A3, h, t), yy);
+    const d3 K3 = K(A3, yy);
     yy = axpy(B41, K1, y); yy = axpy(B42, K2, yy); yy = axpy(B43, K3, yy);
-    const d3 K4 = K(__builtin_fma(A4, h, t), yy);
+    const d3 K4 = K(A4, yy);
     yy = axpy(B51, K1, y); yy = axpy(B52, K2, yy); yy = axpy(B53, K3, yy); yy = axpy(B54, K4, yy);
-    const d3 K5 = K(__builtin_fma(A5, h, t), yy);
+    const d3 K5 = K(A5, yy);
     yy = axpy(B61, K1, y); yy = axpy(B62, K2, yy); yy = axpy(B63, K3, yy); yy = axpy(B64, K4, yy); yy = axpy(B65, K5, yy);
-    const d3 K6 = K(__builtin_fma(A6, h, t), yy);
+    const d3 K6 = K(A6, yy);
     R.yy1 = yy;
     d3 ws = axpy(CH1, K1, y);
     ws = axpy(CH3, K3, ws); ws = axpy(CH4, K4, ws); ws = axpy(CH5, K5, ws); ws = axpy(CH6, K6, ws);

@@ -2,8 +2,8 @@
 // not fill the chip.
 //
 // What bounds a small ensemble is one lane's chain of trial steps: with one
-// wave per SIMD nothing else can issue, and a lone wave needs 5.5 cycles for
-// an FP64 instruction and 9 for one that waits for the result before it.  A
+// wave per SIMD nothing else can issue, and a lone wave issues one instruction
+// in 4.3 cycles, whether or not it needs the result before it.  A
 // one-lane trial is about 1,000 instructions, the segment set-up that some
 // lane of a wave needs on most trips included (fast: 2.1 us on neutrons,
 // 3.2 us on He-3, whose segments are short; exact 5.4 and 7.1 us; 1.6 us per
@@ -17,11 +17,9 @@
 //     needs them for its state; a lane of a quad holds a third of that state);
 //   * the next segment record is loaded while the current one is integrated;
 //   * the pulse's stage cosines are split over the quad.
-// Per trial 1.0 us on neutrons and 1.5 us on He-3 (1,000 particles, fast),
-// 2.4 and 3.2 us exact.  RK45 (half the stages, and a controller that is a
-// chain of 60 dependent operations, a logarithm and an exponential): 0.88 us
-// fast, of one lane 1.15 (and 1.40 before its sums were chains of FMAs);
-// exact 1.60 and 2.92 us.
+// Per trial 0.86 us on neutrons and 1.3 us on He-3 (1,000 particles, fast),
+// 2.4 and 3.1 us exact.  RK45: 0.51 us fast, of one lane 1.15 (and 1.40 before
+// its sums were chains of FMAs); exact 1.41 and 2.92 us.
 // Every value is formed by the one-lane trial's operations in its order, so
 // accept/reject decisions and results are those of the one-lane kernels bit
 // for bit; a quad's four lanes always agree on the control flow.
@@ -150,8 +148,31 @@ struct QPulse {
 struct QDop {
     double x, xf, facold, k1, posneg;   // (posneg: exact variant)
     int32_t reject, last;
-    uint32_t nstep;
+    uint32_t left;                      // trials left before nmax is exceeded
 };
+
+// What the fast DOP853 trial reads of the caller's parameters.  A scalar load
+// costs a wave alone on its SIMD some 50 cycles, nine of them a fifth of a
+// trial's time, and all scalar registers are taken: here each lane of a quad
+// holds one of four values, and a use is a quad move of two instructions
+// (64 neutrons x 0.5 s: 1.26 and 1.11 ms).  (The exact trial has no vector
+// registers left for it: spilling two, it was 3 % slower.)
+struct DopCtl {
+    double a;         // lanes 0..3: atol, rtol, safe, hmin
+    double b;         // lanes 0..2: fac1, fac2, hmax
+    bool fixed;       // fixed step size
+    bool plain;       // no power needed (dop_factors)
+};
+__device__ __forceinline__ void dop_ctl_load(DopCtl& C, const SimParams& P) {
+    const uint32_t l = __lane_id() & 3u;
+    C.a = l == 0 ? P.atol : l == 1 ? P.rtol : l == 2 ? P.safe : P.hmin;
+    C.b = l == 0 ? P.fac1 : l == 1 ? P.fac2 : P.hmax;
+    asm volatile("" : "+v"(C.a), "+v"(C.b));
+    C.fixed = P.fixed != 0;
+    C.plain = !P.pow_beta_on && P.expo1 == 0.125;
+}
+// QDop::left of a new segment: the trials before nmax is exceeded
+__device__ __forceinline__ uint32_t dop_trials(const SimParams& P) { return min(P.nmax, 0xfffffffeu) + 1u; }
 
 // y x w of the lane's component, w given by its components a and b
 __device__ __forceinline__ double q_cross(double y, double wa, double wb) {
@@ -171,23 +192,20 @@ struct QQuad {
 };
 
 // dop_trial_fast_t (st_integrators.h) on a quad.  About 250 vector
-// instructions and 60 quad moves without a pulse; alone on its SIMD a wave
-// takes 0.95 us for them, 7 cycles each (an FP64 instruction of a lone wave
-// takes 5.5 cycles, 9 when it needs the result before it).  Writing the stage
-// sums so that older products fill the waits of the newest one, with the
-// order pinned, measured the same (0.99 and 0.98 us on 1,000 neutrons).
+// instructions and 70 quad moves without a pulse, 0.80 us alone on a SIMD.
 template <bool ADJ, bool PULSE>
-__device__ __forceinline__ int q_trial_fast(const SimParams& P, const DopTab& T, QDop& D, double& y, double& h,
+__device__ __forceinline__ int q_trial_fast(const SimParams& P, const DopCtl& C, const DopTab& T, QDop& D, double& y, double& h,
                                             double seg_t0, const QPoly& q, const QPulse& pl,
                                             uint32_t& nacc, uint32_t& nrej, QQuad* Q) {
 #pragma clang fp contract(fast)
-    if (D.nstep > P.nmax) return -1;
+    if (D.left == 0) return -1;
+    D.left--;
     if (D.x + 1.01 * h - D.xf > 0.0) {
         h = D.xf - D.x;
         D.last = 1;
     }
-    if (h < P.hmin && D.last != 1) h = P.hmin;
-    D.nstep++;
+    const double hmin = q_all<3>(C.a);
+    if (h < hmin && D.last != 1) h = hmin;
     const double x = D.x;
     const double tx = x - seg_t0;
     QPoly hq = q;
@@ -303,7 +321,7 @@ __device__ __forceinline__ int q_trial_fast(const SimParams& P, const DopTab& T,
         na = __builtin_fma(pl.ma, c12, na);
         nb = __builtin_fma(pl.mb, c12, nb);
     }
-    const double is = fast_rcp(P.atol + P.rtol * __builtin_fmax(fabs(y), fabs(y1)));
+    const double is = fast_rcp(q_all<0>(C.a) + q_all<1>(C.a) * __builtin_fmax(fabs(y), fabs(y1)));
     e = __builtin_fma(-T.bhh2, K9, e);
     e = __builtin_fma(-T.bhh3, K12, e);
     const double k1n = q_cross(y1, na, nb);
@@ -313,31 +331,36 @@ __device__ __forceinline__ int q_trial_fast(const SimParams& P, const DopTab& T,
     const double deno = e1 + 0.01 * err2;
     const double err = (deno <= 0.0) ? 0.0 : e1 * fast_rsq(3.0 * deno);
     double grow, shrink;
-    dop_factors(P, err, D.facold, grow, shrink);
-    double hnew = h * grow;
-    if (err <= 1.0 || P.fixed) {
-        D.facold = max_d(err, 1.0E-4);
-        nacc++;
-        D.k1 = k1n;
-        if constexpr (ADJ) {
+    if (C.plain) {   // dop_factors without a power
+        double inv = __builtin_inf();
+        if (err > 0.0) inv = fast_sqrt(fast_sqrt(fast_rsq(err)));   // err^(-1/8)
+        shrink = __builtin_fmax(q_all<0>(C.b), q_all<2>(C.a) * inv);
+        grow = __builtin_fmin(q_all<1>(C.b), shrink);
+    } else {
+        dop_factors(P, err, D.facold, grow, shrink);
+        if (err <= 1.0 || C.fixed) D.facold = max_d(err, 1.0E-4);
+    }
+    const bool ok = err <= 1.0 || C.fixed, done = ok && D.last;
+    nacc += ok;
+    nrej += !ok;
+    if constexpr (ADJ) {
+        if (ok) {
             Q->n0 = Q->n0 + h * q0;
             Q->n1 = Q->n1 + h * q1;
             Q->n2 = Q->n2 + h * q2;
         }
-        y = y1;
-        D.x = xph;
-        if (D.last) return 1;
-        if (fabs(hnew) > P.hmax) hnew = P.hmax;
-        if (D.reject) hnew = min_d(fabs(hnew), fabs(h));
-        D.reject = 0;
-    } else {
-        nrej++;
-        hnew = h * shrink;
-        D.reject = 1;
-        D.last = 0;
     }
-    if (!P.fixed) h = hnew;
-    return 0;
+    D.k1 = ok ? k1n : D.k1;
+    y = ok ? y1 : y;
+    D.x = ok ? xph : D.x;
+    double hnew = h * (ok ? grow : shrink);
+    const double hmax = q_all<2>(C.b);
+    hnew = ok && fabs(hnew) > hmax ? hmax : hnew;
+    hnew = ok && D.reject ? min_d(fabs(hnew), fabs(h)) : hnew;
+    h = done || C.fixed ? h : hnew;
+    D.reject = ok ? (done ? D.reject : 0) : 1;
+    D.last = ok ? D.last : 0;
+    return done;
 }
 
 // ---------------------------------------------------------------------------
@@ -395,13 +418,13 @@ __device__ __forceinline__ double q_rhs_exact(const QExact& X, bool gravity, dou
 template <bool PULSE>
 __device__ __forceinline__ int q_trial_exact(const SimParams& P, const DopTab& T, QDop& D, double& y, double& h,
                                              double t0, const QExact& X, uint32_t& nacc, uint32_t& nrej) {
-    if (D.nstep > P.nmax) return -1;
+    if (D.left == 0) return -1;
+    D.left--;
     if ((D.x + 1.01 * h - D.xf) * D.posneg > 0.0) {
         h = D.xf - D.x;
         D.last = 1;
     }
     if (h < P.hmin && D.last != 1) h = P.hmin;
-    D.nstep++;
     const double x = D.x, xph = x + h;
     const bool gravity = P.gravity;
     double hp0 = 0.0, hp1 = 0.0, hp2 = 0.0;
@@ -499,6 +522,78 @@ __device__ __forceinline__ void rk_tab_load(RkTab& T) {
     ST_RK_RESIDENT(X)
 #undef X
 }
+// What every trial reads besides, resident as well: the controller's series
+// and limits, and the caller's step-size parameters.  Alone on its SIMD a wave
+// issues an instruction in 4.3 cycles but waits some 50 for a scalar load, and
+// builds a literal with two instructions; of a trial's 522 issue slots 163
+// went by in waits and 97 in scalar instructions.  With these resident and
+// the step control in selects in place of branches, fast trials on 1,000
+// neutrons take 0.51 us (before: 0.90), exact ones 1.41 (1.63).
+// (0 and 1 of the series are inline constants; e[2] is too.)
+struct RkCtl {
+    double l[11], e[14];             // TAYLOR_HOST[2], [3]
+    double ln2_hi, ln2_lo, inv_ln2, clamp, root_half, grow, damp, accept, floor2;
+    double h0, hmax, hmin, tol2, tol2x4;
+    uint32_t nmax;
+    bool fixed;
+};
+__device__ __forceinline__ void rk_ctl_load(RkCtl& C, const SimParams& P) {
+    C.l[0] = C.e[0] = C.e[1] = 1.0;
+    C.e[2] = 0.5;
+#define ST_RK_CTL(N, ROW, K) N[K] = TAYLOR_HOST[ROW][K]; asm volatile("" : "+v"(N[K]));
+    ST_RK_CTL(C.l, 2, 1) ST_RK_CTL(C.l, 2, 2) ST_RK_CTL(C.l, 2, 3) ST_RK_CTL(C.l, 2, 4) ST_RK_CTL(C.l, 2, 5)
+    ST_RK_CTL(C.l, 2, 6) ST_RK_CTL(C.l, 2, 7) ST_RK_CTL(C.l, 2, 8) ST_RK_CTL(C.l, 2, 9) ST_RK_CTL(C.l, 2, 10)
+    ST_RK_CTL(C.e, 3, 3) ST_RK_CTL(C.e, 3, 4) ST_RK_CTL(C.e, 3, 5) ST_RK_CTL(C.e, 3, 6) ST_RK_CTL(C.e, 3, 7)
+    ST_RK_CTL(C.e, 3, 8) ST_RK_CTL(C.e, 3, 9) ST_RK_CTL(C.e, 3, 10) ST_RK_CTL(C.e, 3, 11) ST_RK_CTL(C.e, 3, 12)
+    ST_RK_CTL(C.e, 3, 13)
+#undef ST_RK_CTL
+#define ST_RK_CTL(N, V) C.N = V; asm volatile("" : "+s"(C.N));
+    ST_RK_CTL(ln2_hi, LN2_HI) ST_RK_CTL(ln2_lo, LN2_LO) ST_RK_CTL(inv_ln2, INV_LN2) ST_RK_CTL(clamp, 2000.0)
+    ST_RK_CTL(root_half, 0.70710678118654752440) ST_RK_CTL(grow, 0.7 / 7.0) ST_RK_CTL(damp, -0.4 / 7.0)
+    ST_RK_CTL(accept, 0.81) ST_RK_CTL(floor2, 1.0E-32)
+    ST_RK_CTL(h0, P.h0) ST_RK_CTL(hmax, P.hmax) ST_RK_CTL(hmin, P.hmin)
+#undef ST_RK_CTL
+    C.tol2 = P.rtol * P.rtol;
+    C.tol2x4 = 4.0 * C.tol2;
+    asm volatile("" : "+v"(C.tol2), "+v"(C.tol2x4));
+    C.nmax = P.nmax;
+    C.fixed = P.fixed != 0;
+}
+template <int N>
+__device__ __forceinline__ double q_series(const double (&c)[N], double x) {
+    double a = c[N - 1];
+#pragma unroll
+    for (int k = N - 2; k >= 0; --k) a = __builtin_fma(x, a, c[k]);
+    return a;
+}
+// ctl_log, ctl_exp and rk_factor_fast from the resident coefficients
+__device__ __forceinline__ double q_ctl_log(const RkCtl& C, double x) {
+    int e;
+    double m = frexp(x, &e);
+    if (m < C.root_half) {
+        m *= 2.0;
+        e -= 1;
+    }
+    const double r0 = __builtin_amdgcn_rcp(m + 1.0);
+    const double sv = (m - 1.0) * __builtin_fma(r0, __builtin_fma(-(m + 1.0), r0, 1.0), r0);
+    const double p = (2.0 * sv) * q_series(C.l, sv * sv);
+    double l = __builtin_fma((double)e, C.ln2_hi, __builtin_fma((double)e, C.ln2_lo, p));
+    if (!__builtin_amdgcn_class(x, 0x180)) l = log(x);   // not a positive finite number
+    return l;
+}
+__device__ __forceinline__ double q_ctl_exp(const RkCtl& C, double y) {
+    const double n = fmin(fmax(rint(y * C.inv_ln2), -C.clamp), C.clamp);
+    const double r = __builtin_fma(-n, C.ln2_lo, __builtin_fma(-n, C.ln2_hi, y));
+    return ldexp(q_series(C.e, r), (int)n);
+}
+__device__ __forceinline__ double q_rk_factor(const RkCtl& C, double e2_in, double& prev_lr, bool& small) {
+    const double e2 = std_max(e2_in, C.floor2);
+    const double lr = 0.5 * q_ctl_log(C, C.tol2 * fast_rcp(e2));
+    const double q = q_ctl_exp(C, __builtin_fma(C.damp, prev_lr, C.grow * lr));
+    prev_lr = lr;
+    small = e2 < C.tol2x4;
+    return q;
+}
 // RkState with the lane's component of yy1
 struct QRk {
     double t, tf, lastH, prev_ratio, prev_lr, yy1;
@@ -515,49 +610,57 @@ __device__ __forceinline__ void q_rk_begin(QRk& R, double t0, double t_end, doub
     R.prev_ratio = 1.0;
     R.prev_lr = 0.0;
 }
+// rk_bounds with one branch, taken at an error (h stays)
+__device__ __forceinline__ int q_rk_bounds(const RkCtl& C, QRk& R, double& h) {
+    R.nstep++;
+    const bool over = (uint32_t)R.nstep > C.nmax, below = !C.fixed && h < C.hmin && !(h > C.hmax);
+    if (over || below) return over ? -2 : -1;
+    const double endDt = R.tf - R.t;
+    const double hn = C.fixed ? C.h0 : (h > C.hmax ? C.hmax : h);
+    R.stop = hn >= endDt;
+    R.lastH = R.stop ? h : hn;
+    h = R.stop ? endDt : hn;
+    return 0;
+}
 // end of an iteration: accept or reject, next step size
-__device__ __forceinline__ int q_rk_end(const SimParams& P, QRk& R, double& y, double ws, double& h, double q_, bool small,
+__device__ __forceinline__ int q_rk_end(const RkCtl& C, QRk& R, double& y, double ws, double& h, double q_, bool small,
                                         uint32_t& nacc, uint32_t& nrej) {
     q_ = std_min(q_, 4.0);
-    if ((q_ > 0.81 && small) || P.fixed) {
-        nacc++;
-        y = ws;
-        R.t += h;
-        if (R.stop) {
-            h = R.lastH;
-            return 1;
-        }
-    } else {
-        nrej++;
-        if (R.stop) R.stop = false;
-    }
-    if (!P.fixed) h = h * q_;
-    return 0;
+    const bool ok = (q_ > C.accept && small) || C.fixed;
+    const bool done = ok && R.stop;
+    nacc += ok;
+    nrej += !ok;
+    y = ok ? ws : y;
+    R.t = ok ? R.t + h : R.t;
+    const double next = C.fixed ? h : h * q_;
+    h = done ? R.lastH : next;
+    R.stop = done;
+    return done;
 }
 // rk_trial_fast (st_integrators.h) on a quad; the pulse's cosines at the six
 // stage times are split over the quad.
 template <bool PULSE>
-__device__ __forceinline__ int q_trial_rk_fast(const SimParams& P, const RkTab& T, QRk& R, double& y, double& h,
+__device__ __forceinline__ int q_trial_rk_fast(const RkCtl& C, const RkTab& T, QRk& R, double& y, double& h,
                                                double t0, const QPoly& q, const QPulse& pl, uint32_t& nacc,
                                                uint32_t& nrej) {
-    if (const int b = rk_bounds(P, R.t, R.tf, R.lastH, R.stop, R.nstep, h)) return b;
-    const double t = R.t;
+    if (const int b = q_rk_bounds(C, R, h)) return b;
+    const double t = R.t, tx = t - t0;
     const QPoly hq{h * q.a0, h * q.a1, h * q.a2, h * q.b0, h * q.b1, h * q.b2};
-    const double t2 = __builtin_fma(T.A2, h, t), t3 = __builtin_fma(T.A3, h, t), t4 = __builtin_fma(T.A4, h, t),
-                 t5 = __builtin_fma(rk::A5, h, t), t6 = __builtin_fma(T.A6, h, t);
     double hp0 = 0.0, hp1 = 0.0, ha = 0.0, hb = 0.0;
     if constexpr (PULSE) {
         if (pl.on) {
             const uint32_t l = __lane_id() & 3u;
-            hp0 = phase_cos(pl.pw * (l == 0 ? t : l == 1 ? t2 : l == 2 ? t3 : t4));
-            hp1 = phase_cos(pl.pw * (l == 0 ? t5 : t6));
+            const double c0 = l == 1 ? T.A2 : l == 2 ? T.A3 : T.A4, c1 = l == 0 ? rk::A5 : T.A6;
+            const double t0_ = __builtin_fma(c0, h, t);
+            hp0 = phase_cos(pl.pw * (l == 0 ? t : t0_));
+            hp1 = phase_cos(pl.pw * __builtin_fma(c1, h, t));
             ha = h * pl.ma;
             hb = h * pl.mb;
         }
     }
-    auto K = [&](double tt, double yy, double cosv) -> double {
+    auto K = [&](double tau, double yy, double cosv) -> double {
         double wa, wb;
-        q_field(tt - t0, hq, wa, wb);
+        q_field(tau, hq, wa, wb);
         if constexpr (PULSE) {
             wa = __builtin_fma(ha, cosv, wa);
             wb = __builtin_fma(hb, cosv, wb);
@@ -565,22 +668,22 @@ __device__ __forceinline__ int q_trial_rk_fast(const SimParams& P, const RkTab& 
         return q_cross(yy, wa, wb);
     };
 #define QF(S, A, K) S = __builtin_fma(T.A, K, S)
-    const double K1 = K(t, R.yy1, q_all<0>(hp0));
+    const double K1 = K(tx, R.yy1, q_all<0>(hp0));
     double yy = y;
     QF(yy, B21, K1);
-    const double K2 = K(t2, yy, q_all<1>(hp0));
+    const double K2 = K(__builtin_fma(T.A2, h, tx), yy, q_all<1>(hp0));
     yy = y;
     QF(yy, B31, K1); QF(yy, B32, K2);
-    const double K3 = K(t3, yy, q_all<2>(hp0));
+    const double K3 = K(__builtin_fma(T.A3, h, tx), yy, q_all<2>(hp0));
     yy = y;
     QF(yy, B41, K1); QF(yy, B42, K2); QF(yy, B43, K3);
-    const double K4 = K(t4, yy, q_all<3>(hp0));
+    const double K4 = K(__builtin_fma(T.A4, h, tx), yy, q_all<3>(hp0));
     yy = y;
     QF(yy, B51, K1); QF(yy, B52, K2); QF(yy, B53, K3); QF(yy, B54, K4);
-    const double K5 = K(t5, yy, q_all<0>(hp1));
+    const double K5 = K(__builtin_fma(rk::A5, h, tx), yy, q_all<0>(hp1));
     yy = y;
     QF(yy, B61, K1); QF(yy, B62, K2); QF(yy, B63, K3); QF(yy, B64, K4); QF(yy, B65, K5);
-    const double K6 = K(t6, yy, q_all<1>(hp1));
+    const double K6 = K(__builtin_fma(T.A6, h, tx), yy, q_all<1>(hp1));
     R.yy1 = yy;
     double ws = y;
     QF(ws, CH1, K1); QF(ws, CH3, K3); QF(ws, CH4, K4); QF(ws, CH5, K5); QF(ws, CH6, K6);
@@ -589,14 +692,14 @@ __device__ __forceinline__ int q_trial_rk_fast(const SimParams& P, const RkTab& 
 #undef QF
     const d3 e = q_vec(te);
     bool small;
-    const double f = rk_factor_fast(P.rtol, __builtin_fma(e.z, e.z, __builtin_fma(e.y, e.y, e.x * e.x)), R.prev_lr, small);
-    return q_rk_end(P, R, y, ws, h, f, small, nacc, nrej);
+    const double f = q_rk_factor(C, __builtin_fma(e.z, e.z, __builtin_fma(e.y, e.y, e.x * e.x)), R.prev_lr, small);
+    return q_rk_end(C, R, y, ws, h, f, small, nacc, nrej);
 }
 // rk_trial_exact on a quad
 template <bool PULSE>
-__device__ __forceinline__ int q_trial_rk_exact(const SimParams& P, const RkTab& T, QRk& R, double& y, double& h,
+__device__ __forceinline__ int q_trial_rk_exact(const SimParams& P, const RkCtl& C, const RkTab& T, QRk& R, double& y, double& h,
                                                 double t0, const QExact& X, uint32_t& nacc, uint32_t& nrej) {
-    if (const int b = rk_bounds(P, R.t, R.tf, R.lastH, R.stop, R.nstep, h)) return b;
+    if (const int b = q_rk_bounds(C, R, h)) return b;
     const bool gravity = P.gravity;
     const double t = R.t, t2 = t + T.A2 * h, t3 = t + T.A3 * h, t4 = t + T.A4 * h, t5 = t + rk::A5 * h, t6 = t + T.A6 * h;
     double hp0 = 0.0, hp1 = 0.0;
@@ -639,7 +742,7 @@ __device__ __forceinline__ int q_trial_rk_exact(const SimParams& P, const RkTab&
     const double p = pow(low ? ratio : R.prev_ratio, low ? 0.7 / 7.0 : -0.4 / 7.0);
     const double f = q_all<0>(p) * q_all<2>(p);
     R.prev_ratio = ratio;
-    return q_rk_end(P, R, y, ws, h, f, error < 2 * tol, nacc, nrej);
+    return q_rk_end(C, R, y, ws, h, f, error < 2 * tol, nacc, nrej);
 }
 
 // The products make_poly reads, for the lane's components a = c+1 and b = c+2.
@@ -691,8 +794,15 @@ __device__ __forceinline__ void quad_spin() {
     constexpr bool DOP = INTEG == INT_DOP853;
     DopTab T;
     RkTab TR;
-    if constexpr (DOP) dop_tab_load<false>(T);
-    else rk_tab_load(TR);
+    RkCtl C;
+    DopCtl CD;
+    if constexpr (DOP) {
+        dop_tab_load<false>(T);
+        if constexpr (VAR == VAR_FAST) dop_ctl_load(CD, args().P);
+    } else {
+        rk_tab_load(TR);
+        rk_ctl_load(C, args().P);
+    }
     // a plain handle's physics in LDS, one copy per workgroup
     __shared__ Phys shared_phys;
     if constexpr (!BATCH) {
@@ -733,7 +843,7 @@ __device__ __forceinline__ void quad_spin() {
     };
     take();
     while (phase != S_DONE) {
-        if (lead) ++cnt[3];
+        cnt[3] += lead;
         if (phase == S_NEXT) {
             while (phase == S_NEXT) {
                 if (L.j >= L.nrec) {
@@ -768,7 +878,7 @@ __device__ __forceinline__ void quad_spin() {
                         dop.facold = 1.0E-4;
                         dop.last = 0;
                         dop.reject = 0;
-                        dop.nstep = 0;
+                        dop.left = dop_trials(args().P);
                         if constexpr (VAR == VAR_EXACT) {
                             dop.posneg = sign_d(1.0, rec.t - seg_t0);
                             dop.k1 = q_rhs_exact(X, args().P.gravity, seg_t0, seg_t0, y,
@@ -805,12 +915,20 @@ __device__ __forceinline__ void quad_spin() {
             }
         }
         if (phase == S_INT) {
+            // Trials until some quad of the wave ends its segment (DOP853 with
+            // more than four particles in the wave: one at a time, since some
+            // quad ends its segment on most trips; He-3 at 16 a wave: 1.20
+            // against 1.24 ms).
             int st;
-            const SimParams& P = args().P;
-            if constexpr (DOP && VAR == VAR_EXACT) st = q_trial_exact<PULSE>(P, T, dop, y, L.tempH, seg_t0, X, L.acc, L.rej);
-            else if constexpr (DOP) st = q_trial_fast<false, PULSE>(P, T, dop, y, L.tempH, seg_t0, q, pl, L.acc, L.rej, nullptr);
-            else if constexpr (VAR == VAR_EXACT) st = q_trial_rk_exact<PULSE>(P, TR, rk, y, L.tempH, seg_t0, X, L.acc, L.rej);
-            else st = q_trial_rk_fast<PULSE>(P, TR, rk, y, L.tempH, seg_t0, q, pl, L.acc, L.rej);
+            for (;;) {
+                const SimParams& P = args().P;
+                if constexpr (DOP && VAR == VAR_EXACT) st = q_trial_exact<PULSE>(P, T, dop, y, L.tempH, seg_t0, X, L.acc, L.rej);
+                else if constexpr (DOP) st = q_trial_fast<false, PULSE>(P, CD, T, dop, y, L.tempH, seg_t0, q, pl, L.acc, L.rej, nullptr);
+                else if constexpr (VAR == VAR_EXACT) st = q_trial_rk_exact<PULSE>(P, C, TR, rk, y, L.tempH, seg_t0, X, L.acc, L.rej);
+                else st = q_trial_rk_fast<PULSE>(C, TR, rk, y, L.tempH, seg_t0, q, pl, L.acc, L.rej);
+                if ((DOP && ppw > 4) || __any(st != 0)) break;
+                cnt[3] += lead;
+            }
             if (st != 0) {
                 const PipeArgs& A = args().A;
                 const RunArgs& R = A.R;
@@ -874,6 +992,8 @@ __global__ __launch_bounds__(256, 2) void k_adj_quad(const QuadAdjArgs) {
     const bool lead = first && (lane & 3u) == 0u, owner = first && (lane & 3u) != 3u;
     DopTab T;
     dop_tab_load<true>(T);
+    DopCtl CD;
+    dop_ctl_load(CD, args().P);
     __shared__ Phys shared_phys;
     // per lane: its gradient sums, and p0 and v0 of the segment being
     // integrated (registers go to the tableau)
@@ -980,7 +1100,7 @@ __global__ __launch_bounds__(256, 2) void k_adj_quad(const QuadAdjArgs) {
             dop.facold = 1.0E-4;
             dop.last = 0;
             dop.reject = 0;
-            dop.nstep = 0;
+            dop.left = dop_trials(args().P);
             double wa = q.a0, wb = q.b0;
             if constexpr (PULSE) {
                 const double cosv = pl.on ? phase_cos(pl.pw * rec.t) : 0.0;
@@ -991,7 +1111,7 @@ __global__ __launch_bounds__(256, 2) void k_adj_quad(const QuadAdjArgs) {
             phase = S_INT;
         }
         if (phase == S_INT) {
-            const int st = q_trial_fast<true, PULSE>(args().P, T, dop, u, h, 0.0, q, pl, nacc, nrej, &Q);
+            const int st = q_trial_fast<true, PULSE>(args().P, CD, T, dop, u, h, 0.0, q, pl, nacc, nrej, &Q);
             if (st < 0) {
                 fail = st;
                 --j;
