@@ -727,6 +727,7 @@ static int run_pipeline(st_handle* h, RunArgs R) {
     A.next_count = h->d_small + 1;
     A.integ = integ;
     A.phys = h->d_phys;
+    A.n_phys = h->n_cfg;
     A.no_recs = h->no_recs ? 1u : 0u;
     uint32_t n_list = h->n;
     int cur = 0;
@@ -1393,6 +1394,7 @@ ST_API int st_adjoint(st_handle* h, const void* blocks_dev, const double* seeds,
     A.next_list = next_list;
     A.integ = h->opt.integratorType;
     A.phys = h->d_phys;
+    A.n_phys = h->n_cfg;
     AdjArgs J;
     memset(&J, 0, sizeof J);
     J.recs = h->d_recs;

@@ -55,6 +55,7 @@ struct PipeArgs {
     uint32_t fail_cap;
     int32_t integ;           // integratorType
     const Phys* phys;        // batched handles: physics per configuration (F_CFG indexes it)
+    uint32_t n_phys;         // its entries
     // graph-captured chunks: the list length is read from here (set on the
     // device by the chunk head) instead of n_list; nullptr otherwise
     const uint32_t* n_list_dev;
@@ -653,19 +654,76 @@ __device__ __forceinline__ void spin_block(const RunArgs& R, const SpinLane& L) 
     if (R.blocks) write_block_spin(R.blocks + (uint64_t)L.k * R.block_bytes, R.n, L.pid, L.S);
 }
 
+// entries of a batched handle's physics the spin kernels hold in LDS (25 KB)
+constexpr uint32_t LDS_PHYS = 64;
+
+// The record a lane needs next, brought to LDS while the current one is
+// integrated.  Loaded where it is needed, a record (and the physics, loaded
+// after it) kept the whole wave waiting for memory on nearly every trip, 43 %
+// of its cycles on He-3: some lane of 64 is always at a segment's end, and
+// there are no 16 registers to hold a record in.  (The loads write LDS by lane
+// of the wave, 16 bytes each at the row's start + 16 * lane.)  k_spin, fast
+// DOP853, He-3 x 0.2 s: 65,536 particles 2.29 and 1.98 ms, 262,144 5.44 and
+// 4.52 ms; at 1,048,576 the card's power bounds it, and the clock falls by as
+// much as the waits did.
+template <bool USED>
+struct NextRec {
+    char* rows;     // the wave's four rows of 64 x 16 bytes
+    __device__ __forceinline__ NextRec() {
+        if constexpr (!USED) return;
+        __shared__ __attribute__((aligned(16))) char buf[4][4 * 1024];
+        rows = buf[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];
+    }
+    __device__ __forceinline__ void fetch(const char* at) const {
+        typedef __attribute__((address_space(1))) void gvoid;
+        typedef __attribute__((address_space(3))) void lvoid;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the row has been read
+        __builtin_amdgcn_global_load_lds((gvoid*)(at), (lvoid*)(rows), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((gvoid*)(at + 16), (lvoid*)(rows + 1024), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((gvoid*)(at + 32), (lvoid*)(rows + 2048), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((gvoid*)(at + 48), (lvoid*)(rows + 3072), 16, 0, 0);
+    }
+    __device__ __forceinline__ SegRec take() const {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        const char* r = rows + 16 * __lane_id();
+        auto d = [&](int q, int i) { return *reinterpret_cast<const double*>(r + 1024 * q + 8 * i); };
+        SegRec s;
+        s.t = d(0, 0); s.px = d(0, 1); s.py = d(1, 0); s.pz = d(1, 1); s.vx = d(2, 0); s.vy = d(2, 1); s.vz = d(3, 0);
+        s.flags = *reinterpret_cast<const uint64_t*>(r + 3072 + 8);
+        return s;
+    }
+};
+
 template <int VAR, int INTEG, bool BATCH, bool PULSE>
 __device__ __forceinline__ void spin_body(const SimParams& P, const DevState& D, const PipeArgs& A) {
+    // (the others take many trials per segment: RK45 8 % slower, at its register
+    // line, exact RKF45 15 %, which reads the physics in every stage)
+    constexpr bool AHEAD = INTEG == INT_DOP853 || INTEG == INT_MAGNUS || (VAR == VAR_FAST && INTEG == INT_RKF45);
     const RunArgs& R = A.R;
     SpinLane L;
-    // physics of the lane's current particle
-    // (a plain handle's single entry is read through the same table: uniform
-    // scalar loads at each segment set-up instead of ~50 SGPRs held across
-    // the loop)
+    // physics of the lane's current particle from a copy in LDS: a plain
+    // handle's single entry, and a batched handle's table where it fits (fast
+    // variant, which reads it at a segment's set-up only)
+    constexpr bool TABLE = AHEAD && BATCH && VAR == VAR_FAST;
+    __shared__ Phys lds_phys[TABLE ? LDS_PHYS : 1];
+    const bool table = TABLE && A.n_phys <= LDS_PHYS;
+    if (AHEAD && (!BATCH || table)) {
+        const uint32_t words = (BATCH ? A.n_phys : 1u) * (uint32_t)(sizeof(Phys) / 4);
+        for (uint32_t i = threadIdx.x; i < words; i += blockDim.x)
+            reinterpret_cast<uint32_t*>(lds_phys)[i] = reinterpret_cast<const uint32_t*>(A.phys)[i];
+        __syncthreads();
+    }
     auto phys = [&]() -> const Phys& {
         if constexpr (BATCH)
             return A.phys[L.cfg];
+        else if constexpr (AHEAD)
+            return lds_phys[0];
         else
             return A.phys[0];
+    };
+    NextRec<AHEAD> next;
+    auto fetch = [&](uint32_t j) {
+        if (AHEAD && j < L.nrec) next.fetch(rec_at_seq(A, L.pid, j, L.page));
     };
     DopState dop;
     RkState rk;
@@ -687,6 +745,7 @@ __device__ __forceinline__ void spin_body(const SimParams& P, const DevState& D,
         const uint32_t q = acquire_index(R.queue);
         if (q < n_list) {
             spin_load<BATCH>(D, A, A.list[q], L);
+            fetch(0);
             phase = S_NEXT;
         }
     }
@@ -702,19 +761,26 @@ __device__ __forceinline__ void spin_body(const SimParams& P, const DevState& D,
                     const uint32_t q = acquire_index(R.queue);
                     if (q < n_list) {
                         spin_load<BATCH>(D, A, A.list[q], L);
+                        fetch(0);
                         phase = S_NEXT;
                         continue;
                     }
                     break;
                 }
-                const SegRec rec = load_rec(rec_at_seq(A, L.pid, L.j, L.page));
+                const SegRec rec = AHEAD ? next.take() : load_rec(rec_at_seq(A, L.pid, L.j, L.page));
+                fetch(L.j + 1);
                 cur_flags = (uint32_t)rec.flags;
                 if (rec.flags & R_FIRST) L.tempH = L.h;
                 if ((rec.flags & R_INTEGRATE) && !L.stopped) {
                     seg.t0 = L.t_spin;
                     seg.p0 = d3{rec.px, rec.py, rec.pz};
                     seg.v0 = d3{rec.vx, rec.vy, rec.vz};
-                    if (VAR == VAR_FAST) poly = make_poly(P, phys(), seg);
+                    if constexpr (TABLE) {
+                        if (table) poly = make_poly(P, lds_phys[L.cfg], seg);
+                        else poly = make_poly(P, phys(), seg);
+                    } else if constexpr (VAR == VAR_FAST) {
+                        poly = make_poly(P, phys(), seg);
+                    }
                     if (INTEG == INT_DOP853) {
                         if (VAR == VAR_EXACT) dop_begin_exact(P, phys(), dop, L.S, seg, rec.t);
                         else dop_begin_fast(P, phys(), dop, L.S, seg, poly, rec.t);
