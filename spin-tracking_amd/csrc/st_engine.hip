@@ -464,10 +464,13 @@ static const void* spin_symbol(int variant, int integ, bool batch, bool pulse) {
 // 1.86 ms, 4.41 and 2.35 ms, 4.50 and 3.59 ms, 4.55 and 4.58 ms.  RK45,
 // neutrons x 0.5 ms: 10.7 and 4.8 ms at 8,192, 10.8 and 7.7 ms at 32,768
 // 10.8 and 10.6 ms at 49,152 (exact 27.2 and 13.1, 27.4 and 22.0, 27.4 and
-// 30.7 ms).  0: the integrator has no such kernel, or the field hooks have
-// their own form.
+// 30.7 ms).  Fast MagnusCFET, He-3 x 0.2 s: 2.34 and 1.17 ms at 32,768, 2.4
+// and 1.95 ms at 49,152.  0: the integrator has no such kernel, or the field
+// hooks have their own form.
 static uint32_t quad_limit(const st_handle* h) {
-    if ((h->opt.integratorType != INT_DOP853 && h->opt.integratorType != INT_RK45) || !ST_FIELDS_POLYNOMIAL) return 0;
+    const int integ = h->opt.integratorType;
+    if (!ST_FIELDS_POLYNOMIAL) return 0;
+    if (integ != INT_DOP853 && integ != INT_RK45 && !(integ == INT_MAGNUS && h->ext.variant == ST_VARIANT_FAST)) return 0;
     return 32u * (uint32_t)h->n_simd;
 }
 // particles per wave: one until every SIMD has a wave, then doubling to 16
@@ -493,6 +496,7 @@ static hipError_t spin_quad_v(st_handle* h, const PipeArgs& A) {
 }
 static hipError_t spin_quad(st_handle* h, const PipeArgs& A) {
     const bool fast = h->ext.variant == ST_VARIANT_FAST;
+    if (h->opt.integratorType == INT_MAGNUS) return spin_quad_v<VAR_FAST, INT_MAGNUS>(h, A);
     if (h->opt.integratorType == INT_RK45)
         return fast ? spin_quad_v<VAR_FAST, INT_RK45>(h, A) : spin_quad_v<VAR_EXACT, INT_RK45>(h, A);
     return fast ? spin_quad_v<VAR_FAST, INT_DOP853>(h, A) : spin_quad_v<VAR_EXACT, INT_DOP853>(h, A);

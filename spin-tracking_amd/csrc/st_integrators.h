@@ -888,9 +888,12 @@ ST_HD __forceinline__ d3 rodriguez_v(const d3& k, const d3& v) {
 // vector once (q v q* as v + w t + u x t, t = 2 u x v), in place of a
 // 30-operation vector rotation per factor; the same rotations, rounded
 // differently.
+ST_HD __forceinline__ double len2_fma(const d3& g) {
+    return __builtin_fma(g.z, g.z, __builtin_fma(g.y, g.y, g.x * g.x));
+}
 ST_HD __forceinline__ Quat rot_quat_half(const d3& g) {
 #pragma clang fp contract(fast)
-    const double t2 = g.x * g.x + g.y * g.y + g.z * g.z;   // (theta/2)^2
+    const double t2 = len2_fma(g);   // (theta/2)^2
     if (t2 > 0.0 && t2 <= 0.25 * FAST_ROT_MAX_X2) {
         double ch, sh;
         cos_sinc_doubled<1, false, true>(t2, ch, sh);
@@ -898,17 +901,18 @@ ST_HD __forceinline__ Quat rot_quat_half(const d3& g) {
     }
     return rodriguez_quat(d3{-2.0 * g.x, -2.0 * g.y, -2.0 * g.z}, 1.0);
 }
+// (the FMAs are written out: the one-lane and the quad kernels form the same bits)
 ST_HD __forceinline__ Quat q_mult_fast(const Quat& a, const Quat& b) {
-#pragma clang fp contract(fast)
-    return Quat{a.w * b.w - a.x * b.x - a.y * b.y - a.z * b.z, a.w * b.x + a.x * b.w + a.y * b.z - a.z * b.y,
-                a.w * b.y + a.y * b.w + a.z * b.x - a.x * b.z, a.w * b.z + a.z * b.w + a.x * b.y - a.y * b.x};
+    auto f = [](double x, double y, double z) -> double { return __builtin_fma(x, y, z); };
+    return Quat{f(-a.z, b.z, f(-a.y, b.y, f(-a.x, b.x, a.w * b.w))), f(-a.z, b.y, f(a.y, b.z, f(a.x, b.w, a.w * b.x))),
+                f(-a.x, b.z, f(a.z, b.x, f(a.y, b.w, a.w * b.y))), f(-a.y, b.x, f(a.x, b.y, f(a.z, b.w, a.w * b.z)))};
 }
 ST_HD __forceinline__ d3 qrot_fast(const Quat& q, const d3& v) {
-#pragma clang fp contract(fast)
-    const double tx = 2.0 * (q.y * v.z - q.z * v.y), ty = 2.0 * (q.z * v.x - q.x * v.z),
-                 tz = 2.0 * (q.x * v.y - q.y * v.x);
-    return d3{v.x + q.w * tx + (q.y * tz - q.z * ty), v.y + q.w * ty + (q.z * tx - q.x * tz),
-              v.z + q.w * tz + (q.x * ty - q.y * tx)};
+    auto f = [](double x, double y, double z) -> double { return __builtin_fma(x, y, z); };
+    const double tx = 2.0 * f(q.y, v.z, -(q.z * v.y)), ty = 2.0 * f(q.z, v.x, -(q.x * v.z)),
+                 tz = 2.0 * f(q.x, v.y, -(q.y * v.x));
+    return d3{f(q.w, tx, v.x) + f(q.y, tz, -(q.z * ty)), f(q.w, ty, v.y) + f(q.z, tx, -(q.x * tz)),
+              f(q.w, tz, v.z) + f(q.x, ty, -(q.y * tx))};
 }
 
 // the quaternion of a rotation by |k| dt: half angle p = |k| dt / 2,
@@ -1057,8 +1061,7 @@ ST_HD __forceinline__ int bounds_v2(const SimParams& P, RkState& R, double& h) {
 template <int VAR>
 ST_HD __forceinline__ double err_arg(const d3& d) {
     if constexpr (VAR == VAR_FAST) {
-#pragma clang fp contract(fast)
-        return d.x * d.x + d.y * d.y + d.z * d.z;
+        return len2_fma(d);
     } else {
         return len3(d);
     }
@@ -1275,10 +1278,11 @@ ST_HD inline int rk2_trial(const SimParams& P, const Phys& Fp, RkState& R, d3& y
 #else
                 const double* m = CFET_MOM_HOST.m[r];
 #endif
-                d3 k{m[0] * u0.x + m[1] * u1.x + m[2] * u2.x, m[0] * u0.y + m[1] * u1.y + m[2] * u2.y,
-                     m[0] * u0.z + m[1] * u1.z + m[2] * u2.z};
+                auto f = [](double x, double y, double z) -> double { return __builtin_fma(x, y, z); };
+                d3 k{f(m[2], u2.x, f(m[1], u1.x, m[0] * u0.x)), f(m[2], u2.y, f(m[1], u1.y, m[0] * u0.y)),
+                     f(m[2], u2.z, f(m[1], u1.z, m[0] * u0.z))};
                 if (pon) {
-                    const double pe = m[3] * hp[0] + m[4] * hp[1] + m[5] * hp[2] + m[6] * hp[3] + m[7] * hp[4];
+                    const double pe = f(m[7], hp[4], f(m[6], hp[3], f(m[5], hp[2], f(m[4], hp[1], m[3] * hp[0]))));
                     k.x += q.paxis == 0 ? pe : 0.0;
                     k.y += q.paxis == 1 ? pe : 0.0;
                     k.z += q.paxis == 2 ? pe : 0.0;

@@ -49,6 +49,10 @@ __device__ __forceinline__ double q_all(double v) {
 }
 __device__ __forceinline__ d3 q_vec(double v) { return d3{q_all<0>(v), q_all<1>(v), q_all<2>(v)}; }
 
+// lane I's vector in all four lanes
+template <int I>
+__device__ __forceinline__ d3 q_vec3(const d3& v) { return d3{q_all<I>(v.x), q_all<I>(v.y), q_all<I>(v.z)}; }
+
 // v[c], c = 0..2
 __device__ __forceinline__ double q_pick(const d3& v, uint32_t c) { return c == 0 ? v.x : (c == 1 ? v.y : v.z); }
 
@@ -745,6 +749,171 @@ __device__ __forceinline__ int q_trial_rk_exact(const SimParams& P, const RkCtl&
     return q_rk_end(C, R, y, ws, h, f, error < 2 * tol, nacc, nrej);
 }
 
+// ---------------------------------------------------------------------------
+// MagnusCFET (integratorType 2, fast variant) on a quad
+// ---------------------------------------------------------------------------
+// The one-lane trial forms sixteen rotations one after another, each with its
+// scalar loads of coefficients to wait for: 8.4 us on He-3 with a wave per
+// SIMD.  On a quad each lane forms four of them, from coefficients it keeps:
+//   lane 0: factors 0, 3, 6, 9 of the order-8 chain, lane 1: 1, 4, 7, 10,
+//   lane 2: 2, 5, 8 and the order-6 chain's last, lane 3: that chain's 0..3.
+// The products then follow the one-lane trial's order, the order-8 chain in
+// lanes 0 and 1, the order-6 chain in lanes 2 and 3, each factor brought from
+// its lane by quad moves.  k_spin, He-3 x 0.2 s: 4,096 particles 2.19 and
+// 0.79 ms, 32,768 2.34 and 1.17 ms (65,536, past the limit: 2.25 and 2.19 ms).
+struct MagTab {
+    double m[4][3];          // the lane's four exponents (CFET_MOM)
+    double c[8], s[8];       // the series of half_series<true>
+};
+__device__ __forceinline__ uint32_t mag_row(uint32_t l, uint32_t slot) {
+    return l < 3 ? (l == 2 && slot == 3 ? 15u : 3 * slot + l) : 11 + slot;
+}
+__device__ __forceinline__ double mag_coef(uint32_t row, int k) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return CFET_MOM.m[row][k];
+#else
+    return CFET_MOM_HOST.m[row][k];
+#endif
+}
+__device__ __forceinline__ void mag_tab_load(MagTab& T) {
+    const uint32_t l = __lane_id() & 3u;
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            T.m[j][k] = mag_coef(mag_row(l, j), k);
+            asm volatile("" : "+v"(T.m[j][k]));
+        }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        T.c[k] = TAYLOR_HOST[0][k];
+        T.s[k] = TAYLOR_HOST[1][k];
+        if (k > 1) asm volatile("" : "+v"(T.c[k]));   // (1 and -1/2 are inline constants)
+        if (k > 0) asm volatile("" : "+v"(T.s[k]));
+    }
+}
+// rot_quat_half from the resident series
+__device__ __forceinline__ Quat q_rot_half(const MagTab& T, const d3& g) {
+#pragma clang fp contract(fast)
+    const double t2 = len2_fma(g);
+    const bool extra = t2 >= 1.0;   // beyond one halving (cos_sinc_doubled<1, true, true>)
+    int d = 1;
+    double x2 = t2 * 0.25;
+    if (__any(extra)) {
+        int E;
+        (void)frexp(t2, &E);
+        d = E + 2 > 2 ? (E + 3) >> 1 : 1;
+        x2 = ldexp(t2, -2 * d);
+    }
+    double c = q_series(T.c, x2), s = q_series(T.s, x2);
+    auto twice = [&]() {
+        const double s2 = s * s;
+        s = s * c;
+        c = 1.0 - (2.0 * x2) * s2;
+        x2 *= 4.0;
+    };
+    const bool good = t2 > 0.0 && t2 <= 0.25 * FAST_ROT_MAX_X2;
+    if (__any(extra && good))
+        for (int i = good ? d : 1; i > 1; --i) twice();
+    twice();
+    Quat r{c, g.x * s, g.y * s, g.z * s};
+    if (!good) r = rodriguez_quat(d3{-2.0 * g.x, -2.0 * g.y, -2.0 * g.z}, 1.0);
+    return r;
+}
+// lane A's value in lanes 0 and 1, lane B's in lanes 2 and 3
+template <int A, int B>
+__device__ __forceinline__ Quat q_pair(const Quat& q) {
+    constexpr int CTRL = A | A << 2 | B << 4 | B << 6;
+    return Quat{quad_perm<CTRL>(q.w), quad_perm<CTRL>(q.x), quad_perm<CTRL>(q.y), quad_perm<CTRL>(q.z)};
+}
+// bounds_v2 with one branch, taken at an error (h stays)
+__device__ __forceinline__ int q_bounds_v2(const RkCtl& C, QRk& R, double& h) {
+    R.nstep++;
+    const double endDt = R.tf - R.t;
+    const bool ends = !C.fixed && h >= endDt;
+    const bool over = (uint32_t)R.nstep > C.nmax, below = !C.fixed && !ends && h < C.hmin && !(h > C.hmax);
+    if (over || below) return over ? -2 : -1;
+    R.lastH = h;
+    R.stop = C.fixed ? R.stop : ends;
+    h = C.fixed ? C.h0 : ends ? endDt : (h > C.hmax ? C.hmax : h);
+    return 0;
+}
+template <bool PULSE>
+__device__ __forceinline__ int q_trial_magnus(const RkCtl& C, const MagTab& T, QRk& R, double& y, double& h, double t0,
+                                              const Poly& q, uint32_t c, uint32_t& nacc, uint32_t& nrej) {
+#pragma clang fp contract(fast)
+    if (const int b = q_bounds_v2(C, R, h)) return b;
+    const double t = R.t;
+    const double tau = t - t0, h2 = h * h, h3 = h2 * h, tt = 2.0 * tau;
+    const d3 u0{h * (q.w0.x + tau * (q.w1.x + tau * q.w2.x)), h * (q.w0.y + tau * (q.w1.y + tau * q.w2.y)),
+                h * (q.w0.z + tau * (q.w1.z + tau * q.w2.z))};
+    const d3 u1{h2 * (q.w1.x + tt * q.w2.x), h2 * (q.w1.y + tt * q.w2.y), h2 * (q.w1.z + tt * q.w2.z)};
+    const d3 u2{h3 * q.w2.x, h3 * q.w2.y, h3 * q.w2.z};
+    auto f = [](double x, double y, double z) -> double { return __builtin_fma(x, y, z); };
+    const uint32_t l = __lane_id() & 3u;
+    double hp[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    if constexpr (PULSE) {
+        if (q.pon) {   // h * pulse at the five nodes, four of them a lane each
+            using namespace cfet;
+            const double X = l == 0 ? X1 : l == 1 ? X2 : l == 2 ? X3 : X4;
+            const double a = h * (q.pag * phase_cos(q.pw * (t + X * h)));
+            hp[0] = q_all<0>(a); hp[1] = q_all<1>(a); hp[2] = q_all<2>(a); hp[3] = q_all<3>(a);
+            hp[4] = h * (q.pag * phase_cos(q.pw * (t + X5 * h)));
+        }
+    }
+    auto rot = [&](int j) -> Quat {
+        const double* m = T.m[j];
+        d3 k{f(m[2], u2.x, f(m[1], u1.x, m[0] * u0.x)), f(m[2], u2.y, f(m[1], u1.y, m[0] * u0.y)),
+             f(m[2], u2.z, f(m[1], u1.z, m[0] * u0.z))};
+        if constexpr (PULSE) {
+            if (q.pon) {
+                const uint32_t r = mag_row(l, j);
+                const double pe = f(mag_coef(r, 7), hp[4],
+                                    f(mag_coef(r, 6), hp[3],
+                                      f(mag_coef(r, 5), hp[2], f(mag_coef(r, 4), hp[1], mag_coef(r, 3) * hp[0]))));
+                k.x += q.paxis == 0 ? pe : 0.0;
+                k.y += q.paxis == 1 ? pe : 0.0;
+                k.z += q.paxis == 2 ? pe : 0.0;
+            }
+        }
+        return q_rot_half(T, k);
+    };
+    const Quat r0 = rot(0), r1 = rot(1), r2 = rot(2), r3 = rot(3);
+    // order 8 | order 6
+    Quat p = q_pair<0, 3>(r0);
+    {
+        const Quat b = q_pair<1, 3>(Quat{l == 3 ? r1.w : r0.w, l == 3 ? r1.x : r0.x, l == 3 ? r1.y : r0.y, l == 3 ? r1.z : r0.z});
+        p = q_mult_fast(b, p);       // factor 1 | 1
+    }
+    {
+        const Quat b = q_pair<2, 3>(Quat{l == 3 ? r2.w : r0.w, l == 3 ? r2.x : r0.x, l == 3 ? r2.y : r0.y, l == 3 ? r2.z : r0.z});
+        p = q_mult_fast(b, p);       // 2 | 2
+    }
+    {
+        const Quat b = q_pair<0, 3>(Quat{l == 3 ? r3.w : r1.w, l == 3 ? r3.x : r1.x, l == 3 ? r3.y : r1.y, l == 3 ? r3.z : r1.z});
+        p = q_mult_fast(b, p);       // 3 | 3
+    }
+    {
+        const Quat b = q_pair<1, 2>(Quat{l == 2 ? r3.w : r1.w, l == 2 ? r3.x : r1.x, l == 2 ? r3.y : r1.y, l == 2 ? r3.z : r1.z});
+        p = q_mult_fast(b, p);       // 4 | 4, the order-6 chain's last
+    }
+    Quat p8 = p;                     // (lanes 2 and 3: repeated work)
+    p8 = q_mult_fast(q_pair<2, 2>(r1), p8);
+    p8 = q_mult_fast(q_pair<0, 0>(r2), p8);
+    p8 = q_mult_fast(q_pair<1, 1>(r2), p8);
+    p8 = q_mult_fast(q_pair<2, 2>(r2), p8);
+    p8 = q_mult_fast(q_pair<0, 0>(r3), p8);
+    p8 = q_mult_fast(q_pair<1, 1>(r3), p8);
+    const bool six = l >= 2;
+    const Quat qq{six ? p.w : p8.w, six ? p.x : p8.x, six ? p.y : p8.y, six ? p.z : p8.z};
+    const d3 v = qrot_fast(qq, q_vec(y));
+    const d3 y8 = q_vec3<0>(v), y6 = q_vec3<2>(v);
+    const d3 d{y8.x - y6.x, y8.y - y6.y, y8.z - y6.z};
+    bool small;
+    const double fac = q_rk_factor(C, len2_fma(d), R.prev_lr, small);
+    return q_rk_end(C, R, y, q_pick(y8, c), h, fac, small, nacc, nrej);
+}
+
 // The products make_poly reads, for the lane's components a = c+1 and b = c+2.
 __device__ __forceinline__ void q_pulse_load(QPulse& pl, const Phys& F, uint32_t c, double sign = 1.0) {
     const int32_t a = c == 2 ? 0 : (int32_t)c + 1, b = c == 0 ? 2 : (int32_t)c - 1;
@@ -791,16 +960,19 @@ __device__ __forceinline__ void quad_spin() {
     const uint32_t ppw = args().ppw;
     const bool first = (lane >> 2) < ppw;
     const bool lead = first && (lane & 3u) == 0u, owner = first && (lane & 3u) != 3u;
-    constexpr bool DOP = INTEG == INT_DOP853;
+    constexpr bool DOP = INTEG == INT_DOP853, MAG = INTEG == INT_MAGNUS;
+    static_assert(!MAG || VAR == VAR_FAST, "MagnusCFET on quads is the fast variant's");
     DopTab T;
     RkTab TR;
+    MagTab TM;
     RkCtl C;
     DopCtl CD;
     if constexpr (DOP) {
         dop_tab_load<false>(T);
         if constexpr (VAR == VAR_FAST) dop_ctl_load(CD, args().P);
     } else {
-        rk_tab_load(TR);
+        if constexpr (MAG) mag_tab_load(TM);
+        else rk_tab_load(TR);
         rk_ctl_load(C, args().P);
     }
     // a plain handle's physics in LDS, one copy per workgroup
@@ -814,7 +986,7 @@ __device__ __forceinline__ void quad_spin() {
     QExact X;
     auto physics = [&](const Phys& F) {
         if constexpr (VAR == VAR_EXACT) q_exact_load(X, args().P, F, c);
-        else if constexpr (PULSE) q_pulse_load(pl, F, c);
+        else if constexpr (PULSE && !MAG) q_pulse_load(pl, F, c);
     };
     if constexpr (!BATCH) physics(shared_phys);
     SpinLane L;      // (S unused: the lane's component is y)
@@ -822,6 +994,7 @@ __device__ __forceinline__ void quad_spin() {
     QDop dop;
     QRk rk;
     QPoly q;
+    Poly full;       // (MagnusCFET: all components)
     auto seg_end = [&]() { return DOP ? dop.xf : rk.tf; };
     double seg_t0 = 0.0;
     SegRec nxt;      // record L.j, loaded while record L.j - 1 is integrated
@@ -868,6 +1041,13 @@ __device__ __forceinline__ void quad_spin() {
                     if constexpr (VAR == VAR_EXACT) {
                         X.p0 = q_pick(d3{rec.px, rec.py, rec.pz}, c);
                         X.v0 = q_pick(d3{rec.vx, rec.vy, rec.vz}, c);
+                    } else if constexpr (MAG) {
+                        Seg seg;
+                        seg.t0 = seg_t0;
+                        seg.p0 = d3{rec.px, rec.py, rec.pz};
+                        seg.v0 = d3{rec.vx, rec.vy, rec.vz};
+                        full = make_poly(args().P, BATCH ? A.phys[L.cfg] : shared_phys, seg);
+                        if constexpr (!PULSE) full.pon = 0;
                     } else {
                         q_make_poly(q, BATCH ? A.phys[L.cfg] : shared_phys, d3{rec.px, rec.py, rec.pz},
                                     d3{rec.vx, rec.vy, rec.vz}, c);
@@ -925,6 +1105,7 @@ __device__ __forceinline__ void quad_spin() {
                 if constexpr (DOP && VAR == VAR_EXACT) st = q_trial_exact<PULSE>(P, T, dop, y, L.tempH, seg_t0, X, L.acc, L.rej);
                 else if constexpr (DOP) st = q_trial_fast<false, PULSE>(P, CD, T, dop, y, L.tempH, seg_t0, q, pl, L.acc, L.rej, nullptr);
                 else if constexpr (VAR == VAR_EXACT) st = q_trial_rk_exact<PULSE>(P, C, TR, rk, y, L.tempH, seg_t0, X, L.acc, L.rej);
+                else if constexpr (MAG) st = q_trial_magnus<PULSE>(C, TM, rk, y, L.tempH, seg_t0, full, c, L.acc, L.rej);
                 else st = q_trial_rk_fast<PULSE>(C, TR, rk, y, L.tempH, seg_t0, q, pl, L.acc, L.rej);
                 if ((DOP && ppw > 4) || __any(st != 0)) break;
                 cnt[3] += lead;

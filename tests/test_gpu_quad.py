@@ -23,6 +23,8 @@ def options(kind, n, seed, integ=0):
         st.set_fields(o, yi=(0.0, 1.0, 0.0))
     if integ == 1:      # RK45: far more steps per second at a loose tolerance already
         st.set_fields(o, integratorType=1, rtol=1e-9, tf=o.tf / 20.0, ioutInt=o.ioutInt / 20.0)
+    if integ == 2:      # MagnusCFET: steps of tens of radians on the neutrons' smooth field
+        st.set_fields(o, integratorType=2, rtol=1e-6)
     return o
 
 
@@ -60,6 +62,13 @@ def test_quad_equals_one_lane(kind, variant, n, integ):
         y = braw[k * bbb:(k + 1) * bbb].view(st.snapshot_block_dtype(n + FILLER))[0]
         for name in x.dtype.names:
             assert x[name].tobytes() == y[name][:n].tobytes(), (k, name)
+
+
+# MagnusCFET has quads in its fast variant only
+@pytest.mark.parametrize("n", [1, 17, 1025])
+@pytest.mark.parametrize("kind", ["he3", "dressing", "neutron"])
+def test_magnus_quad_equals_one_lane(kind, n):
+    test_quad_equals_one_lane(kind, st.VARIANT_FAST, n, 2)
 
 
 # the walk back (k_adj_quad against k_adj): gradients of one configuration
