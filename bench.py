@@ -57,10 +57,10 @@ HBM_PEAK_GBS = 8000.0
 SPIN_HBM_BYTES_PER_RECORD = 74.5
 # The same kernel's executed FP64 rate from the hardware counters
 # (SQ_INSTS_VALU_{FMA,MUL,ADD,TRANS}_F64, an FMA counted as 2 operations) over
-# its rocprofv3 duration on this workload; the fast variant executes fewer
+# its launch times on this workload; the fast variant executes fewer
 # FP64 operations per step than the reference formulation above counts.
-HW_COUNTED = {"frac_fp64_peak": 0.471, "TFLOPs": 37.0,
-              "source": "profiles/k_spin_o3_k_kin_fast_dop853_he3_1M_2intervals.md"}
+HW_COUNTED = {"frac_fp64_peak": 0.485, "TFLOPs": 38.1,
+              "source": "profiles/lone_wave_and_1M_counters.md"}
 
 
 def build_workload(n, integrator):
