@@ -502,6 +502,24 @@ static hipError_t spin_quad(st_handle* h, const PipeArgs& A) {
     return fast ? spin_quad_v<VAR_FAST, INT_DOP853>(h, A) : spin_quad_v<VAR_EXACT, INT_DOP853>(h, A);
 }
 
+// One wave per SIMD (k_spin_lone): 64 particles each.  k_spin and k_spin_lone,
+// neutrons x 0.5 s: 2.94 and 2.78 ms at 36,864, 3.12 and 2.95 ms at 65,536
+// (He-3 x 0.2 s: 1.73 and 1.64, 1.96 and 1.89 ms).  Past that, the third wave
+// per SIMD that k_spin has room for comes into play.
+static uint32_t lone_limit(const st_handle* h) {
+    if (h->opt.integratorType != INT_DOP853 || h->ext.variant != ST_VARIANT_FAST || !ST_FIELDS_POLYNOMIAL) return 0;
+    return 64u * (uint32_t)h->n_simd;
+}
+template <bool BATCH, bool PULSE>
+static hipError_t launch_lone(st_handle* h, const PipeArgs& A) {
+    hipLaunchKernelGGL((k_spin_lone<BATCH, PULSE>), dim3((A.n_list + 255) / 256), dim3(256), 0, h->stream, h->P, h->D, A);
+    return hipGetLastError();
+}
+static hipError_t spin_lone(st_handle* h, const PipeArgs& A) {
+    if (h->batch) return h->any_pulse ? launch_lone<true, true>(h, A) : launch_lone<true, false>(h, A);
+    return h->any_pulse ? launch_lone<false, true>(h, A) : launch_lone<false, false>(h, A);
+}
+
 template <bool BATCH, bool PULSE>
 static hipError_t launch_adj(st_handle* h, const AdjArgs& J) {
     if (J.n_list <= 32u * (uint32_t)h->n_simd) {
@@ -764,7 +782,9 @@ static int run_pipeline(st_handle* h, RunArgs R) {
             // counts in d_small[1..2] and does not touch d_small[0]
             const int grid = std::min<int>(h->grid_spin, (int)((n_list + 255) / 256));
             if (h->ktime_on) HIPCHK(h, hipEventRecord(h->kev[2], h->stream));
-            HIPCHK(h, n_list <= quad_limit(h) ? spin_quad(h, A) : spin(h, dim3(grid), A));
+            HIPCHK(h, n_list <= quad_limit(h)   ? spin_quad(h, A)
+                      : n_list <= lone_limit(h) ? spin_lone(h, A)
+                                                : spin(h, dim3(grid), A));
             if (h->ktime_on) HIPCHK(h, hipEventRecord(h->kev[3], h->stream));
         } else if (spectral) {
             // one launch per register block of filters, each with its own queue

@@ -311,12 +311,33 @@ struct AdjQuad {
 };
 
 
+// The tableau entries of the fast trial: the later stages' weights and the
+// error's, which take three products each, and the rest.
+#define ST_DOP_LATE(X)                                                                                              \
+    X(a81) X(a84) X(a85) X(a86) X(a87) X(a91) X(a94) X(a95) X(a96) X(a97) X(a98) X(a101) X(a104) X(a105) X(a106) X(a107) \
+    X(a108) X(a109) X(a111) X(a114) X(a115) X(a116) X(a117) X(a118) X(a119) X(a1110) X(a121) X(a124) X(a125)        \
+    X(a126) X(a127) X(a128) X(a129) X(a1210) X(a1211)
+#define ST_DOP_EARLY(X)                                                                                             \
+    X(a21) X(a31) X(a32) X(a41) X(a43) X(a51) X(a53) X(a54) X(a61) X(a64) X(a65) X(a71) X(a74) X(a75) X(a76) X(c2)   \
+    X(c3) X(c4) X(c5) X(c6) X(c7) X(c8) X(c9) X(c10) X(c11) X(b1) X(b6) X(b7) X(b8) X(b9) X(b10) X(b11) X(b12)      \
+    X(bhh1) X(bhh2) X(bhh3) X(er1) X(er6) X(er7) X(er8) X(er9) X(er10) X(er11) X(er12)
+// as literals
+struct DopLiterals {
+#define X(n) static constexpr double n = dop::n;
+    ST_DOP_LATE(X)
+    ST_DOP_EARLY(X)
+#undef X
+};
 // PULSE = false compiles the pulse term out (configurations without one).
-template <bool ADJ, bool PULSE = true>
+template <bool ADJ, bool PULSE = true, typename TAB = DopLiterals>
 ST_HD inline int dop_trial_fast_t(const SimParams& P, const Phys& F, DopState& D, d3& y, double& h,
-                                  const Seg& S, const Poly& q, uint32_t& nacc, uint32_t& nrej, AdjQuad* Q) {
+                                  const Seg& S, const Poly& q, uint32_t& nacc, uint32_t& nrej, AdjQuad* Q,
+                                  const TAB& T = TAB()) {
 #pragma clang fp contract(fast)
-    using namespace dop;
+#define X(n) const double n = T.n;
+    ST_DOP_LATE(X)
+    ST_DOP_EARLY(X)
+#undef X
     if (D.nstep > P.nmax) return -1;
     if ((D.x + 1.01 * h - D.xf) * D.posneg > 0.0) {
         h = D.xf - D.x;
@@ -483,10 +504,11 @@ ST_HD inline int dop_trial_fast_t(const SimParams& P, const Phys& F, DopState& D
     return 0;
 }
 
-template <bool PULSE = true>
+template <bool PULSE = true, typename TAB = DopLiterals>
 ST_HD __forceinline__ int dop_trial_fast(const SimParams& P, const Phys& F, DopState& D, d3& y, double& h,
-                                         const Seg& S, const Poly& q, uint32_t& nacc, uint32_t& nrej) {
-    return dop_trial_fast_t<false, PULSE>(P, F, D, y, h, S, q, nacc, nrej, nullptr);
+                                         const Seg& S, const Poly& q, uint32_t& nacc, uint32_t& nrej,
+                                         const TAB& T = TAB()) {
+    return dop_trial_fast_t<false, PULSE, TAB>(P, F, D, y, h, S, q, nacc, nrej, nullptr, T);
 }
 
 // ---------------------------------------------------------------------------

@@ -707,7 +707,23 @@ struct NextRec {
     }
 };
 
-template <int VAR, int INTEG, bool BATCH, bool PULSE>
+// The later stages' weights in vector registers for the launch, the rest as
+// literals.  (The empty statements make each value opaque once per launch.)
+struct DopResident {
+#define X(n) double n;
+    ST_DOP_LATE(X)
+#undef X
+#define X(n) static constexpr double n = dop::n;
+    ST_DOP_EARLY(X)
+#undef X
+    __device__ __forceinline__ DopResident() {
+#define X(n) n = dop::n; asm volatile("" : "+v"(n));
+        ST_DOP_LATE(X)
+#undef X
+    }
+};
+
+template <int VAR, int INTEG, bool BATCH, bool PULSE, typename TAB = DopLiterals>
 __device__ __forceinline__ void spin_body(const SimParams& P, const DevState& D, const PipeArgs& A) {
     // (the others take many trials per segment: RK45 8 % slower, at its register
     // line, exact RKF45 15 %, which reads the physics in every stage)
@@ -747,6 +763,7 @@ __device__ __forceinline__ void spin_body(const SimParams& P, const DevState& D,
         else
             return rk.tf;
     };
+    const TAB tab;
     Seg seg;
     Poly poly;
     uint32_t cur_flags = 0;   // low flag bits of the record being integrated (IEND, STOP, coll_type, wall_hit)
@@ -824,7 +841,7 @@ __device__ __forceinline__ void spin_body(const SimParams& P, const DevState& D,
             int st;
             if constexpr (INTEG == INT_DOP853) {
                 if (VAR == VAR_EXACT) st = dop_trial_exact(P, phys(), dop, L.S, L.tempH, seg, L.acc, L.rej);
-                else st = dop_trial_fast<PULSE>(P, phys(), dop, L.S, L.tempH, seg, poly, L.acc, L.rej);
+                else st = dop_trial_fast<PULSE, TAB>(P, phys(), dop, L.S, L.tempH, seg, poly, L.acc, L.rej, tab);
             } else {
                 st = rk_any_trial<VAR, INTEG>(P, phys(), rk, L.S, L.tempH, seg, poly, L.acc, L.rej);
             }
@@ -877,6 +894,13 @@ __global__ __launch_bounds__(256) void k_spin(const SimParams P, const DevState 
 template <int VAR, int INTEG, bool BATCH, bool PULSE>
 __global__ __launch_bounds__(256, 3) void k_spin_o3(const SimParams P, const DevState D, const PipeArgs A) {
     spin_body<VAR, INTEG, BATCH, PULSE>(P, D, A);
+}
+// Fast DOP853 for lists of at most one wave per SIMD: more registers cost no
+// occupancy there, and a literal costs a lone wave two issue slots, 190 of a
+// trip's 1,250 (65,536 neutrons x 0.5 s: 3.12 and 2.95 ms).
+template <bool BATCH, bool PULSE>
+__global__ __launch_bounds__(256, 2) void k_spin_lone(const SimParams P, const DevState D, const PipeArgs A) {
+    spin_body<VAR_FAST, INT_DOP853, BATCH, PULSE, DopResident>(P, D, A);
 }
 // ... and held to 128 (four waves per SIMD), for the quaternion trials
 template <int VAR, int INTEG, bool BATCH, bool PULSE>

@@ -19,7 +19,8 @@ def options(c, n, integ):
 
 
 @pytest.mark.parametrize("integ", [0, 2])
-@pytest.mark.parametrize("n_cfg,n", [(64, 514), (65, 509)])
+# (the last: past one wave per SIMD, 65,536, against plain lists below it)
+@pytest.mark.parametrize("n_cfg,n", [(64, 514), (65, 509), (2, 33000)])
 def test_table_in_lds_and_in_memory(n_cfg, n, integ):
     print(f"[batch table] {n_cfg} x {n} integratorType={integ}", flush=True)
     opts = [options(c, n, integ) for c in range(n_cfg)]
