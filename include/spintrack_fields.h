@@ -41,6 +41,12 @@
  *   ST_FIELDS_PULSE_COS_AXIS  pulse is a*cos(w*t) on one axis (zero when
  *                             a == 0, so the kernels may skip it).
  *
+ * ST_VARIANT_EXACT evaluates the hooks as written whatever the traits say, for
+ * every ensemble size.  (Its kernels for small ensembles form the default
+ * hooks' fields themselves; they run where the compiler finds the hooks to be
+ * the same operations, and otherwise the ensemble takes the kernels that call
+ * the hooks.)
+ *
  * With either trait 0, ST_VARIANT_EXACT runs the hooks as written and
  * st_create refuses ST_VARIANT_FAST, st_adjoint and integratorType 6's fast
  * sampler with ST_E_UNSUPPORTED.

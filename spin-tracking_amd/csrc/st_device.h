@@ -566,6 +566,39 @@ ST_HD __forceinline__ d3 omega_exact(const SimParams& P, const Phys& F, double t
     return d3{Bx * F.gamma, By * F.gamma, Bz * F.gamma};
 }
 
+// Whether the field hooks form each component by itself and by the default
+// hooks' operations: row i of the gradient is r[0]*G[3i] + r[1]*G[3i+1] +
+// r[2]*G[3i+2], summed in that order, and the pulse is +0 off its axis.  The
+// exact trials with four lanes per particle (st_quad.h) evaluate one component
+// per lane and stand in for such hooks only (a hook's three components in each
+// lane would be ten operations and four selects more in each of a trial's
+// thirteen evaluations).  The traits cannot tell: a linear gradient may be
+// summed in another order, and an edit may have left them at 1.
+// The compiler decides: with the hooks inlined, both sides of a comparison
+// become one value exactly where they are the same operations on the same
+// inputs, and only then is its outcome a constant.  Any other hook, or a build
+// without optimisation, gives false.  (The inputs are opaque: volatile reads.)
+inline bool fields_by_component() {
+    volatile double opaque = 0.0;
+    auto same = [](double a, double b) __attribute__((always_inline)) {
+        const bool eq = __builtin_bit_cast(uint64_t, a) == __builtin_bit_cast(uint64_t, b);
+        return __builtin_constant_p(eq) && eq;
+    };
+    double r[3], G[9];
+    for (int i = 0; i < 3; ++i) r[i] = opaque;
+    for (int i = 0; i < 9; ++i) G[i] = opaque;
+    const double t = opaque, a = opaque, w = opaque;
+    bool ok = true;
+    double B[3];
+    st_field_grad(r, G, B);
+    for (int c = 0; c < 3; ++c) ok = ok & same(B[c], r[0] * G[3 * c] + r[1] * G[3 * c + 1] + r[2] * G[3 * c + 2]);
+    for (int axis = 0; axis < 3; ++axis) {
+        st_field_pulse(t, a, w, axis, B);
+        for (int c = 0; c < 3; ++c) ok = ok & (c == axis || same(B[c], 0.0));
+    }
+    return ok;
+}
+
 // Bloch (:83-88): y x (gamma B)
 ST_HD __forceinline__ d3 rhs_exact(const SimParams& P, const Phys& F, double t, const d3& y, const Seg& S) {
     return cross3(y, omega_exact(P, F, t, S));

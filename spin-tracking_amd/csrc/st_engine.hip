@@ -466,10 +466,12 @@ static const void* spin_symbol(int variant, int integ, bool batch, bool pulse) {
 // 10.8 and 10.6 ms at 49,152 (exact 27.2 and 13.1, 27.4 and 22.0, 27.4 and
 // 30.7 ms).  Fast MagnusCFET, He-3 x 0.2 s: 2.34 and 1.17 ms at 32,768, 2.4
 // and 1.95 ms at 49,152.  0: the integrator has no such kernel, or the field
-// hooks have their own form.
+// hooks have a form that its trial does not evaluate (the fast variant's field
+// is the polynomial the traits promise, the exact variant's is the hooks').
 static uint32_t quad_limit(const st_handle* h) {
     const int integ = h->opt.integratorType;
     if (!ST_FIELDS_POLYNOMIAL) return 0;
+    if (h->ext.variant == ST_VARIANT_EXACT && !fields_by_component()) return 0;
     if (integ != INT_DOP853 && integ != INT_RK45 && !(integ == INT_MAGNUS && h->ext.variant == ST_VARIANT_FAST)) return 0;
     return 32u * (uint32_t)h->n_simd;
 }

@@ -402,7 +402,8 @@ __device__ __forceinline__ double q_pulse_exact(const QExact& X, double t) {
     return X.axis == 0 ? pl[0] : (X.axis == 1 ? pl[1] : pl[2]);
 }
 // Bloch's y x omega at time t, component c (rhs_exact, st_device.h); pulse:
-// the pulse's value at t
+// the pulse's value at t.  The gradient is the default hook's, written out:
+// a handle with other hooks never comes here (fields_by_component, st_device.h).
 __device__ __forceinline__ double q_rhs_exact(const QExact& X, bool gravity, double t, double t0, double y, double pulse) {
     const double d = t - t0;
     double p = X.p0 + X.v0 * d, v = X.v0;
