@@ -193,7 +193,6 @@ using namespace st;
 
 namespace {
 thread_local std::string g_create_error;
-constexpr int N_WORK = 8;   // spin: accepted, rejected, segments, trips; kin: events, trips
 }  // namespace
 
 struct st_handle {
@@ -481,14 +480,13 @@ static uint32_t quad_ppw(const st_handle* h, uint32_t n) {
     while (ppw < 16 && ppw * (uint32_t)h->n_simd < n) ppw *= 2;
     return ppw;
 }
-// workgroups of four waves, at most two waves per SIMD
-static uint32_t quad_grid(const st_handle* h, uint32_t n, uint32_t ppw) {
-    return (std::min(2 * (uint32_t)h->n_simd, (n + ppw - 1) / ppw) + 3) / 4;
-}
+// workgroups of four waves that hold the whole list: each wave takes ppw
+// particles, once
+static uint32_t quad_grid(uint32_t n, uint32_t ppw) { return (n + 4 * ppw - 1) / (4 * ppw); }
 template <int VAR, int INTEG, bool BATCH, bool PULSE>
 static hipError_t launch_quad(st_handle* h, const PipeArgs& A) {
     QuadArgs Q{h->P, h->D, A, quad_ppw(h, A.n_list)};
-    hipLaunchKernelGGL((k_spin_quad<VAR, INTEG, BATCH, PULSE>), dim3(quad_grid(h, A.n_list, Q.ppw)), dim3(256), 0, h->stream, Q);
+    hipLaunchKernelGGL((k_spin_quad<VAR, INTEG, BATCH, PULSE>), dim3(quad_grid(A.n_list, Q.ppw)), dim3(256), 0, h->stream, Q);
     return hipGetLastError();
 }
 template <int VAR, int INTEG>
@@ -526,7 +524,7 @@ template <bool BATCH, bool PULSE>
 static hipError_t launch_adj(st_handle* h, const AdjArgs& J) {
     if (J.n_list <= 32u * (uint32_t)h->n_simd) {
         QuadAdjArgs Q{h->P, h->D, J, quad_ppw(h, J.n_list)};
-        hipLaunchKernelGGL((k_adj_quad<BATCH, PULSE>), dim3(quad_grid(h, J.n_list, Q.ppw)), dim3(256), 0, h->stream, Q);
+        hipLaunchKernelGGL((k_adj_quad<BATCH, PULSE>), dim3(quad_grid(J.n_list, Q.ppw)), dim3(256), 0, h->stream, Q);
     } else {
         // two waves per SIMD resident
         const uint32_t grid = std::min((J.n_list + 255) / 256, 2u * (uint32_t)h->n_simd / 4);
@@ -1031,7 +1029,7 @@ static int create_common(const st_options& opt, const st_ext& x, uint32_t n, st_
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, std::max(h->device, 0)) == hipSuccess)
         h->n_simd = 4 * cus;
     hipError_t e = hipMalloc(&h->state, h->state_bytes);
-    if (e == hipSuccess) e = hipMalloc(&h->d_work, N_WORK * sizeof(unsigned long long));
+    if (e == hipSuccess) e = hipMalloc(&h->d_work, WORK_BYTES);
     if (e == hipSuccess) e = hipMalloc(&h->d_small, 256);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&h->own_stream, hipStreamNonBlocking);
     if (e != hipSuccess) {
@@ -1042,7 +1040,7 @@ static int create_common(const st_options& opt, const st_ext& x, uint32_t n, st_
     h->D.base = (char*)h->state;
     h->D.stride = field_stride(h->n);
     h->stream = h->own_stream;
-    e = hipMemsetAsync(h->d_work, 0, N_WORK * sizeof(unsigned long long), h->stream);
+    e = hipMemsetAsync(h->d_work, 0, WORK_BYTES, h->stream);
     if (e != hipSuccess) {
         fail(nullptr, ST_E_HIP, "hipMemsetAsync failed: %s", hipGetErrorString(e));
         st_destroy(h);
@@ -1198,7 +1196,7 @@ ST_API int st_init_subset(st_handle* h, uint32_t first, uint32_t stride) {
         hipLaunchKernelGGL(k_init<false>, grid, dim3(bs), 0, h->stream, h->P, h->D, h->n, o.seed, first, stride, o.t0,
                            o.tf, nullptr, nullptr, nullptr, 1u);
     HIPCHK(h, hipGetLastError());
-    HIPCHK(h, hipMemsetAsync(h->d_work, 0, N_WORK * sizeof(unsigned long long), h->stream));
+    HIPCHK(h, hipMemsetAsync(h->d_work, 0, WORK_BYTES, h->stream));
     // the pipeline's record buffer (up to tens of GB) is allocated here, with
     // the ensemble, rather than inside the first advance
     if (h->ext.engine == ST_ENGINE_PIPELINE) {
@@ -1383,14 +1381,14 @@ ST_API int st_adjoint(st_handle* h, const void* blocks_dev, const double* seeds,
     const int bs = 256;
     if (!h->d_adj) HIPCHK(h, hipMalloc(&h->d_adj, (size_t)field_stride(h->n) * A_COUNT));
     if (!h->d_replay) HIPCHK(h, hipMalloc(&h->d_replay, h->state_bytes));
-    const size_t scratch_bytes = 256 + sizeof(uint32_t) * (size_t)h->n * 4 + sizeof(double) * 3 * K * h->n_cfg;
+    const size_t scratch_bytes = WORK_BYTES + 256 + sizeof(uint32_t) * (size_t)h->n * 4 + sizeof(double) * 3 * K * h->n_cfg;
     if (h->d_scratch) HIPCHK(h, hipFree(h->d_scratch));
     h->d_scratch = nullptr;
     HIPCHK(h, hipMalloc(&h->d_scratch, scratch_bytes));
     char* sp = h->d_scratch;
-    unsigned long long* work = (unsigned long long*)sp;    // 8 counters
-    uint32_t* small = (uint32_t*)(sp + 64);                // queue, next_count, fail_count
-    uint32_t* next_list = (uint32_t*)(sp + 256);
+    unsigned long long* work = (unsigned long long*)sp;    // the replay's counters
+    uint32_t* small = (uint32_t*)(sp + WORK_BYTES);        // queue, next_count, fail_count
+    uint32_t* next_list = small + 64;
     uint32_t* fail_list = next_list + h->n;                // 3 per particle
     double* d_seeds = (double*)(fail_list + 3 * (size_t)h->n);
     HIPCHK(h, hipMemcpyAsync(d_seeds, seeds, sizeof(double) * 3 * K * h->n_cfg, hipMemcpyHostToDevice, h->stream));
@@ -2000,10 +1998,14 @@ ST_API int st_kernel_times(st_handle* h, double ms[2], uint64_t launches[2]) {
 
 ST_API int st_work_counters(st_handle* h, uint64_t out[6]) {
     if (!h || !out) return fail(h, ST_E_ARG, "null argument");
-    unsigned long long w[N_WORK];
+    unsigned long long w[WORK_COPIES][WORK_STRIDE];
+    static_assert(sizeof w == WORK_BYTES, "");
     HIPCHK(h, hipMemcpyAsync(w, h->d_work, sizeof w, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
-    for (int j = 0; j < 6; ++j) out[j] = w[j];
+    for (int j = 0; j < 6; ++j) {
+        out[j] = 0;
+        for (const auto& copy : w) out[j] += copy[j];
+    }
     return ST_OK;
 }
 

@@ -56,19 +56,14 @@ __device__ __forceinline__ d3 q_vec3(const d3& v) { return d3{q_all<I>(v.x), q_a
 // v[c], c = 0..2
 __device__ __forceinline__ double q_pick(const d3& v, uint32_t c) { return c == 0 ? v.x : (c == 1 ? v.y : v.z); }
 
-// Work queue of a wave whose quads hold ppw particles (slot s = quad % ppw):
-// one atomic per wave, consecutive indices to the slots that ask.  All quads
-// of a slot ask together (they run the same particle).
-__device__ __forceinline__ uint32_t quad_acquire(uint32_t* queue, uint32_t ppw) {
-    const uint64_t mask = __ballot(1);
-    const uint64_t first = ppw >= 16 ? ~0ull : (1ull << (4 * ppw)) - 1ull;
-    const uint64_t quads = mask & first & 0x1111111111111111ull;
-    const int leader = __ffsll((unsigned long long)mask) - 1;
-    const uint32_t lane = __lane_id();
-    uint32_t base = 0;
-    if ((int)lane == leader) base = atomicAdd(queue, (uint32_t)__popcll(quads));
-    base = __shfl(base, leader);
-    return base + (uint32_t)__popcll(quads & ((1ull << (4 * ((lane >> 2) % ppw))) - 1ull));
+// List position of a quad's first particle: a wave holds ppw of them (slot =
+// quad % ppw), and the grid covers the list.  (Taken from a work queue, two
+// requests a wave, each cost 11 ns on the queue's one address, as the work
+// counters did; st_state.h.  The loops still look for a next particle, a grid
+// further on: with that branch gone the compiler keeps 30 registers more and
+// spills inside the trial, 16,384 He-3 2.54 and 3.36 ms.)
+__device__ __forceinline__ uint32_t quad_index(uint32_t ppw) {
+    return (blockIdx.x * 4u + (threadIdx.x >> 6)) * ppw + ((__lane_id() >> 2) & (ppw - 1u));
 }
 
 // The launch's arguments, one by-value kernel parameter, read through an
@@ -1003,12 +998,13 @@ __device__ __forceinline__ void quad_spin() {
     uint32_t cnt[4] = {0, 0, 0, 0};   // accepted, rejected, segments, trips (of this launch)
     enum { S_DONE = 0, S_NEXT = 1, S_INT = 2 };
     int phase = S_DONE;
-    const uint32_t n_list = list_len(args().A);
+    uint32_t pos = quad_index(ppw);
     auto take = [&]() {
         const PipeArgs& A = args().A;
         const DevState& D = args().D;
-        const uint32_t i = quad_acquire(A.R.queue, ppw);
-        if (i >= n_list) return;
+        const uint32_t i = pos;
+        pos += 4u * gridDim.x * ppw;
+        if (i >= A.n_list) return;
         spin_load<BATCH>(D, A, A.list[i], L);
         y = q_pick(L.S, c);
         if constexpr (BATCH) physics(A.phys[L.cfg]);
@@ -1016,6 +1012,10 @@ __device__ __forceinline__ void quad_spin() {
         phase = S_NEXT;
     };
     take();
+    // The fast RK45 trial's place within a cache line is worth up to 3 % to a
+    // lone wave (8,192 neutrons, whole run: 18.8 to 19.5 ms over the sixteen
+    // places of the same code); from the start of one it takes 18.87.
+    if constexpr (INTEG == INT_RK45 && VAR == VAR_FAST) asm volatile(".p2align 6");
     while (phase != S_DONE) {
         cnt[3] += lead;
         if (phase == S_NEXT) {
@@ -1204,9 +1204,11 @@ __global__ __launch_bounds__(256, 2) void k_adj_quad(const QuadAdjArgs) {
         nxt = get_rec(A.recs, A.C, pid, (uint32_t)i);
         nxt_t0 = i > 0 ? get_rec(A.recs, A.C, pid, (uint32_t)(i - 1)).t : A.ck.ld(F_T, pid * 8u);
     };
+    uint32_t pos = quad_index(ppw);
     auto take = [&]() {
         const AdjArgs& A = args().A;
-        const uint32_t i = quad_acquire(A.queue, ppw);
+        const uint32_t i = pos;
+        pos += 4u * gridDim.x * ppw;
         if (i >= A.n_list) return;
         pid = A.list[i];
         const uint32_t o = pid * 8u;

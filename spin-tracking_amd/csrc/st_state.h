@@ -159,10 +159,22 @@ __device__ __forceinline__ uint32_t acquire_index(uint32_t* queue) {
     return base + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
 }
 
-// Wave reduction of per-lane counters, one atomic per wave; call with the
-// whole wave converged.
+// Work counters (spin: accepted, rejected, segments, trips; kinematics: events,
+// trips), in WORK_COPIES copies a cache line apart that the host adds up: an
+// atomic on one line takes 11 ns wherever it comes from, and a launch of 2,048
+// waves ends with four each (32,768 neutrons for 1 ms, one trial each: k_spin_quad
+// 105 us with one copy and a work queue, 21 with neither; k_kin of 1,000
+// neutrons 36 and 16).
+constexpr uint32_t WORK_COPIES = 64, WORK_STRIDE = 16;
+constexpr size_t WORK_BYTES = sizeof(unsigned long long) * WORK_COPIES * WORK_STRIDE;
+
+// Wave reduction of per-lane counters, one atomic per wave and counter; call
+// with the whole wave converged.
 template <int N>
 __device__ __forceinline__ void flush_counters(unsigned long long* dst, unsigned long long (&c)[N]) {
+    // (the copy by the cycle counter: a workgroup's index would have to be kept
+    // in a register through the caller's loop)
+    dst += ((uint32_t)__builtin_readcyclecounter() / 4u % WORK_COPIES) * WORK_STRIDE;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
         unsigned long long v = c[j];
