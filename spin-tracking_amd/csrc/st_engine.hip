@@ -647,8 +647,8 @@ static int save_ckpt(st_handle* h, const uint32_t* list, uint32_t n_list) {
 // The chunk loop as a captured HIP graph of K chunks (K even, so the list
 // buffers alternate back to list 0), replayed until the device reports an
 // empty next list: one host round trip per K chunks.  Kernel shapes are fixed
-// (k_kin over all n lanes, k_spin over its persistent grid, k_fixup over 64
-// groups); each reads this chunk's list length and failure count on the
+// (k_kin over all n lanes, k_spin over its persistent grid or what n needs of
+// it, k_fixup over 64 groups); each reads this chunk's list length and failure count on the
 // device.  The graph holds the run's arguments, so it is captured per call.
 // The kinematics kernel over a list of n particles, kbs lanes per workgroup.
 // Up to 32 particles per SIMD a wave takes as few of them (a power of two) as
@@ -682,7 +682,9 @@ static int run_pipeline_graph(st_handle* h, PipeArgs A, SpinFn spin, int kbs) {
         hipLaunchKernelGGL(k_chunk_head, dim3(1), dim3(1), 0, h->stream, h->d_small);
         launch_kin(h, h->D, A, h->n, kbs);
         e = hipGetLastError();
-        if (e == hipSuccess && spin) e = spin(h, dim3(h->grid_spin), A);
+        // (no more workgroups than the ensemble can use: each wave asks the
+        // queue at least once, in every chunk)
+        if (e == hipSuccess && spin) e = spin(h, dim3(std::min<int>(h->grid_spin, (int)((h->n + 255) / 256))), A);
         if (e == hipSuccess) {
             if (h->batch)
                 hipLaunchKernelGGL(k_fixup<true>, dim3(64), dim3(64), 0, h->stream, h->P, h->D, A, FIXUP_FROM_DEVICE);
