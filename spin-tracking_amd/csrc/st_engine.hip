@@ -347,14 +347,21 @@ static SimParams derive_params(const st_options& o, const st_ext& x) {
 static uint64_t field_stride(uint32_t n) { return ((uint64_t)8 * n + 255) & ~(uint64_t)255; }
 
 // ---- kernel selection ------------------------------------------------------
-template <int VAR, int INTEG, bool PERSIST, bool PULSE = true>
+template <int VAR, int INTEG, bool PERSIST, bool PULSE = true, bool ALIGN = true>
 static hipError_t launch_fused(st_handle* h, dim3 grid, dim3 block, const RunArgs& R) {
-    hipLaunchKernelGGL((k_engine<VAR, INTEG, PERSIST, PULSE>), grid, block, 0, h->stream, h->P, h->D, R);
+    hipLaunchKernelGGL((k_engine<VAR, INTEG, PERSIST, PULSE, ALIGN>), grid, block, 0, h->stream, h->P, h->D, R);
     return hipGetLastError();
 }
 using FusedFn = hipError_t (*)(st_handle*, dim3, dim3, const RunArgs&);
+// Exact RK45 in one persistent launch: with its stages kept apart the kernel
+// holds two waves per SIMD instead of one, but a lone wave runs 9 % slower, so
+// up to 64 particles per SIMD it takes the other form.  Dressing x 40 us, kept
+// apart and not: 1.13 and 1.03 ms at 1,000 particles, 1.19 and 1.10 at 65,536,
+// 1.76 and 2.10 at 131,072 (one launch per output time: 1.07 and 1.82, 1.26 and
+// 2.40, always kept apart).
+static bool align_fused(const st_handle* h) { return h->n > 64u * (uint32_t)h->n_simd; }
 template <bool PERSIST>
-static FusedFn pick_fused(int variant, int integ, bool pulse) {
+static FusedFn pick_fused(int variant, int integ, bool pulse, bool align) {
     if (variant == ST_VARIANT_FAST) {
         if (integ == 0)
             return pulse ? launch_fused<VAR_FAST, INT_DOP853, PERSIST, true>
@@ -363,7 +370,9 @@ static FusedFn pick_fused(int variant, int integ, bool pulse) {
         return launch_fused<VAR_FAST, INT_NONE, PERSIST>;
     }
     if (integ == 0) return launch_fused<VAR_EXACT, INT_DOP853, PERSIST>;
-    if (integ == 1) return launch_fused<VAR_EXACT, INT_RK45, PERSIST>;
+    if (integ == 1)
+        return align || !PERSIST ? launch_fused<VAR_EXACT, INT_RK45, PERSIST>
+                                 : launch_fused<VAR_EXACT, INT_RK45, PERSIST, true, !PERSIST>;
     return launch_fused<VAR_EXACT, INT_NONE, PERSIST>;
 }
 static const void* fused_symbol(int variant, int integ, bool pulse) {
@@ -844,11 +853,12 @@ static int run_fused(st_handle* h, RunArgs R, bool persist) {
         if (r) return r;
         HIPCHK(h, hipMemsetAsync(h->d_small, 0, sizeof(uint32_t), h->stream));
         const int grid = std::min<int>(h->grid_fused, (int)((h->n + 255) / 256));
-        hipError_t e = pick_fused<true>(h->ext.variant, h->opt.integratorType, h->any_pulse)(h, dim3(grid), dim3(256), R);
+        hipError_t e = pick_fused<true>(h->ext.variant, h->opt.integratorType, h->any_pulse, align_fused(h))(
+            h, dim3(grid), dim3(256), R);
         if (e != hipSuccess) return fail(h, ST_E_HIP, "engine launch failed: %s", hipGetErrorString(e));
     } else {
         const int bs = h->ext.block_size > 0 ? std::min(256, (h->ext.block_size + 63) / 64 * 64) : 256;
-        hipError_t e = pick_fused<false>(h->ext.variant, h->opt.integratorType, h->any_pulse)(
+        hipError_t e = pick_fused<false>(h->ext.variant, h->opt.integratorType, h->any_pulse, true)(
             h, dim3((h->n + bs - 1) / bs), dim3(bs), R);
         if (e != hipSuccess) return fail(h, ST_E_HIP, "engine launch failed: %s", hipGetErrorString(e));
     }

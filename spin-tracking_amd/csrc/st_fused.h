@@ -140,7 +140,9 @@ enum { PH_DONE = 0, PH_OPEN = 1, PH_EVENT = 2, PH_INT = 3, PH_CLOSE = 4 };
 
 // PULSE = false: the fast DOP853 trial's pulse-free form (handles without a
 // pulse term), the same form the pipeline's spin kernel takes for them
-template <int VAR, int INTEG, bool PERSIST, bool PULSE = true>
+// ALIGN = false: the exact RK45 trial's stages not kept apart (align_fused,
+// st_engine.hip)
+template <int VAR, int INTEG, bool PERSIST, bool PULSE = true, bool ALIGN = true>
 __global__ __launch_bounds__(256) void k_engine(const SimParams P, const DevState D, const RunArgs R) {
     const Phys& F = P.ph;
     Lane L;
@@ -226,7 +228,8 @@ __global__ __launch_bounds__(256) void k_engine(const SimParams P, const DevStat
                 if (VAR == VAR_EXACT) st = dop_trial_exact(P, F, dop, L.S, L.tempH, seg, L.acc, L.rej);
                 else st = dop_trial_fast<PULSE>(P, F, dop, L.S, L.tempH, seg, poly, L.acc, L.rej);
             } else if (INTEG == INT_RK45) {
-                st = rk_any_trial<VAR, INT_RK45>(P, F, rk, L.S, L.tempH, seg, poly, L.acc, L.rej);
+                if constexpr (VAR == VAR_FAST) st = rk_trial_fast(P, rk, L.S, L.tempH, seg, poly, L.acc, L.rej);
+                else st = rk_trial_exact<ALIGN>(P, F, rk, L.S, L.tempH, seg, L.acc, L.rej);
             } else {
                 st = 1;  // unreachable: without an integrator no lane enters PH_INT
             }

@@ -646,6 +646,8 @@ ST_HD inline int rk_trial_fast(const SimParams& P, RkState& R, d3& y, double& h,
 // One iteration of the reference's while(1) (:267-335).  Returns 0 to
 // continue, 1 when the call returns 0 (done), -1 / -2 for the reference's
 // error returns.
+// (ALIGN: its stages aligned and kept apart, ST_CODE_ALIGN.)
+template <bool ALIGN = true>
 ST_HD inline int rk_trial_exact(const SimParams& P, const Phys& Fp, RkState& R, d3& y, double& h, const Seg& S,
                                 uint32_t& nacc, uint32_t& nrej) {
     using namespace rk;
@@ -674,26 +676,26 @@ ST_HD inline int rk_trial_exact(const SimParams& P, const Phys& Fp, RkState& R, 
     const double t = R.t;
     d3 yy1 = R.yy1;
     d3 k1 = F(t, yy1);
-    ST_CODE_ALIGN(k1.x);
+    if constexpr (ALIGN) ST_CODE_ALIGN(k1.x);
     {
         const double c = h * B21;
         ST_V3(yy1, y.x + c * k1.x, y.y + c * k1.y, y.z + c * k1.z);
     }
     d3 k2 = F(t + A2 * h, yy1);
-    ST_CODE_ALIGN(k2.x);
+    if constexpr (ALIGN) ST_CODE_ALIGN(k2.x);
     {
         const double c1 = h * B31, c2_ = h * B32;
         ST_V3(yy1, y.x + c1 * k1.x + c2_ * k2.x, y.y + c1 * k1.y + c2_ * k2.y, y.z + c1 * k1.z + c2_ * k2.z);
     }
     d3 k3 = F(t + A3 * h, yy1);
-    ST_CODE_ALIGN(k3.x);
+    if constexpr (ALIGN) ST_CODE_ALIGN(k3.x);
     {
         const double c1 = h * B41, c2_ = h * B42, c3_ = h * B43;
         ST_V3(yy1, y.x + c1 * k1.x + c2_ * k2.x + c3_ * k3.x, y.y + c1 * k1.y + c2_ * k2.y + c3_ * k3.y,
               y.z + c1 * k1.z + c2_ * k2.z + c3_ * k3.z);
     }
     d3 k4 = F(t + A4 * h, yy1);
-    ST_CODE_ALIGN(k4.x);
+    if constexpr (ALIGN) ST_CODE_ALIGN(k4.x);
     {
         const double c1 = h * B51, c2_ = h * B52, c3_ = h * B53, c4_ = h * B54;
         ST_V3(yy1, y.x + c1 * k1.x + c2_ * k2.x + c3_ * k3.x + c4_ * k4.x,
@@ -701,7 +703,7 @@ ST_HD inline int rk_trial_exact(const SimParams& P, const Phys& Fp, RkState& R, 
               y.z + c1 * k1.z + c2_ * k2.z + c3_ * k3.z + c4_ * k4.z);
     }
     d3 k5 = F(t + A5 * h, yy1);
-    ST_CODE_ALIGN(k5.x);
+    if constexpr (ALIGN) ST_CODE_ALIGN(k5.x);
     {
         const double c1 = h * B61, c2_ = h * B62, c3_ = h * B63, c4_ = h * B64, c5_ = h * B65;
         ST_V3(yy1, y.x + c1 * k1.x + c2_ * k2.x + c3_ * k3.x + c4_ * k4.x + c5_ * k5.x,
@@ -709,7 +711,7 @@ ST_HD inline int rk_trial_exact(const SimParams& P, const Phys& Fp, RkState& R, 
               y.z + c1 * k1.z + c2_ * k2.z + c3_ * k3.z + c4_ * k4.z + c5_ * k5.z);
     }
     d3 k6 = F(t + A6 * h, yy1);
-    ST_CODE_ALIGN(k6.x);
+    if constexpr (ALIGN) ST_CODE_ALIGN(k6.x);
     R.yy1 = yy1;
     d3 ws, te;
     ST_V3(ws, y.x + h * (k1.x * CH1 + k2.x * CH2 + k3.x * CH3 + k4.x * CH4 + k5.x * CH5 + k6.x * CH6),
