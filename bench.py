@@ -55,11 +55,12 @@ HBM_PEAK_GBS = 8000.0
 # a 1 GiB device copy (FETCH_SIZE x 2.000, WRITE_SIZE x 1.000); the
 # algorithmic figure is 64 B per record plus the per-particle spin state.
 SPIN_HBM_BYTES_PER_RECORD = 74.5
-# The same kernel's executed FP64 rate from the hardware counters
-# (SQ_INSTS_VALU_{FMA,MUL,ADD,TRANS}_F64, an FMA counted as 2 operations) over
-# its launch times on this workload; the fast variant executes fewer
+# The FP64 rate the same kernel issues, from the hardware counters
+# (SQ_INSTS_VALU_{FMA,MUL,ADD,TRANS}_F64 x 64 lanes, an FMA counted as 2
+# operations) over its launch times on this workload.  Lanes that are masked
+# off count too: 48 of 64 are active on average.  The fast variant needs fewer
 # FP64 operations per step than the reference formulation above counts.
-HW_COUNTED = {"frac_fp64_peak": 0.485, "TFLOPs": 38.1,
+HW_COUNTED = {"frac_fp64_peak": 0.485, "TFLOPs": 38.1, "active_lanes_of_64": 48,
               "source": "profiles/lone_wave_and_1M_counters.md"}
 
 

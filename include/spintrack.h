@@ -102,7 +102,9 @@ typedef struct st_ext {
                                until every particle is done -- one host round trip per replay
                                instead of per chunk; 0 = host-driven chunk loop.  Runs with
                                checkpointing or per-kernel timing on, and integratorType 6, use the
-                               host-driven loop. */
+                               host-driven loop.  Captured chunks run one lane per particle at every
+                               size, with the same results; the host-driven loop's kernels for lists
+                               of at most 32 particles per SIMD are up to twice as fast */
     int32_t spectrum_sum;   /* integratorType 6: which particles' covariance spectra each interval adds
                                to the run's spectrum.  0 = the reference CPU path's: its in-place tree
                                (src/particle.cpp:826-834) leaves particles 0 and 2^k < numParticles

@@ -705,8 +705,9 @@ ST_HD __forceinline__ void small_sincos(double th, double& s, double& c) {
 // last bit of the difference, so the reduced argument is good to half an ulp
 // of pi/4 -- then the Taylor series (terms to r^16 and r^17; the first omitted
 // ones are below 3e-18).  Within 2 ulp of 1 absolute
-// (tests/host_device_math_main.cpp) at a quarter of its instructions; its
-// large-argument path, with a private array, is left to phases above 2^45.
+// (tests/host_phase_main.cpp) at a quarter of the library sincos's
+// instructions, whose large-argument path, with a private array, is left to
+// phases above 2^45.
 constexpr double PIO2_1 = 0x1.921fb54442d18p+0, PIO2_2 = 0x1.1a62633145c07p-54, PIO2_3 = -0x1.f1976b7ed8fbcp-110;
 ST_HD __forceinline__ void phase_sincos(double x, double& s, double& c) {
     if (!(fabs(x) < 0x1p45)) {

@@ -466,14 +466,15 @@ static const void* spin_symbol(int variant, int integ, bool batch, bool pulse) {
 // Four lanes per particle (st_quad.h) as long as all of the list is on the
 // chip at once: 16 quads in each of two waves per SIMD, 32,768 particles on
 // 256 compute units.  k_spin of one lane and of four, He-3 x 0.2 s: 1.82 and
-// 0.79 ms at 1,000, 1.96 and 1.20 ms at 16,384, 2.01 and 1.59 ms at 32,768,
-// 2.14 and 2.48 ms at 49,152 (neutrons x 0.5 s: 2.97 and 2.42 ms at 32,768,
+// 0.80 ms at 1,000, 1.96 and 1.18 ms at 16,384, 2.01 and 1.56 ms at 32,768,
+// 2.14 and 2.48 ms at 49,152 (neutrons x 0.5 s: 2.97 and 2.35 ms at 32,768,
 // 3.10 and 3.52 ms at 49,152).  The exact variant on the same He-3: 4.32 and
-// 1.86 ms, 4.41 and 2.35 ms, 4.50 and 3.59 ms, 4.55 and 4.58 ms.  RK45,
-// neutrons x 0.5 ms: 10.7 and 4.8 ms at 8,192, 10.8 and 7.7 ms at 32,768
+// 1.86 ms, 4.41 and 2.34 ms, 4.50 and 3.6 ms, 4.55 and 4.58 ms.  RK45,
+// neutrons x 0.5 ms: 10.7 and 4.7 ms at 8,192, 10.8 and 7.7 ms at 32,768
 // 10.8 and 10.6 ms at 49,152 (exact 27.2 and 13.1, 27.4 and 22.0, 27.4 and
-// 30.7 ms).  Fast MagnusCFET, He-3 x 0.2 s: 2.34 and 1.17 ms at 32,768, 2.4
-// and 1.95 ms at 49,152.  0: the integrator has no such kernel, or the field
+// 30.7 ms).  Fast MagnusCFET, He-3 x 0.2 s: 2.34 and 1.11 ms at 32,768, 2.4
+// and 1.95 ms at 49,152.  Short calls gain too: 32,768 neutrons x 1 ms, one
+// trial each, 41 and 21 us.  0: the integrator has no such kernel, or the field
 // hooks have a form that its trial does not evaluate (the fast variant's field
 // is the polynomial the traits promise, the exact variant's is the hooks').
 static uint32_t quad_limit(const st_handle* h) {
@@ -1493,7 +1494,6 @@ ST_API int st_adjoint(st_handle* h, const void* blocks_dev, const double* seeds,
         A.list = c.list;
         A.n_list = c.n_list;
         A.C = (uint32_t)(hi - lo) * h->rec_cap;
-        const dim3 grid((c.n_list + bs - 1) / bs);
         launch_kin(h, DR, A, c.n_list, bs);
         HIPCHK(h, hipGetLastError());
         J.list = c.list;

@@ -747,7 +747,7 @@ ST_HD inline int rk_trial_exact(const SimParams& P, const Phys& Fp, RkState& R, 
 // ---------------------------------------------------------------------------
 // integratorTypes 2-5: integrateMagnusCFET (src/integrator.cpp:620-723),
 // integrateRK45Quaternion (:428-522), integrateRKF45 (:339-426) and
-// integrateRKF45Quaternion (:524-618).  Same protocol as rk_trial: one call is
+// integrateRKF45Quaternion (:524-618).  Same protocol as rk_trial_exact: one call is
 // one iteration of the reference's while(1), state in RkState (yy1 is used by
 // RKF45 only).  The arithmetic follows the reference's order in both variants;
 // the fast variant takes gamma*B from the segment polynomial.
@@ -1092,8 +1092,8 @@ ST_HD __forceinline__ double err_arg(const d3& d) {
 }
 
 // Controller and accept test (e.g. :400-424); 1 when the call ends.  The
-// fast variant forms the step factor from logs of the squared norm, as in
-// rk_trial.
+// fast variant forms the step factor from logs of the squared norm
+// (rk_factor_fast).
 template <int VAR>
 ST_HD __forceinline__ int control_v2(const SimParams& P, RkState& R, d3& y, const d3& ynew, double& h,
                                      double err_in, uint32_t& nacc, uint32_t& nrej) {
